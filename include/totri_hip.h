@@ -281,8 +281,10 @@ int totri_volume_render_exhaustive_grad_volume(
  *           Gaussians, channels 1..A the weighted attribute means
  *   truncation  > 0 skips RBFs farther than truncation * sigma from a voxel;
  *               <= 0 sums all RBFs (the reference's behaviour)
- *   workspace   truncated splats list each brick's RBFs first; the size
- *               comes from the query (0 without truncation)
+ *   workspace   truncated splats list each brick's RBFs first, and need what
+ *               the query says.  Untruncated splats of few voxels and many
+ *               RBFs split the RBFs over workgroups when they get the queried
+ *               bytes, and run unsplit (slower) with less or with NULL.
  */
 size_t totri_rbf2volume_gaussian_forward_workspace(int64_t B, int64_t N, int64_t A,
                                                    int64_t D, int64_t H, int64_t W,
@@ -306,6 +308,22 @@ int totri_rbf2volume_gaussian_grad(const float* rbf, int64_t B, int64_t N, int64
                                    float* rbf_grad, int64_t D, int64_t H, int64_t W,
                                    const float volume_start[3], const float volume_end[3],
                                    float truncation, void* stream);
+
+/*
+ * S2 with scratch memory.  Untruncated, the grid's rows are split over
+ * workgroups and the parts added in a fixed order: with the queried bytes a
+ * few RBFs fill the GPU too.  With less, or with NULL, it runs unsplit, which
+ * is what totri_rbf2volume_gaussian_grad does.
+ */
+size_t totri_rbf2volume_gaussian_grad_workspace(int64_t B, int64_t N, int64_t A, int64_t D,
+                                                int64_t H, int64_t W, float truncation);
+int totri_rbf2volume_gaussian_grad_split(const float* rbf, int64_t B, int64_t N, int64_t A,
+                                         const float* volume, const float* volume_grad,
+                                         float* rbf_grad, int64_t D, int64_t H, int64_t W,
+                                         const float volume_start[3],
+                                         const float volume_end[3], float truncation,
+                                         void* workspace, size_t workspace_bytes,
+                                         void* stream);
 
 /*
  * Batched confocal step (serving).  No counterpart in the reference, whose

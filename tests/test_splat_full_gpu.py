@@ -1,0 +1,98 @@
+"""Untruncated RBF splat and gradient (matrix products over RBFs and over grid
+rows) against the CPU oracle, at the edges of their tiles: 16 z slices and 32
+columns (forward), 16 rows, 16 x and 32 RBFs (gradient), chunks of 32 RBFs per
+wave, groups of 3 attributes (forward) and channel pairs (gradient).
+
+Tolerance 1e-5 relative L2 against FP64: a Gaussian's exponent k r^2 carries
+about four roundings of 2^-24 relative, terms that matter against the 1e-8
+guard have |k r^2| < 27, so their relative error stays below
+27 ln 2 * 4 * 2^-24 = 4.5e-6."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.cases import rel_l2
+
+VS, VE = (-1.0, -1.0, 0.5), (1.0, 1.0, 2.5)
+
+CASES = [  # B, N, A, (D, H, W)
+    (1, 1, 0, (1, 1, 1)),
+    (1, 31, 1, (15, 3, 11)),
+    (2, 33, 2, (16, 4, 8)),
+    (1, 32, 3, (17, 5, 13)),
+    (1, 64, 4, (33, 1, 31)),
+    (1, 300, 8, (49, 6, 16)),
+    (2, 65, 1, (65, 7, 17)),
+    (1, 1500, 1, (12, 10, 9)),     # few voxels, many RBFs: the RBFs are split
+    (1, 40, 1, (40, 41, 15)),      # few RBFs, many rows: the rows are split
+]
+
+
+def _rbf(rng, B, N, A):
+    return np.concatenate([rng.uniform(-1, 1, (B, N, 2)), rng.uniform(0.5, 2.5, (B, N, 1)),
+                           rng.uniform(0.08, 0.3, (B, N, 1)), rng.random((B, N, A))],
+                          2).astype(np.float32)
+
+
+def _calls(rbf, res, G, ws):
+    """Forward and gradient through the C entry points, with or without scratch."""
+    from totrilib_amd import _lib
+    lib = _lib.load()
+    B, N, C = rbf.shape
+    A, (D, H, W) = C - 4, res
+    r, g = torch.from_numpy(rbf).cuda(), torch.from_numpy(G).cuda()
+    vol, grad = torch.empty_like(g), torch.empty_like(r)
+    st = torch.cuda.current_stream().cuda_stream
+    nf = lib.totri_rbf2volume_gaussian_forward_workspace(B, N, A, D, H, W, 0.0) if ws else 0
+    ng = lib.totri_rbf2volume_gaussian_grad_workspace(B, N, A, D, H, W, 0.0) if ws else 0
+    buf = torch.empty(max(nf, ng, 4), dtype=torch.uint8, device="cuda")
+    p = lambda n: buf.data_ptr() if n else None  # noqa: E731
+    assert lib.totri_rbf2volume_gaussian_forward(
+        r.data_ptr(), B, N, A, vol.data_ptr(), D, H, W, _lib.f3(VS), _lib.f3(VE), 0.0, p(nf), nf,
+        ctypes.c_void_p(st)) == 0
+    assert lib.totri_rbf2volume_gaussian_grad_split(
+        r.data_ptr(), B, N, A, vol.data_ptr(), g.data_ptr(), grad.data_ptr(), D, H, W,
+        _lib.f3(VS), _lib.f3(VE), 0.0, p(ng), ng, ctypes.c_void_p(st)) == 0
+    torch.cuda.synchronize()
+    return vol.cpu().numpy(), grad.cpu().numpy(), nf, ng
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,A,res", CASES)
+def test_full_splat_tiles(B, N, A, res):
+    rng = np.random.default_rng(N + A)
+    rbf = _rbf(rng, B, N, A)
+    G = rng.standard_normal((B, 1 + A) + res).astype(np.float32)
+    ref = O.splat_forward(rbf, res, VS, VE, mode=O.PURE64)
+    gref = O.splat_grad(rbf, ref, G, VS, VE, mode=O.PURE64)
+    split = []
+    for ws in (True, False):
+        vol, grad, nf, ng = _calls(rbf, res, G, ws)
+        assert rel_l2(vol, ref) < 1e-5
+        assert rel_l2(grad, gref) < 1e-5
+        split.append((nf, ng))
+    if N == 1500:
+        assert split[0][0] > 0
+    if N == 40:
+        assert split[0][1] > 0
+
+
+@pytest.mark.gpu
+def test_full_splat_zero_sigma():
+    """An RBF of sigma 0 on a voxel gives NaN there and nothing elsewhere."""
+    rng = np.random.default_rng(3)
+    res = (9, 5, 7)
+    rbf = _rbf(rng, 1, 40, 1)
+    clean = rbf[:, :39].copy()
+    rbf[0, 39] = (0.0, 0.0, 1.5, 0.0, 1.0)      # the grid's middle voxel
+    G = rng.standard_normal((1, 2) + res).astype(np.float32)
+    vol, _, _, _ = _calls(rbf, res, G, True)
+    want = O.splat_forward(clean, res, VS, VE, mode=O.PURE64)
+    at = np.zeros(res, bool)
+    at[4, 2, 3] = True
+    assert np.isnan(vol[0, :, at]).all()
+    assert np.isfinite(vol[0, :, ~at]).all()
+    assert rel_l2(vol[0][:, ~at], want[0][:, ~at]) < 1e-5

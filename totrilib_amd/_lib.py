@@ -107,6 +107,12 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _F3, _F3,
          _c_f, _c_p]),
+    "totri_rbf2volume_gaussian_grad_workspace": (
+        _c_sz, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_f]),
+    "totri_rbf2volume_gaussian_grad_split": (
+        _c_int,
+        [_c_p, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _F3, _F3,
+         _c_f, _c_p, _c_sz, _c_p]),
     "totri_confocal_job_workspace": (_c_sz, [_c_p]),
     "totri_confocal_batch_table_bytes": (_c_sz, []),
     "totri_confocal_batch_prepare": (_c_int, [_c_p, _c_int, _c_p, _c_sz]),

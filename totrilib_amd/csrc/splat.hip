@@ -10,17 +10,23 @@
 // be given: RBFs with |q - c|^2 > (trunc sigma)^2 are skipped (trunc <= 0
 // keeps every RBF, which reproduces the reference).
 //
-// S1: a workgroup owns a brick of 8 x 8 x 4 voxels (one per lane).  RBFs are
-// streamed through LDS in chunks; each chunk is culled against the brick's
-// bounding box and the survivors are compacted in index order, so every
-// voxel sums its RBFs in the reference's order.
+// S1, truncated: a workgroup owns a brick of 8 x 8 x 4 voxels (one per lane).
+// RBFs are streamed through LDS in chunks; each chunk is culled against the
+// brick's bounding box and the survivors are compacted in index order, so
+// every voxel sums its RBFs in the reference's order.
 //
-// S2: one wave per RBF walks the voxels of the RBF's support box (the whole
-// volume without truncation) and reduces its gradient over the wave in a
-// fixed order; the reference instead launches one block per (16 columns x
-// 4 slices, RBF) and adds per-block partial sums with float atomics.
+// S2, truncated: one wave per RBF walks the voxels of the RBF's support box
+// and reduces its gradient over the wave in a fixed order; the reference
+// instead launches one block per (16 columns x 4 slices, RBF) and adds
+// per-block partial sums with float atomics.
+//
+// Without truncation every RBF reaches every voxel, and a Gaussian on a grid
+// is a product of one factor per axis: both directions are contractions on
+// the matrix cores (splat_sep_kernel, splat_grad_sep_kernel).
 #include <math.h>
 #include <string.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -296,43 +302,7 @@ __global__ __launch_bounds__(256) void splat_forward_kernel(
     }
   }
 
-  // Untruncated (the reference's default): every RBF reaches every voxel, so
-  // there is nothing to cull; the chunk is walked directly, four RBFs per
-  // step (their loads overlap), summed in index order.
-  for (int c0 = 0; n_list < 0 && !(g.trunc > 0.f) && c0 < g.N; c0 += kChunk) {
-    const int nc = min(kChunk, g.N - c0);
-    __syncthreads();
-    for (int e = tid; e < nc * C; e += blockDim.x) prm[e] = rb[(size_t)c0 * C + e];
-    for (int e = tid; e < nc; e += blockDim.x) pk[e] = gauss_k(rb[(size_t)(c0 + e) * C + 3]);
-    __syncthreads();
-    int k = 0;
-    for (; k + 4 <= nc; k += 4) {
-      float w4[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float* p = prm + (k + u) * C;
-        w4[u] = gauss_exp2(rbf_r2(x, y, z, p[0], p[1], p[2]), pk[k + u]);  // :77
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float* p = prm + (k + u) * C;
-#pragma unroll
-        for (int a = 0; a < kMaxAttr; ++a)
-          if (a < g.A) attr[a] += w4[u] * p[4 + a];          // :78-80
-        sum += w4[u];                                        // :81
-      }
-    }
-    for (; k < nc; ++k) {
-      const float* p = prm + k * C;
-      const float wgt = gauss_exp2(rbf_r2(x, y, z, p[0], p[1], p[2]), pk[k]);
-#pragma unroll
-      for (int a = 0; a < kMaxAttr; ++a)
-        if (a < g.A) attr[a] += wgt * p[4 + a];
-      sum += wgt;
-    }
-  }
-
-  for (int c0 = 0; n_list < 0 && g.trunc > 0.f && c0 < g.N; c0 += kChunk) {
+  for (int c0 = 0; n_list < 0 && c0 < g.N; c0 += kChunk) {
     const int nc = min(kChunk, g.N - c0);
     __syncthreads();
     for (int e = tid; e < nc * C; e += blockDim.x) prm[e] = rb[(size_t)c0 * C + e];
@@ -503,145 +473,468 @@ __global__ __launch_bounds__(kS2Waves * 64) void splat_grad_kernel(
   }
 }
 
-// S2 without truncation: every RBF sees every voxel, so a wave per RBF would
-// read the whole volume once per RBF.  Here a workgroup's waves own
-// kGradRpw RBFs each and share voxel tiles staged in LDS: per voxel the tile
-// holds its coordinates, dL/dV0, 1/V0 (guarded as in the forward), the sum
-// over attributes of dL/dVa * Va and dL/dVa, structure of arrays.  Each lane
-// sums its voxels in tile order, then the wave reduces in a fixed order.
-constexpr int kGradWaves = 8;        // waves per workgroup
-constexpr int kGradTileFloats = 14336;
+// ---------------------------------------------------------------------------
+// Untruncated splats (the reference's default) as matrix products
+// ---------------------------------------------------------------------------
+//
+// g_i(z, y, x) = exp2(k dz^2) * exp2(k (dx^2 + dy^2)), so with the (y, x)
+// columns flattened
+//   V0[z][col]         = sum_i Ez[z][i] * Exy[i][col]
+//   (V0 Va)[z][col]    = sum_i Ez[z][i] * (Exy[i][col] a_i)
+// is a matrix product over the RBFs: per (voxel, RBF) pair and channel one
+// multiply-add on the FP32 matrix cores, where the direct form spends about
+// ten vector instructions.  Both factors are formed in registers as the
+// product's operands (an exponential serves MT or NT tiles), so nothing but
+// the RBFs is read and only the volume is written.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// AT: the attribute count when known at compile time (0 or 1), or -1 (any,
-// up to kMaxAttr, read from g.A).  RPW: RBFs per wave.
-template <int AT, int RPW>
-__global__ __launch_bounds__(kGradWaves * 64) void splat_grad_all_kernel(
-    const float* __restrict__ rbf, const float* __restrict__ vol,
-    const float* __restrict__ vgrad, float* __restrict__ rbf_grad, SplatGeom g, int tv) {
-  constexpr int AN = AT >= 0 ? AT : kMaxAttr;  // attribute slots
-  extern __shared__ float tile[];  // [6 + A][tv]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int b = blockIdx.y;
-  const int A = AT >= 0 ? AT : g.A;
-  const int C = 4 + A;
-  const int i0 = uniform_i32((blockIdx.x * kGradWaves + wave) * RPW);  // scalar registers
-  // this wave's RBFs (indices past N carry sigma 1 and are not written)
-  float xr[RPW], yr[RPW], zr[RPW], si2[RPW], si3[RPW], nh[RPW], av[RPW][AN > 0 ? AN : 1];
-#pragma unroll
-  for (int r = 0; r < RPW; ++r) {
-    const int i = i0 + r;
-    const float* p = rbf + ((size_t)b * g.N + (i < g.N ? i : 0)) * C;
-    xr[r] = p[0];
-    yr[r] = p[1];
-    zr[r] = p[2];
-    const float sg = i < g.N ? p[3] : 1.f;
-    const float si = 1.f / sg;                                 // :38
-    si2[r] = si * si;
-    si3[r] = si2[r] * si;
-    nh[r] = gauss_k(sg);
-#pragma unroll
-    for (int a = 0; a < AN; ++a) av[r][a] = a < A ? p[4 + a] : 0.f;
-  }
-  float acc[RPW][4 + AN];
-#pragma unroll
-  for (int r = 0; r < RPW; ++r)
-#pragma unroll
-    for (int c = 0; c < 4 + AN; ++c) acc[r][c] = 0.f;
+__device__ __forceinline__ f32x4 mfma_16x16x4(float a, float b, f32x4 c) {
+  // D[row][col] += sum_k A[row][k] B[k][col]; lane l holds A[l % 16][l / 16],
+  // B[l / 16][l % 16] and D[4 (l / 16) + 0..3][l % 16]
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
-  const int V = g.D * g.H * g.W;
-  const float* v0b = vol + (size_t)b * (1 + A) * V;
-  const float* g0b = vgrad + (size_t)b * (1 + A) * V;
-  float* tx = tile;
-  float* ty = tile + tv;
-  float* tz = tile + 2 * tv;
-  float* tg = tile + 3 * tv;
-  float* ti = tile + 4 * tv;
-  float* tp = tile + 5 * tv;
-  float* ta = tile + 6 * tv;  // [A][tv]
-  for (int v0 = 0; v0 < V; v0 += tv) {
-    const int nt = min(tv, V - v0);
-    __syncthreads();
-    for (int e = threadIdx.x; e < nt; e += blockDim.x) {
-      const int v = v0 + e;
-      const int xi = v % g.W, yi = (v / g.W) % g.H, zi = v / (g.W * g.H);
-      tx[e] = splat_coord(xi, g.W, g.sx, g.ex);
-      ty[e] = splat_coord(yi, g.H, g.sy, g.ey);
-      tz[e] = splat_coord(zi, g.D, g.sz, g.ez);
-      tg[e] = g0b[v];
-      if (A > 0) {
-        float w0 = v0b[v];
-        if (w0 < 1.e-8f) w0 = 1.f;                             // :167-169
-        ti[e] = 1.f / w0;                                      // :170
-        float pa = 0.f;
-        for (int a = 0; a < A; ++a) {
-          const float dla = g0b[(size_t)(1 + a) * V + v];
-          pa += dla * v0b[(size_t)(1 + a) * V + v];
-          ta[a * tv + e] = dla;
-        }
-        tp[e] = pa;
-      }
-    }
-    __syncthreads();
-    for (int e = lane; e < nt; e += 64) {
-      const float x = tx[e], y = ty[e], z = tz[e], dl0 = tg[e];
-      float inv = 0.f, pa = 0.f, dla[AN > 0 ? AN : 1];
-      if (AN > 0) {
-        inv = ti[e];
-        pa = tp[e];
+constexpr int kSepWaves = 8;    // waves per workgroup; they share an output tile
+constexpr int kSepChunk = 32;   // RBFs a wave stages at once
+constexpr int kSepCols = 32;    // columns per tile: two 16-column products
+constexpr int kSepNT = kSepCols / 16;
+constexpr int kSepAttr = 3;     // attribute channels per workgroup, at most
+
+// exp2(r2 k) of an RBF whose sigma^2 underflows (k = -inf) is NaN on its
+// centre and 0 elsewhere, which no product of axis factors reproduces: such
+// RBFs take no part in the product and are added afterwards.
+__device__ __forceinline__ bool sep_degenerate(float k) { return k == -INFINITY; }
+
+// One workgroup: 16 MT z rows x 32 columns, C channels (the sum and C - 1
+// attributes from a0), over the RBF chunks of its split.  Its eight waves
+// take every eighth chunk and add their tiles through LDS in wave order.
+// part == nullptr: writes the volume; else raw sums [split][B][1 + A][V].
+// Bound by the matrix cores: 20,000 RBFs -> 128^3 with one attribute take
+// 1.6 ms (106 TFLOP/s of matrix products; the card's library FP32 product
+// reaches 154), where the direct form took 16.1 ms; 2,000 -> 64 x 80 x 96
+// 0.050 ms (0.52).
+template <int C, int MT>
+__global__ __launch_bounds__(kSepWaves * 64) void splat_sep_kernel(
+    const float* __restrict__ rbf, float* __restrict__ vol, float* __restrict__ part,
+    SplatGeom g, int n_split) {
+  constexpr int P = MT * kSepNT;  // 16 x 16 tiles of a workgroup
+  // staged RBFs during the walk, partial tiles after it
+  constexpr int kStage = kSepWaves * kSepChunk * (4 + C - 1) * (int)sizeof(float);
+  constexpr int kRed = P * kSepWaves * 64 * (int)sizeof(f32x4);
+  __shared__ __align__(16) char lds[kStage > kRed ? kStage : kRed];
+  const int lane = threadIdx.x & 63, wave = uniform_i32(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int HW = g.H * g.W;
+  const int n_col = (HW + kSepCols - 1) / kSepCols, n_z = (g.D + 16 * MT - 1) / (16 * MT);
+  const int tile = blockIdx.x / n_col;
+  const int col0 = (blockIdx.x - tile * n_col) * kSepCols;
+  const int z0 = (tile % n_z) * (16 * MT);
+  const int a0 = (tile / n_z) * kSepAttr;
+  const int b = blockIdx.y, split = blockIdx.z;
+  const int RC = 4 + g.A;
+  const float* rb = rbf + (size_t)b * g.N * RC;
+
+  float x[kSepNT], y[kSepNT], z[MT];
 #pragma unroll
-        for (int a = 0; a < AN; ++a) dla[a] = (AT >= 0 || a < A) ? ta[a * tv + e] : 0.f;
-      }
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        const float dx = x - xr[r], dy = y - yr[r], dz = z - zr[r];
-        float r2 = dx * dx;
-        r2 = r2 + dy * dy;
-        r2 = r2 + dz * dz;
-        const float wgt = gauss_exp2(r2, nh[r]);               // :15-29, :150
-        const float ws = si2[r] * wgt;
-        const float dxr = dx * ws, dyr = dy * ws, dzr = dz * ws; // :39-41
-        const float dsr = (r2 * si3[r]) * wgt;                   // :42-46
-        float t = dl0;
-        if (AN > 0) {
-          float sa = 0.f;
-#pragma unroll
-          for (int a = 0; a < AN; ++a) {
-            sa += dla[a] * av[r][a];
-            acc[r][4 + a] += (dla[a] * wgt) * inv;             // :178
-          }
-          t = dl0 + (sa - pa) * inv;                           // :176-180
-        }
-        acc[r][0] += dxr * t;                                  // :181-184
-        acc[r][1] += dyr * t;
-        acc[r][2] += dzr * t;
-        acc[r][3] += dsr * t;
-      }
-    }
+  for (int n = 0; n < kSepNT; ++n) {
+    const int col = min(col0 + 16 * n + r, HW - 1);
+    x[n] = splat_coord(col % g.W, g.W, g.sx, g.ex);
+    y[n] = splat_coord(col / g.W, g.H, g.sy, g.ey);
   }
 #pragma unroll
-  for (int r = 0; r < RPW; ++r) {
-    const int i = i0 + r;
-    float* out = rbf_grad + ((size_t)b * g.N + (i < g.N ? i : 0)) * C;
+  for (int m = 0; m < MT; ++m) z[m] = splat_coord(min(z0 + 16 * m + r, g.D - 1), g.D, g.sz, g.ez);
+
+  f32x4 acc[MT][kSepNT][C];
 #pragma unroll
-    for (int c = 0; c < 4 + AN; ++c) {
-      if (c < C) {
-        const float sum = wave_sum_f32(acc[r][c]);
-        if (lane == 0 && i < g.N) out[c] = sum;
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < kSepNT; ++n)
+#pragma unroll
+      for (int c = 0; c < C; ++c) acc[m][n][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  float4* prm = (float4*)lds + wave * kSepChunk;                     // {x, y, z, k}
+  float* att = (float*)((float4*)lds + kSepWaves * kSepChunk) + wave * kSepChunk * (C - 1);
+  const int n_chunk = (g.N + kSepChunk - 1) / kSepChunk;
+  int degenerate = 0;
+  for (int ch = split * kSepWaves + wave; ch < n_chunk; ch += kSepWaves * n_split) {
+    if (lane < kSepChunk) {
+      const int i = ch * kSepChunk + lane;
+      // past the end: infinitely far away
+      float4 v = make_float4(INFINITY, 0.f, 0.f, -1.f);
+      float a[C > 1 ? C - 1 : 1];
+#pragma unroll
+      for (int c = 0; c < C - 1; ++c) a[c] = 0.f;
+      if (i < g.N) {
+        const float* p = rb + (size_t)i * RC;
+        const float k = gauss_k(p[3]);
+        if (sep_degenerate(k)) {
+          degenerate = 1;
+        } else {
+          v = make_float4(p[0], p[1], p[2], k);
+#pragma unroll
+          for (int c = 0; c < C - 1; ++c) a[c] = a0 + c < g.A ? p[4 + a0 + c] : 0.f;
+        }
       }
+      prm[lane] = v;
+#pragma unroll
+      for (int c = 0; c < C - 1; ++c) att[c * kSepChunk + lane] = a[c];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int j = 0; j < kSepChunk / 4; ++j) {  // four RBFs a product
+      const float4 p = prm[4 * j + q];
+      float at[C > 1 ? C - 1 : 1];
+#pragma unroll
+      for (int c = 0; c < C - 1; ++c) at[c] = att[c * kSepChunk + 4 * j + q];
+      float ez[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const float dz = z[m] - p.z;
+        ez[m] = gauss_exp2(dz * dz, p.w);
+      }
+#pragma unroll
+      for (int n = 0; n < kSepNT; ++n) {
+        const float dx = x[n] - p.x, dy = y[n] - p.y;
+        const float e = gauss_exp2(fmaf(dx, dx, dy * dy), p.w);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const float ec = c == 0 ? e : e * at[c - 1];
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[m][n][c] = mfma_16x16x4(ez[m], ec, acc[m][n][c]);
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+
+  const int any_degenerate = __syncthreads_or(degenerate);
+  // Tile p of the workgroup goes to wave p, which adds the waves' parts.
+  f32x4* red = (f32x4*)lds;  // [P][kSepWaves][64]
+  f32x4 sum[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    if (c > 0) __syncthreads();
+#pragma unroll
+    for (int p = 0; p < P; ++p) red[(p * kSepWaves + wave) * 64 + lane] = acc[p / kSepNT][p % kSepNT][c];
+    __syncthreads();
+    sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (wave < P)
+      for (int w = 0; w < kSepWaves; ++w) sum[c] += red[(wave * kSepWaves + w) * 64 + lane];
+  }
+  if (wave >= P) return;
+  const int col = col0 + 16 * (wave % kSepNT) + r;
+  const int zr = z0 + 16 * (wave / kSepNT) + 4 * q;
+  if (col >= HW) return;
+  if (any_degenerate && split == 0) {
+    const float xc = splat_coord(col % g.W, g.W, g.sx, g.ex);
+    const float yc = splat_coord(col / g.W, g.H, g.sy, g.ey);
+    for (int i = 0; i < g.N; ++i) {
+      const float* p = rb + (size_t)i * RC;
+      const float k = gauss_k(p[3]);
+      if (!sep_degenerate(k)) continue;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float zc = splat_coord(min(zr + u, g.D - 1), g.D, g.sz, g.ez);
+        const float w = gauss_exp2(rbf_r2(xc, yc, zc, p[0], p[1], p[2]), k);
+        sum[0][u] += w;
+#pragma unroll
+        for (int c = 1; c < C; ++c)
+          if (a0 + c - 1 < g.A) sum[c][u] += w * p[4 + a0 + c - 1];
+      }
+    }
+  }
+  const size_t V = (size_t)g.D * HW;
+  float* ob = (part ? part + (size_t)split * g.B * (1 + g.A) * V : vol) + (size_t)b * (1 + g.A) * V;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (zr + u >= g.D) break;
+    const size_t vi = (size_t)(zr + u) * HW + col;
+    const float s0 = sum[0][u];
+    if (a0 == 0) ob[vi] = s0;                                  // :83
+    const float den = part || s0 < 1.e-8f ? 1.f : s0;          // :85-87
+#pragma unroll
+    for (int c = 1; c < C; ++c)
+      if (a0 + c - 1 < g.A) ob[(size_t)(a0 + c) * V + vi] = sum[c][u] / den;  // :89-91
+  }
+}
+
+// The splits' raw sums, added in split order and normalised.
+__global__ void splat_sep_finish_kernel(const float* __restrict__ part, int n_split,
+                                        float* __restrict__ vol, int B, int A, size_t V) {
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < (size_t)B * V;
+       e += (size_t)gridDim.x * blockDim.x) {
+    const size_t b = e / V, v = e - b * V;
+    const size_t at = b * (1 + A) * V + v, step = (size_t)B * (1 + A) * V;
+    float den = 1.f;
+    for (int c = 0; c <= A; ++c) {
+      float s = 0.f;
+      for (int k = 0; k < n_split; ++k) s += part[(size_t)k * step + at + (size_t)c * V];
+      vol[at + (size_t)c * V] = s / den;
+      if (c == 0) den = s < 1.e-8f ? 1.f : s;
     }
   }
 }
 
-template <int AT, int RPW>
-int launch_grad_all(const float* rbf, const float* volume, const float* volume_grad,
-                    float* rbf_grad, const SplatGeom& g, hipStream_t st) {
-  const int per = kGradWaves * RPW;
-  const int tv = (kGradTileFloats / (6 + g.A)) & ~63;
-  hipLaunchKernelGGL((splat_grad_all_kernel<AT, RPW>),
-                     dim3((unsigned)((g.N + per - 1) / per), (unsigned)g.B),
-                     dim3(kGradWaves * 64), (size_t)(6 + g.A) * tv * sizeof(float), st, rbf,
-                     volume, volume_grad, rbf_grad, g, tv);
-  return check_launch("splat_grad_all_kernel");
+// S2 without truncation.  With F0 = dL/dV0 - sum_a dL/dVa Va / V0 and
+// Fa = dL/dVa / V0 (V0 guarded as in the forward), an RBF's gradient is a set
+// of moments of F = F0 + sum_a a_{i,a} Fa under its Gaussian: of 1, dx, dy,
+// dz and r^2, and of 1 under each Fa.  The sum over x of a (z, y) row,
+//   P_j[row][i] = sum_x F[row][x] * (exp2(k dx^2) dx^j),  j = 0, 1, 2
+// is a matrix product, and holds nearly all of the work: each of its entries
+// stands for W (voxel, RBF) pairs.  The rest, exp2(k (dy^2 + dz^2)) and its
+// moments, is done once per (row, RBF) on the product's output registers,
+// where a lane holds one RBF (column) and four rows.
+//
+// One workgroup: 32 RBFs, the row tiles (16 rows) of its segment, dealt over
+// its four waves.  The attribute channels come in pairs, one walk over the
+// rows per pair (more accumulators would halve the waves in flight).
+// 20,000 RBFs -> 128^3 with one attribute take 6.1 ms (83 TFLOP/s of matrix
+// products; forming F and the Gaussians takes most of the rest), where the
+// direct form (a voxel tile in LDS, every RBF against every voxel) took
+// 34.8 ms; 2,000 -> 64 x 80 x 96 0.17 ms (2.19).
+constexpr int kGradWaves = 4;
+constexpr int kGradRbf = 32;  // RBFs per workgroup: two 16-column products
+constexpr int kGradNT = kGradRbf / 16;
+constexpr int kGradCoord = 4096;  // coordinates kept in LDS, at most
+
+// AT: the attribute count when known at compile time (0 or 1), or -1.
+template <int NC, int AT>
+__global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_sep_kernel(
+    const float* __restrict__ rbf, const float* __restrict__ vol,
+    const float* __restrict__ vgrad, float* __restrict__ out, SplatGeom g, int n_seg) {
+  __shared__ float coord[kGradCoord + 16];
+  __shared__ float red[kGradWaves][kGradRbf][4 + kMaxAttr];
+  __shared__ float mean[kMaxAttr];
+  const int lane = threadIdx.x & 63, wave = uniform_i32(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int i0 = blockIdx.x * kGradRbf, seg = blockIdx.y, b = blockIdx.z;
+  const int A = AT >= 0 ? AT : g.A, RC = 4 + A, W = g.W;
+  const int n_rows = g.D * g.H, n_tiles = (n_rows + 15) / 16;
+  const size_t V = (size_t)n_rows * W;
+  const float* v0b = vol + (size_t)b * (1 + A) * V;
+  const float* g0b = vgrad + (size_t)b * (1 + A) * V;
+
+  // coordinate tables [D][H][W, to 16]: usual grids fit
+  const bool tabled = (size_t)g.D + g.H + W <= kGradCoord;
+  const float* cz = coord;
+  const float* cy = coord + g.D;
+  const float* cx = coord + g.D + g.H;
+  if (tabled) {
+    for (int e = threadIdx.x; e < g.D; e += blockDim.x) coord[e] = splat_coord(e, g.D, g.sz, g.ez);
+    for (int e = threadIdx.x; e < g.H; e += blockDim.x)
+      coord[g.D + e] = splat_coord(e, g.H, g.sy, g.ey);
+    for (int e = threadIdx.x; e < ((W + 15) & ~15); e += blockDim.x)
+      coord[g.D + g.H + e] = splat_coord(min(e, W - 1), W, g.sx, g.ex);
+  }
+  // A common attribute value taken out of both terms of F0 + a Fa, which
+  // nearly cancel where one RBF stands alone (Va = a there): the mean of the
+  // workgroup's RBFs.
+  if ((int)threadIdx.x < A) {
+    float m = 0.f;
+    for (int n = 0; n < kGradRbf; ++n)
+      m += rbf[((size_t)b * g.N + min(i0 + n, g.N - 1)) * RC + 4 + threadIdx.x];
+    m *= 1.f / kGradRbf;
+    mean[threadIdx.x] = fabsf(m) < INFINITY ? m : 0.f;
+  }
+  __syncthreads();
+
+  // this lane's RBFs (past N: sigma 1, not written)
+  float xr[kGradNT], yr[kGradNT], zr[kGradNT], kg[kGradNT];
+  float mx[kGradNT], my[kGradNT], mz[kGradNT], mr[kGradNT];
+#pragma unroll
+  for (int n = 0; n < kGradNT; ++n) {
+    const int i = i0 + 16 * n + r;
+    const float* p = rbf + ((size_t)b * g.N + min(i, g.N - 1)) * RC;
+    xr[n] = p[0];
+    yr[n] = p[1];
+    zr[n] = p[2];
+    kg[n] = gauss_k(i < g.N ? p[3] : 1.f);
+    mx[n] = my[n] = mz[n] = mr[n] = 0.f;
+  }
+  for (int c0 = 0; c0 <= A; c0 += NC) {  // channels c0 .. c0 + NC - 1 (0: F0)
+    float av[kGradNT][NC], ms[kGradNT][NC];
+#pragma unroll
+    for (int n = 0; n < kGradNT; ++n)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int i = min(i0 + 16 * n + r, g.N - 1);
+        av[n][c] = c0 + c == 0 ? 1.f : 0.f;
+        if (c0 + c >= 1 && c0 + c <= A)
+          av[n][c] = rbf[((size_t)b * g.N + i) * RC + 3 + c0 + c] - mean[c0 + c - 1];
+        ms[n][c] = 0.f;
+      }
+    for (int t = seg * kGradWaves + wave; t < n_tiles; t += kGradWaves * n_seg) {
+      f32x4 acc[kGradNT][NC][3];
+#pragma unroll
+      for (int n = 0; n < kGradNT; ++n)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) acc[n][c][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int row = t * 16 + r;
+      const size_t at = (size_t)min(row, n_rows - 1) * W;
+      // One step of 16 x.  Whole steps load without branches, so that their
+      // loads are in flight together (a branch per load: 2.5 times the time);
+      // rows past the last read it again and count as zero.
+      auto step = [&](int x0, auto whole) {
+        const int xa = x0 + 4 * q;
+        auto load4 = [&](const float* src, float* v) {
+          if constexpr (whole) {
+            __builtin_memcpy(v, src + at + xa, 16);
+          } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = src[at + min(xa + u, W - 1)];
+          }
+        };
+        float F[NC][4], inv[4], xs[4];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) load4(g0b + (size_t)min(c0 + c, A) * V, F[c]);
+        if (A > 0) {
+          load4(v0b, inv);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) inv[u] = 1.f / (inv[u] < 1.e-8f ? 1.f : inv[u]);  // :167-170
+        }
+        if (A > 0 && c0 == 0) {
+          float drift[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+          for (int a = 1; a <= A; ++a) {
+            float dla[4], va[4];
+            if (AT == 1) {
+#pragma unroll
+              for (int u = 0; u < 4; ++u) dla[u] = F[NC - 1][u];
+            } else {
+              load4(g0b + (size_t)a * V, dla);
+            }
+            load4(v0b + (size_t)a * V, va);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) drift[u] = fmaf(dla[u], va[u] - mean[a - 1], drift[u]);
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) F[0][u] -= drift[u] * inv[u];
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (c0 + c > 0) F[c][u] *= inv[u];
+            if (row >= n_rows || c0 + c > A || (!whole && xa + u >= W)) F[c][u] = 0.f;
+          }
+        if (tabled) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) xs[u] = cx[xa + u];
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) xs[u] = splat_coord(min(xa + u, W - 1), W, g.sx, g.ex);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+          for (int n = 0; n < kGradNT; ++n) {
+            const float dx = xs[u] - xr[n];
+            float e0 = gauss_exp2(dx * dx, kg[n]);
+            if (sep_degenerate(kg[n])) e0 = 0.f;
+            const float e1 = dx * e0, e2 = dx * e1;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+              acc[n][c][0] = mfma_16x16x4(F[c][u], e0, acc[n][c][0]);
+              acc[n][c][1] = mfma_16x16x4(F[c][u], e1, acc[n][c][1]);
+              acc[n][c][2] = mfma_16x16x4(F[c][u], e2, acc[n][c][2]);
+            }
+          }
+        }
+      };
+      int x0 = 0;
+      for (; x0 + 16 <= W; x0 += 16) step(x0, std::true_type{});
+      if (x0 < W) step(x0, std::false_type{});
+      // rows 4 q .. 4 q + 3 of the tile, one RBF per lane and product
+      const int first = min(t * 16 + 4 * q, n_rows - 1);
+      int zi = first / g.H, yi = first - zi * g.H;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float yc = tabled ? cy[yi] : splat_coord(yi, g.H, g.sy, g.ey);
+        const float zc = tabled ? cz[zi] : splat_coord(zi, g.D, g.sz, g.ez);
+#pragma unroll
+        for (int n = 0; n < kGradNT; ++n) {
+          const float dy = yc - yr[n], dz = zc - zr[n];
+          const float r2 = fmaf(dy, dy, dz * dz);
+          float e = gauss_exp2(r2, kg[n]);
+          if (sep_degenerate(kg[n])) e = 0.f;
+          float p0 = 0.f, p1 = 0.f, p2 = 0.f;
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            const float s = acc[n][c][0][u] * e;
+            ms[n][c] += s;
+            p0 = fmaf(av[n][c], s, p0);
+            p1 = fmaf(av[n][c], acc[n][c][1][u], p1);
+            p2 = fmaf(av[n][c], acc[n][c][2][u], p2);
+          }
+          mx[n] = fmaf(p1, e, mx[n]);
+          my[n] = fmaf(p0, dy, my[n]);
+          mz[n] = fmaf(p0, dz, mz[n]);
+          mr[n] += fmaf(p2, e, p0 * r2);
+        }
+        if (t * 16 + 4 * q + u + 1 < n_rows && ++yi == g.H) {
+          yi = 0;
+          ++zi;
+        }
+      }
+    }
+    // attribute sums of this pair of channels, over the wave's row groups
+#pragma unroll
+    for (int n = 0; n < kGradNT; ++n)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        float s = ms[n][c];
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        if (q == 0 && c0 + c >= 1 && c0 + c <= A) red[wave][16 * n + r][3 + c0 + c] = s;
+      }
+  }
+#pragma unroll
+  for (int n = 0; n < kGradNT; ++n) {
+    float m[4] = {mx[n], my[n], mz[n], mr[n]};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      m[c] += __shfl_xor(m[c], 16, 64);
+      m[c] += __shfl_xor(m[c], 32, 64);
+      if (q == 0) red[wave][16 * n + r][c] = m[c];
+    }
+  }
+  __syncthreads();
+  float* ob = out + ((size_t)seg * g.B + b) * g.N * RC;
+  for (int e = threadIdx.x; e < kGradRbf * RC; e += blockDim.x) {
+    const int n = e / RC, c = e - n * RC;
+    if (i0 + n >= g.N) continue;
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < kGradWaves; ++w) s += red[w][n][c];
+    const float si = 1.f / rbf[((size_t)b * g.N + i0 + n) * RC + 3];       // :38
+    if (c < 3) s = (s * si) * si;                                          // :39-41
+    if (c == 3) s = ((s * si) * si) * si;                                  // :42-46
+    ob[(size_t)(i0 + n) * RC + c] = s;
+  }
+}
+
+// out[e] = sum over segments: sixteen lanes take every sixteenth segment and
+// add up pairwise, in a fixed order.  (One lane per element took 29 us for
+// 768 segments of 300 elements.)
+__global__ __launch_bounds__(256) void splat_sum_segments_kernel(const float* __restrict__ part,
+                                                                 int n_seg,
+                                                                 float* __restrict__ out,
+                                                                 size_t n) {
+  const int k0 = threadIdx.x >> 4;
+  const size_t e = (size_t)blockIdx.x * 16 + (threadIdx.x & 15);
+  __shared__ float red[16][16];
+  float s = 0.f;
+  if (e < n)
+    for (int k = k0; k < n_seg; k += 16) s += part[(size_t)k * n + e];
+  red[k0][threadIdx.x & 15] = s;
+  __syncthreads();
+  for (int m = 8; m >= 1; m >>= 1) {
+    if (k0 < m) red[k0][threadIdx.x & 15] += red[k0 + m][threadIdx.x & 15];
+    __syncthreads();
+  }
+  if (k0 == 0 && e < n) out[e] = red[0][threadIdx.x & 15];
 }
 
 __global__ void fill_zero_i32_kernel(int* __restrict__ p, size_t n) {
@@ -721,11 +1014,118 @@ BinLayout bin_layout(int64_t B, int64_t D, int64_t H, int64_t W) {
 }  // namespace
 }  // namespace totri_hip
 
+namespace totri_hip {
+namespace {
+
+unsigned blocks_for(size_t n) {
+  const size_t b = (n + 255) / 256;
+  return (unsigned)(b < 65536 ? (b > 0 ? b : 1) : 65536);
+}
+
+struct SepPlan {
+  int mt;       // 16-row z tiles per workgroup
+  int groups;   // attribute groups
+  int split;    // RBF splits (more than one only with room for their sums)
+  unsigned grid;  // tiles x groups
+  size_t bytes;   // of the splits' sums
+};
+
+// The RBFs are split over workgroups only where the tiles of the volume leave
+// more than half of the CUs without one; a split costs a write and a read of
+// the volume, and each wave keeps at least two chunks of RBFs.
+SepPlan sep_plan(int64_t B, int64_t N, int64_t A, int64_t D, int64_t H, int64_t W) {
+  SepPlan p;
+  const int64_t zt = (D + 15) / 16, nz = (zt + 3) / 4;
+  p.mt = (int)((zt + nz - 1) / nz);
+  p.groups = A > 0 ? (int)((A + kSepAttr - 1) / kSepAttr) : 1;
+  const int64_t gz = (zt + p.mt - 1) / p.mt;
+  p.grid = (unsigned)((H * W + kSepCols - 1) / kSepCols * gz * p.groups);
+  const int64_t wgs = (int64_t)p.grid * B;
+  const int64_t chunks = (N + kSepChunk - 1) / kSepChunk;
+  int64_t split = wgs > 0 && wgs * 2 <= 256 ? 256 / wgs : 1;
+  if (split > chunks / (2 * kSepWaves)) split = chunks / (2 * kSepWaves);
+  if (split < 1) split = 1;
+  p.split = (int)split;
+  p.bytes = split > 1 ? (size_t)split * B * (1 + A) * D * H * W * sizeof(float) : 0;
+  return p;
+}
+
+template <int C, int MT>
+void launch_sep(const float* rbf, float* vol, float* part, const SplatGeom& g, const SepPlan& p,
+                int split, hipStream_t st) {
+  hipLaunchKernelGGL((splat_sep_kernel<C, MT>), dim3(p.grid, (unsigned)g.B, (unsigned)split),
+                     dim3(kSepWaves * 64), 0, st, rbf, vol, part, g, split);
+}
+
+template <int C>
+void launch_sep_c(const float* rbf, float* vol, float* part, const SplatGeom& g,
+                  const SepPlan& p, int split, hipStream_t st) {
+  switch (p.mt) {
+    case 1: return launch_sep<C, 1>(rbf, vol, part, g, p, split, st);
+    case 2: return launch_sep<C, 2>(rbf, vol, part, g, p, split, st);
+    case 3: return launch_sep<C, 3>(rbf, vol, part, g, p, split, st);
+    default: return launch_sep<C, 4>(rbf, vol, part, g, p, split, st);
+  }
+}
+
+int splat_forward_full(const float* rbf, float* vol, const SplatGeom& g, void* ws,
+                       size_t ws_bytes, hipStream_t st) {
+  const SepPlan p = sep_plan(g.B, g.N, g.A, g.D, g.H, g.W);
+  const int split = ws != nullptr && ws_bytes >= p.bytes ? p.split : 1;
+  float* part = split > 1 ? (float*)ws : nullptr;
+  const int c = 1 + (g.A < kSepAttr ? g.A : kSepAttr);
+  if (c == 1) launch_sep_c<1>(rbf, vol, part, g, p, split, st);
+  if (c == 2) launch_sep_c<2>(rbf, vol, part, g, p, split, st);
+  if (c == 3) launch_sep_c<3>(rbf, vol, part, g, p, split, st);
+  if (c == 4) launch_sep_c<4>(rbf, vol, part, g, p, split, st);
+  int rc = check_launch("splat_sep_kernel");
+  if (rc || split == 1) return rc;
+  const size_t V = (size_t)g.D * g.H * g.W;
+  hipLaunchKernelGGL(splat_sep_finish_kernel, dim3(blocks_for(g.B * V)), dim3(256), 0, st, part,
+                     split, vol, g.B, g.A, V);
+  return check_launch("splat_sep_finish_kernel");
+}
+
+// Row segments of the untruncated gradient: enough workgroups of 32 RBFs for
+// six per CU, while each wave keeps at least two row tiles.  Below 16 steps
+// of 16 rows x 16 x a wave (about 10 us) the second launch costs more than
+// the segments give: 50 RBFs on 16^3 took 8 us longer a call with them.
+int grad_segments(int64_t B, int64_t N, int64_t D, int64_t H, int64_t W) {
+  const int64_t wgs = B * ((N + kGradRbf - 1) / kGradRbf);
+  const int64_t tiles = (D * H + 15) / 16;
+  const int64_t most = tiles / (2 * kGradWaves);
+  if ((tiles + kGradWaves - 1) / kGradWaves * ((W + 15) / 16) < 16) return 1;
+  int64_t seg = wgs > 0 ? (6 * 256 + wgs - 1) / wgs : 1;
+  if (seg > most) seg = most;
+  return (int)(seg < 1 ? 1 : seg);
+}
+
+int splat_grad_full(const float* rbf, const float* vol, const float* vgrad, float* out,
+                    const SplatGeom& g, void* ws, size_t ws_bytes, hipStream_t st) {
+  int seg = grad_segments(g.B, g.N, g.D, g.H, g.W);
+  const size_t n = (size_t)g.B * g.N * (4 + g.A);
+  if (ws == nullptr || ws_bytes < seg * n * sizeof(float)) seg = 1;
+  float* dst = seg > 1 ? (float*)ws : out;
+  const dim3 grid((unsigned)((g.N + kGradRbf - 1) / kGradRbf), (unsigned)seg, (unsigned)g.B);
+  auto kernel = g.A == 0   ? splat_grad_sep_kernel<1, 0>
+                : g.A == 1 ? splat_grad_sep_kernel<2, 1>
+                           : splat_grad_sep_kernel<2, -1>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kGradWaves * 64), 0, st, rbf, vol, vgrad, dst, g, seg);
+  int rc = check_launch("splat_grad_sep_kernel");
+  if (rc || seg == 1) return rc;
+  hipLaunchKernelGGL(splat_sum_segments_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, st,
+                     dst, seg, out, n);
+  return check_launch("splat_sum_segments_kernel");
+}
+
+}  // namespace
+}  // namespace totri_hip
+
 extern "C" size_t totri_rbf2volume_gaussian_forward_workspace(int64_t B, int64_t N, int64_t A,
                                                               int64_t D, int64_t H, int64_t W,
                                                               float truncation) {
-  (void)A;
-  if (!(truncation > 0.f) || B <= 0 || N <= 0 || D <= 0 || H <= 0 || W <= 0) return 0;
+  if (B <= 0 || N <= 0 || A < 0 || D <= 0 || H <= 0 || W <= 0) return 0;
+  if (!(truncation > 0.f)) return sep_plan(B, N, A, D, H, W).bytes;
   return bin_layout(B, D, H, W).end;
 }
 
@@ -743,6 +1143,8 @@ extern "C" int totri_rbf2volume_gaussian_forward(const float* rbf, int64_t B, in
   TOTRI_CHECK_ARG(volume != nullptr && (N == 0 || rbf != nullptr), "null pointer");
   hipStream_t st = (hipStream_t)stream;
   const SplatGeom g = splat_geom(B, N, A, D, H, W, volume_start, volume_end, truncation);
+  if (!(truncation > 0.f))
+    return splat_forward_full(rbf, volume, g, workspace, workspace_bytes, st);
   const int bx = (int)((W + kBX - 1) / kBX), by = (int)((H + kBY - 1) / kBY),
             bz = (int)((D + kBZ - 1) / kBZ);
   SplatBins bins;
@@ -761,8 +1163,7 @@ extern "C" int totri_rbf2volume_gaussian_forward(const float* rbf, int64_t B, in
     bins.cap = l.cap;
     const size_t n = (size_t)B * l.nb;
     TOTRI_CHECK_ARG(n < (1u << 31), "too many bricks");
-    hipLaunchKernelGGL(fill_zero_i32_kernel, dim3((unsigned)((n + 255) / 256 < 65536 ? (n + 255) / 256 : 65536)),
-                       dim3(256), 0, st, bins.count, n);
+    hipLaunchKernelGGL(fill_zero_i32_kernel, dim3(blocks_for(n)), dim3(256), 0, st, bins.count, n);
     rc = check_launch("fill_zero_i32_kernel");
     if (rc) return rc;
     const dim3 grid((unsigned)((N + kBinWaves - 1) / kBinWaves), (unsigned)B);
@@ -776,6 +1177,37 @@ extern "C" int totri_rbf2volume_gaussian_forward(const float* rbf, int64_t B, in
   return check_launch("splat_forward_kernel");
 }
 
+extern "C" size_t totri_rbf2volume_gaussian_grad_workspace(int64_t B, int64_t N, int64_t A,
+                                                           int64_t D, int64_t H, int64_t W,
+                                                           float truncation) {
+  if (truncation > 0.f || B <= 0 || N <= 0 || A < 0 || D <= 0 || H <= 0 || W <= 0) return 0;
+  const int seg = grad_segments(B, N, D, H, W);
+  return seg > 1 ? (size_t)seg * B * N * (4 + A) * sizeof(float) : 0;
+}
+
+extern "C" int totri_rbf2volume_gaussian_grad_split(const float* rbf, int64_t B, int64_t N,
+                                                    int64_t A, const float* volume,
+                                                    const float* volume_grad, float* rbf_grad,
+                                                    int64_t D, int64_t H, int64_t W,
+                                                    const float volume_start[3],
+                                                    const float volume_end[3],
+                                                    float truncation, void* workspace,
+                                                    size_t workspace_bytes, void* stream) {
+  int rc = check_splat(B, N, A, D, H, W, volume_start, volume_end);
+  if (rc) return rc;
+  if (B == 0 || N == 0) return TOTRI_OK;
+  TOTRI_CHECK_ARG(rbf && volume && volume_grad && rbf_grad, "null pointer");
+  const SplatGeom g = splat_geom(B, N, A, D, H, W, volume_start, volume_end, truncation);
+  if (!(truncation > 0.f))
+    return splat_grad_full(rbf, volume, volume_grad, rbf_grad, g, workspace, workspace_bytes,
+                           (hipStream_t)stream);
+  hipLaunchKernelGGL(splat_grad_kernel,
+                     dim3((unsigned)((N + kS2Waves - 1) / kS2Waves), (unsigned)B),
+                     dim3(kS2Waves * 64), 0, (hipStream_t)stream, rbf, volume, volume_grad,
+                     rbf_grad, g);
+  return check_launch("splat_grad_kernel");
+}
+
 extern "C" int totri_rbf2volume_gaussian_grad(const float* rbf, int64_t B, int64_t N,
                                               int64_t A, const float* volume,
                                               const float* volume_grad, float* rbf_grad,
@@ -783,24 +1215,7 @@ extern "C" int totri_rbf2volume_gaussian_grad(const float* rbf, int64_t B, int64
                                               const float volume_start[3],
                                               const float volume_end[3], float truncation,
                                               void* stream) {
-  int rc = check_splat(B, N, A, D, H, W, volume_start, volume_end);
-  if (rc) return rc;
-  if (B == 0 || N == 0) return TOTRI_OK;
-  TOTRI_CHECK_ARG(rbf && volume && volume_grad && rbf_grad, "null pointer");
-  const SplatGeom g = splat_geom(B, N, A, D, H, W, volume_start, volume_end, truncation);
-  if (!(truncation > 0.f)) {
-    // every RBF reaches every voxel: shared voxel tiles
-    hipStream_t st = (hipStream_t)stream;
-    // two RBFs per wave: more per wave share the tile reads but hold more
-    // registers (8 per wave: 151 VGPRs, two waves per SIMD, 61 ms at
-    // 20,000 RBFs -> 128^3; 4: 38.9 ms; 2: 34.9 ms; 1: 45.6 ms)
-    if (A == 0) return launch_grad_all<0, 2>(rbf, volume, volume_grad, rbf_grad, g, st);
-    if (A == 1) return launch_grad_all<1, 2>(rbf, volume, volume_grad, rbf_grad, g, st);
-    return launch_grad_all<-1, 2>(rbf, volume, volume_grad, rbf_grad, g, st);
-  }
-  hipLaunchKernelGGL(splat_grad_kernel,
-                     dim3((unsigned)((N + kS2Waves - 1) / kS2Waves), (unsigned)B),
-                     dim3(kS2Waves * 64), 0, (hipStream_t)stream, rbf, volume, volume_grad,
-                     rbf_grad, g);
-  return check_launch("splat_grad_kernel");
+  return totri_rbf2volume_gaussian_grad_split(rbf, B, N, A, volume, volume_grad, rbf_grad, D, H,
+                                              W, volume_start, volume_end, truncation, nullptr, 0,
+                                              stream);
 }

@@ -70,8 +70,11 @@ def rbf2volume_gaussian_grad(rbf: torch.Tensor, volume: torch.Tensor,
     lib = _lib.load()
     out = OutputSlot(rbf_grad)
     with torch.cuda.device(dev):
-        rc = lib.totri_rbf2volume_gaussian_grad(
+        ws, wsp = workspace(lib.totri_rbf2volume_gaussian_grad_workspace(
+            B, N, A, D, H, W, float(truncation)), dev)
+        rc = lib.totri_rbf2volume_gaussian_grad_split(
             r.data_ptr(), B, N, A, v.data_ptr(), g.data_ptr(), out.ptr(), D, H, W,
-            _lib.f3(volume_start), _lib.f3(volume_end), float(truncation), stream_ptr(dev))
+            _lib.f3(volume_start), _lib.f3(volume_end), float(truncation), wsp,
+            ws.numel() if ws is not None else 0, stream_ptr(dev))
         _lib.check(rc, "rbf2volume_gaussian_grad")
         out.finish()
