@@ -1,0 +1,62 @@
+"""Velten backprojections (A2, A3) bit for bit against the FP32 oracle at the
+edges of their tiling: units of up to sixteen (scan, laser) pairs (laser tiles
+of equal size, one to three kept in registers, or recomputed above), stages of
+LDS rows with and without a remainder, workgroups of 256 and of 1024 lanes,
+points inside the box (no short root) and width / offset pairs whose quotient
+rounds on bin edges.  Sums run in the reference's order, so equality is exact."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+VS, VE = (-1.0, -1.0, 0.5), (1.0, 1.0, 2.5)
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def points(rng, B, n, inside=False):
+    z = np.full((B, n, 1), 1.0 if inside else 0.0)
+    return np.concatenate([rng.uniform(-1, 1, (B, n, 2)), z], 2).astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [1, 2, 3, 4, 5, 6, 7, 8, 9, 13, 16, 17, 25, 33, 48, 49])
+@pytest.mark.parametrize("T", [96, 1000])
+def test_velten_exhaustive_laser_tiles(L, T):
+    from totrilib_amd.reconstruct import BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(100 + L)
+    B, S, res = 2, 7, (5, 6, 11)
+    w, off = 8.0 / T, 0.25
+    scan, laser = points(rng, B, S), points(rng, B, L, inside=L % 2 == 1)
+    lorg = (laser - np.array([0, 0, 1.0])).astype(np.float32) if L % 3 == 0 else None
+    tr = rng.random((B, T, S, L)).astype(np.float32)
+    got = BackprojectionExhaustiveVelten.apply(
+        t(tr), t(scan), t(laser), VolumeDef(VS, VE, res), BinDef(w, off, T), None,
+        None if lorg is None else t(lorg)).cpu().numpy()
+    ref = O.velten_exhaustive(tr, scan, laser, None, lorg, res, VS, VE, w, off, mode=O.FP32)
+    assert np.count_nonzero(ref) > 300
+    assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("res", [(64, 48, 65), (3, 5, 7)])     # 1024 and 256 lanes
+@pytest.mark.parametrize("S,T", [(1, 64), (9, 512), (21, 1500), (5, 3000)])
+def test_velten_stages(res, S, T):
+    from totrilib_amd.reconstruct import BackprojectionConfocalVelten, BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(S + T)
+    w, off = 0.0078125 * 512 / T, 0.0
+    scan, laser = points(rng, 1, S), points(rng, 1, 2)
+    tr = rng.random((1, T, S, 2)).astype(np.float32)
+    vd, bd = VolumeDef(VS, VE, res), BinDef(w, off, T)
+    got = BackprojectionConfocalVelten.apply(t(tr[..., 0]), t(scan), vd, bd).cpu().numpy()
+    ref = O.velten_confocal(tr[..., 0], scan, None, res, VS, VE, w, off, mode=O.FP32)
+    assert ref.any()
+    assert np.array_equal(got.astype(np.float64), ref)
+    got = BackprojectionExhaustiveVelten.apply(t(tr), t(scan), t(laser), vd, bd).cpu().numpy()
+    ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, w, off, mode=O.FP32)
+    assert np.array_equal(got.astype(np.float64), ref)

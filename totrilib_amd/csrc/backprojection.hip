@@ -24,6 +24,7 @@
 // volumes that are summed in chunk order.
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -31,8 +32,6 @@
 
 namespace totri_hip {
 namespace {
-
-constexpr int kStageFloats = 8192;  // LDS floats of staged transient rows (32 KiB)
 
 // Blocks of a grid-stride loop over n elements (capped).
 int grid1d(size_t n, int block = 256) {
@@ -89,19 +88,14 @@ __device__ __forceinline__ int nearest_bin(float dist, float w, float off) {
 // A2: vol[b][z][y][x] = sum_s tr[b][t(s)][s],
 // t = nearest_bin(2 |p_s - o_s| + 2 |p_s - q|)       (backprojection_cuda.cu:152-194)
 //
-// For one scan point, t is a non-decreasing function of the squared distance
-// e = (dx*dx + dy*dy) + dz*dz: every step of the formula (correctly rounded
-// square root, doubling, the sum with 2 |p_s - o_s|, the subtraction of the
-// offset, the division by a positive width, + 0.5, floor, saturating
-// conversion) is monotone.  So t(e) >= k exactly when e >= E_k, with
-// E_k = min{e : t(e) >= k}.  velten_bins_kernel finds E_0 .. E_T per scan
-// point by bisection over the float bit patterns, evaluating the exact
-// formula.  The backprojection then takes a cheap estimate a of t (hardware
-// square root, one FMA with precomputed constants), within one bin of t, and
-// corrects it with two table entries:
-//   t = a - [e < E_a] + [e >= E_(a+1)].
-// That is the exact decision, with no correctly rounded root or division
-// per (voxel, scan point) pair.
+// A cheap estimate of the bin's argument (hardware square root, one FMA with
+// precomputed constants) decides wherever its distance to the next bin edge
+// exceeds a bound on its error; the few samples nearer to an edge take the
+// reference's formula.  That is the exact decision, with no correctly rounded
+// root or division for most (voxel, scan point) pairs, and one gather a pair.
+// (Correcting the estimate with two thresholds of a table per scan point
+// needs no bound but three gathers, and the thresholds a kernel of their own:
+// 0.38 ms at 64^3 voxels, 32 x 32 points, 512 bins, against 0.165 ms.)
 // ---------------------------------------------------------------------------
 
 // The exact bin of squared distance e for a scan point whose origin term is
@@ -112,32 +106,16 @@ __device__ __forceinline__ int velten_bin(float e, float dso2, float w, float of
   return nearest_bin(dist, w, off);
 }
 
-// Per-scan-point constants of the estimate: the point and
-// c = ((dso2 - off) * (1/w)) + 0.5, so that a = floor(fma(sqrt(e), 2/w, c)).
-// c is NaN where the estimate's error bound does not hold (below); those
-// scan points take the exact formula per pair.
-struct VeltenPoint {
-  float px, py, pz, c;
-};
+// Workspace of A2: a header of 8 floats per scan point,
+//   {x, y, z, c, dso2, half, 0, 0}: the estimate is fma(sqrt(e), 2/w, c),
+//   c = ((dso2 - off) * (1/w)) + 0.5, and decides where its fraction lies
+//   within `half` of 1/2; c is NaN where no bound holds (every pair of that
+//   point takes the formula),
+// then one row of nv floats per scan point: bin t at t, a zero at T (nv = T + 1
+// rounded up to a multiple of 4).
+constexpr int kVeltenHead = 8;
 
-// One row of floats per scan point, all parts 16-byte aligned:
-//   [0, 4)             the point's constants (VeltenPoint)
-//   [4, 4 + nv)        its transient bins, vals[1 + t] = bin t, zeros at 0
-//                      and T + 1 (nv = T + 2 rounded up to a multiple of 4)
-//   [4 + nv, 4 + nv + nt)  its thresholds { -inf, E_0, ..., E_T, NaN }
-//                      (nt = T + 3 rounded up to a multiple of 4)
-// so that a group of consecutive scan points is one contiguous block.
-struct VeltenRow {
-  int nv, nt, len;
-};
-
-__host__ __device__ __forceinline__ VeltenRow velten_row(int T) {
-  VeltenRow r;
-  r.nv = (T + 5) & ~3;
-  r.nt = (T + 6) & ~3;
-  r.len = 4 + r.nv + r.nt;
-  return r;
-}
+__host__ __device__ __forceinline__ int velten_row(int T) { return (T + 4) & ~3; }
 
 // Estimate error: the exact chain rounds five times (root, sum, difference,
 // quotient, + 0.5) and the estimate about eight times (hardware root within
@@ -145,154 +123,124 @@ __host__ __device__ __forceinline__ VeltenRow velten_row(int T) {
 // error of at most 2^-24 (2^-23 for the root) of a term no larger than M bins,
 // M = (2 d_max + |dso2| + |off|) / w + 1 with d_max the largest distance from
 // the scan point to the box's corners.  The two differ by under 16 * 2^-24 * M
-// bins; M < 2^16 keeps that below 1/16 of a bin, so the estimate is within
-// one bin of the exact value.
+// bins; the guard takes 17, and M < 2^16 keeps it below 1/14 of a bin.
 constexpr float kVeltenMaxBins = 65536.f;
+constexpr float kVeltenGuard = 17.f * 0x1p-24f;
 
-// Thread (b, s, j), j in [0, T + 3): threshold j of scan point s, that is
-// -inf, E_0, ..., E_T, NaN, where E_k = +inf when no finite e reaches bin k.
-// For an estimate a in [-1, T] the rows' threshold part gives E_a at index
-// a + 1 and E_(a+1) at a + 2 (no e is below -inf, and no e compares >= NaN).
-// Thread j = 0 also writes the point's constants and the zero pads of its
-// bins.
-__global__ __launch_bounds__(256) void velten_bins_kernel(
+// One thread per scan point: its header and the zero slot of its row.
+__global__ __launch_bounds__(256) void velten_head_kernel(
     const float* __restrict__ scan, const float* __restrict__ orig, BoxGeom g, int S, int So,
-    float rw, float* __restrict__ rows) {
-  const int T = g.T;
-  const VeltenRow vr = velten_row(T);
-  const int n = T + 3;
-  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (size_t)g.B * S * n) return;
-  const int j = (int)(id % n);
-  const size_t bs = id / n;  // b * S + s
+    float rw, float* __restrict__ head, float* __restrict__ rows) {
+  const int nv = velten_row(g.T);
+  const size_t bs = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // b * S + s
+  if (bs >= (size_t)g.B * S) return;
   const int b = (int)(bs / S), s = (int)(bs - (size_t)b * S);
-  float* row = rows + bs * vr.len;
   const float* p = scan + bs * 3;
   const float px = p[0], py = p[1], pz = p[2];
   float dso = 0.f;
   if (So > 0) {
     const float* o = orig + ((size_t)b * So + s) * 3;
-    dso = dist3(px, py, pz, o[0], o[1], o[2]);
+    dso = dist3(px, py, pz, o[0], o[1], o[2]);                               // :178-183
   }
   const float dso2 = 2.f * dso;
-  float e;
-  if (j == 0) {
-    e = -INFINITY;
-  } else if (j == n - 1) {
-    e = __builtin_nanf("");
-  } else {
-    // E_k: the smallest e >= 0 (as a bit pattern; monotone for non-negative
-    // floats) with velten_bin(e) >= k.  A guess from the bin's edge in
-    // double, ((k - 1/2) w + off - dso2)^2 / 4, is a few ulps from it: walk
-    // from there while the neighbour agrees, in at most 64 steps, else bisect
-    // over all patterns.  +inf (0x7f800000) always qualifies.
-    const int k = j - 1;
-    const double dk = ((double)k - 0.5) * (double)g.w + (double)g.off - (double)dso2;
-    const double gd = dk > 0.0 ? 0.25 * dk * dk : 0.0;
-    const float gf = gd < 3.0e38 ? (float)gd : INFINITY;
-    unsigned u = __float_as_uint(gf);  // gf >= 0 or NaN (NaN: bisect below)
-    bool found = false;
-    if (gf == gf) {
-      if (velten_bin(__uint_as_float(u), dso2, g.w, g.off) >= k) {
-        for (int it = 0; it < 64; ++it) {  // step down to the first pattern that qualifies
-          if (u == 0u || velten_bin(__uint_as_float(u - 1u), dso2, g.w, g.off) < k) {
-            found = true;
-            break;
-          }
-          --u;
-        }
-      } else {
-        for (int it = 0; it < 64 && u < 0x7f800000u; ++it) {
-          ++u;
-          if (velten_bin(__uint_as_float(u), dso2, g.w, g.off) >= k) {
-            found = true;
-            break;
-          }
-        }
-      }
-    }
-    if (!found) {
-      unsigned lo = 0u, hi = 0x7f800000u;
-      if (velten_bin(0.f, dso2, g.w, g.off) >= k) {
-        hi = 0u;
-      } else {
-        while (hi - lo > 1u) {
-          const unsigned mid = lo + (hi - lo) / 2u;
-          if (velten_bin(__uint_as_float(mid), dso2, g.w, g.off) >= k)
-            hi = mid;
-          else
-            lo = mid;
-        }
-      }
-      u = hi;
-    }
-    e = __uint_as_float(u);
-  }
-  row[4 + vr.nv + j] = e;
-  if (j == 0) {
-    // the largest distance to the box is at a corner
-    float dmax = 0.f;
-    for (int c = 0; c < 8; ++c)
-      dmax = fmaxf(dmax, dist3(px, py, pz, (c & 1) ? g.ex : g.sx, (c & 2) ? g.ey : g.sy,
-                               (c & 4) ? g.ez : g.sz));
-    const float m = (2.f * dmax + fabsf(dso2) + fabsf(g.off)) / g.w + 1.f;
-    const bool est = g.w > 0.f && m < kVeltenMaxBins;  // false for NaN or inf
-    *(float4*)row = make_float4(px, py, pz, est ? (dso2 - g.off) * rw + 0.5f
-                                                : __builtin_nanf(""));
-    row[4] = 0.f;
-    row[4 + T + 1] = 0.f;
-  }
+  // the largest distance to the box is at a corner
+  float dmax = 0.f;
+  for (int c = 0; c < 8; ++c)
+    dmax = fmaxf(dmax, dist3(px, py, pz, (c & 1) ? g.ex : g.sx, (c & 2) ? g.ey : g.sy,
+                             (c & 4) ? g.ez : g.sz));
+  const float m = (2.f * dmax + fabsf(dso2) + fabsf(g.off)) / g.w + 1.f;
+  const bool est = g.w > 0.f && m < kVeltenMaxBins;  // false for NaN or inf
+  float4* h = (float4*)(head + bs * kVeltenHead);
+  h[0] = make_float4(px, py, pz, est ? (dso2 - g.off) * rw + 0.5f : __builtin_nanf(""));
+  h[1] = make_float4(dso2, est ? 0.5f - kVeltenGuard * m : 0.f, 0.f, 0.f);
+  rows[bs * nv + g.T] = 0.f;
 }
 
-// Bin of squared distance e for the scan point of `row` (stage or global):
-// the corrected estimate, or the exact formula where the point's c is NaN.
-// The result is clamped to [-1, T], whose ends read the zero pads.
-template <bool EXACT>
-__device__ __forceinline__ int velten_take_bin(const float* row, const VeltenRow& vr, float e,
-                                               float c, float k2, int T, float dso2,
-                                               const BoxGeom& g) {
-  if (!EXACT) {
-    int a = (int)floorf(__builtin_fmaf(sqrt_fast(e), k2, c));
-    a = min(max(a, -1), T);
-    const float* E = row + 4 + vr.nv + a + 1;
-    return a + (e < E[0] ? -1 : 0) + (e >= E[1] ? 1 : 0);
-  }
-  const int t = velten_bin(e, dso2, g.w, g.off);                             // :177,185-187
-  return min(max(t, -1), T);
-}
-
-__device__ __forceinline__ float velten_sqdist(const float4& p, float qx, float qy, float qz) {
-  const float dx = p.x - qx, dy = p.y - qy, dz = p.z - qz;
+__device__ __forceinline__ float velten_sqdist(float px, float py, float pz, float qx, float qy,
+                                               float qz) {
+  const float dx = px - qx, dy = py - qy, dz = pz - qz;
   float e = dx * dx;
   e = e + dy * dy;
   e = e + dz * dz;
   return e;
 }
 
-// Scan points per unrolled group of the backprojection loop.
-constexpr int kVeltenUnroll = 8;
+// Whether an estimate r lies too near a bin edge to decide (also NaN, inf).
+__device__ __forceinline__ bool velten_near(float r, float half) {
+  return !(fabsf(__builtin_amdgcn_fractf(r) - 0.5f) <= half);
+}
 
-// LDS floats of one stage of scan-point rows (32 KiB, four workgroups per
-// CU), and the float4s per thread that copy one stage with a 256-lane
-// workgroup.
-constexpr int kVeltenStage = kStageFloats;
-constexpr int kVeltenCopy4 = kVeltenStage / 4 / 256;
+// Slot of bin t: bins outside [0, T) read the zero at T.
+__device__ __forceinline__ unsigned velten_slot(int t, int T) {
+  return min((unsigned)t, (unsigned)T);
+}
 
-// One lane per voxel, flat over [D][H][W]; rows as laid out above.  A
-// workgroup stages the rows of R scan points in LDS (STAGED), loading the
-// next group into registers while it works on the current one, or reads
-// them from global memory (rows too long for the stage).  Sums run over scan
-// points in order, as the reference's loop.
-template <bool STAGED>
-__global__ __launch_bounds__(256) void velten_confocal_kernel(
-    const float* __restrict__ rows, const float* __restrict__ orig, float* __restrict__ vol,
-    BoxGeom g, int S, int So, int R, float k2) {
+// Staged rows (A2, A3): two LDS buffers of `cap` floats.  A workgroup writes
+// the next rows, loaded into registers one stage earlier, into one buffer
+// while its waves read the other, so a stage costs one barrier.  Every
+// workgroup reads all rows, so L2 traffic falls with the voxels per workgroup:
+// at 64^3 and 4096 pairs of 512 bins, 1024 lanes (one workgroup per CU) read
+// 2.1 GB where 256 lanes read 8.6 GB (A3: 0.85 -> 0.79 ms).  Volumes that
+// would leave a quarter of the CUs without a workgroup of 1024 keep 256 lanes.
+// Floats per buffer, at most: 72 KiB where a workgroup has a CU to itself,
+// else 40 KiB.
+constexpr int stage_max(int threads) { return threads == 1024 ? 18432 : 10240; }
+
+template <int NTH>
+struct RowStage {
+  static constexpr int kCopy4 = (stage_max(NTH) / 4 + NTH - 1) / NTH;
+  float4 buf[kCopy4];
+  // n4 float4s, 0 <= n4 <= stage_max(NTH) / 4
+  __device__ __forceinline__ void load(const float* src, int n4) {
+#pragma unroll
+    for (int i = 0; i < kCopy4; ++i) {
+      const int e = i * NTH + (int)threadIdx.x;
+      buf[i] = e < n4 ? ((const float4*)src)[e] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+  __device__ __forceinline__ void store(float* dst, int n4) const {
+#pragma unroll
+    for (int i = 0; i < kCopy4; ++i) {
+      const int e = i * NTH + (int)threadIdx.x;
+      if (e < n4) ((float4*)dst)[e] = buf[i];
+    }
+  }
+};
+
+// Lets a kernel take both buffers (launches get 64 KiB by default).
+template <typename K>
+int allow_stage(K kernel) {
+  TOTRI_CHECK_HIP(hipFuncSetAttribute((const void*)kernel,
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      2 * stage_max(1024) * (int)sizeof(float)));
+  return TOTRI_OK;
+}
+
+// Workgroup size and floats per buffer for B volumes of nvox voxels.
+struct StagePlan {
+  int threads, cap;
+};
+
+StagePlan stage_plan(int64_t B, int64_t nvox) {
+  if (B * ((nvox + 1023) / 1024) >= 192) return {1024, stage_max(1024)};
+  // up to two workgroups per CU take full buffers, more of them half
+  return {256, B * ((nvox + 255) / 256) <= 512 ? stage_max(256) : stage_max(256) / 2};
+}
+
+// One lane per voxel, flat over [D][H][W].  The rows of R scan points at a
+// time are staged in LDS (STAGED), or read from global memory (rows too long
+// for the stage).  The headers are uniform and come through the scalar cache.
+// Sums run over scan points in order, as the reference's loop.
+template <bool STAGED, int UN, int NTH>
+__global__ __launch_bounds__(NTH) void velten_confocal_kernel(
+    const float* __restrict__ head, const float* __restrict__ rows, float* __restrict__ vol,
+    BoxGeom g, int S, int R, int cap, float k2, DivConst dw) {
   extern __shared__ float4 lds4[];
   const int T = g.T;
-  const VeltenRow vr = velten_row(T);
+  const int nv = velten_row(T);
   const int b = blockIdx.y;
   const int nvox = g.D * g.H * g.W;
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  const int v = blockIdx.x * NTH + threadIdx.x;
   const bool ok = v < nvox;
   const int vv = ok ? v : 0;
   const int x = vv % g.W;
@@ -302,91 +250,72 @@ __global__ __launch_bounds__(256) void velten_confocal_kernel(
   const float qy = inclusive_coord(y, g.H, g.sy, g.ey);
   const float qz = inclusive_coord(z, g.D, g.sz, g.ez);
   const size_t bS = (size_t)b * S;
-  const float* ob = orig + bS * 3;
   float* stage = (float*)lds4;
-  // the rows of the next group of points, loaded into registers
-  float4 buf[kVeltenCopy4];
+  RowStage<NTH> next;
+  auto load = [&](int s0) { next.load(rows + (bS + s0) * nv, min(R, S - s0) * nv / 4); };
   if (STAGED) {
-    const int n4 = min(R, S) * vr.len / 4;
-    const float4* src = (const float4*)(rows + bS * vr.len);
-#pragma unroll
-    for (int i = 0; i < kVeltenCopy4; ++i) {
-      const int e = i * 256 + (int)threadIdx.x;
-      buf[i] = e < n4 ? src[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+    load(0);
+    next.store(stage, min(R, S) * nv / 4);
+    if (R < S) load(R);
+    __syncthreads();
   }
   float value = 0.f;
+  int cur = 0;
   for (int s0 = 0; s0 < S; s0 += R) {
     const int ns = min(R, S - s0);
-    const float* base = rows + (bS + s0) * vr.len;
-    if (STAGED) {
-      __syncthreads();  // the previous group is no longer read
-      const int n4 = ns * vr.len / 4;
-#pragma unroll
-      for (int i = 0; i < kVeltenCopy4; ++i) {
-        const int e = i * 256 + (int)threadIdx.x;
-        if (e < n4) lds4[e] = buf[i];
-      }
-      __syncthreads();
-      if (s0 + R < S) {
-        const int n4n = min(R, S - s0 - R) * vr.len / 4;
-        const float4* src = (const float4*)(rows + (bS + s0 + R) * vr.len);
-#pragma unroll
-        for (int i = 0; i < kVeltenCopy4; ++i) {
-          const int e = i * 256 + (int)threadIdx.x;
-          buf[i] = e < n4n ? src[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-      }
-      base = stage;
+    const float* base = STAGED ? stage + cur * cap : rows + (bS + s0) * nv;
+    if (STAGED && s0 + R < S) {
+      next.store(stage + (cur ^ 1) * cap, min(R, S - s0 - R) * nv / 4);
+      if (s0 + 2 * R < S) load(s0 + 2 * R);
     }
-    // kVeltenUnroll points at a time (the last group of a stage may have
-    // fewer, nu; its missing slots repeat the last point and add nothing):
-    // their loads and decisions overlap, their values are added in point
-    // order.  A group with a point whose c is NaN takes the per-point path
-    // (the choice is uniform).
-    for (int k = 0; k < ns; k += kVeltenUnroll) {
-      const int nu = min(kVeltenUnroll, ns - k);
-      float4 p[kVeltenUnroll];
-      bool est = true;
+    // UN points at a time: their decisions and gathers overlap, their values
+    // are added in point order.  (No short-circuit in the guard test: a branch
+    // per point serialises the scalar loads, 0.35 ms.)
+    const float* h = head + (bS + s0) * kVeltenHead;
+    int k = 0;
+    for (; k + UN <= ns; k += UN, h += UN * kVeltenHead) {
+      float px[UN], py[UN], pz[UN], c[UN], dso2[UN], half[UN];
 #pragma unroll
-      for (int u = 0; u < kVeltenUnroll; ++u) {
-        p[u] = *(const float4*)(base + (k + min(u, nu - 1)) * vr.len);
-        est = est && p[u].w == p[u].w;
+      for (int u = 0; u < UN; ++u) {
+        px[u] = h[u * kVeltenHead];
+        py[u] = h[u * kVeltenHead + 1];
+        pz[u] = h[u * kVeltenHead + 2];
+        c[u] = h[u * kVeltenHead + 3];
+        dso2[u] = h[u * kVeltenHead + 4];
+        half[u] = h[u * kVeltenHead + 5];
       }
-      if (est) {
-        float a[kVeltenUnroll];
+      float e[UN], a[UN];
+      int t[UN];
+      bool near = false;
 #pragma unroll
-        for (int u = 0; u < kVeltenUnroll; ++u) {
-          const float* r = base + (k + min(u, nu - 1)) * vr.len;
-          const float e = velten_sqdist(p[u], qx, qy, qz);
-          a[u] = r[4 + velten_take_bin<false>(r, vr, e, p[u].w, k2, T, 0.f, g) + 1];
-        }
-        if (nu == kVeltenUnroll) {
-#pragma unroll
-          for (int u = 0; u < kVeltenUnroll; ++u) value += a[u];            // :188-190
-        } else {
-#pragma unroll
-          for (int u = 0; u < kVeltenUnroll; ++u)
-            if (u < nu) value += a[u];
-        }
-      } else {
-        for (int u = 0; u < nu; ++u) {
-          const float* r = base + (k + u) * vr.len;
-          const float4 q = *(const float4*)r;
-          const float e = velten_sqdist(q, qx, qy, qz);
-          int t;
-          if (q.w == q.w) {
-            t = velten_take_bin<false>(r, vr, e, q.w, k2, T, 0.f, g);
-          } else {
-            const int s = s0 + k + u;
-            const float dso = So > 0 ? dist3(q.x, q.y, q.z, ob[3 * s], ob[3 * s + 1],
-                                             ob[3 * s + 2])
-                                     : 0.f;                                  // :178-183
-            t = velten_take_bin<true>(r, vr, e, q.w, k2, T, 2.f * dso, g);
-          }
-          value += r[4 + t + 1];  // bins -1 and T read the zero pads (:188-190)
-        }
+      for (int u = 0; u < UN; ++u) {
+        e[u] = velten_sqdist(px[u], py[u], pz[u], qx, qy, qz);
+        const float r = __builtin_fmaf(sqrt_fast(e[u]), k2, c[u]);
+        t[u] = floor_to_int(r);
+        near |= velten_near(r, half[u]);
       }
+      if (near) {
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+          if (velten_near(__builtin_fmaf(sqrt_fast(e[u]), k2, c[u]), half[u]))
+            t[u] = sqrt_mid_range(e[u]) && dw.ok
+                       ? floor_to_int(div_const(dso2[u] + 2.f * sqrt_rn_mid(e[u]) - g.off, dw) +
+                                      0.5f)
+                       : velten_bin(e[u], dso2[u], g.w, g.off);              // :177,185-187
+      }
+#pragma unroll
+      for (int u = 0; u < UN; ++u) a[u] = base[(k + u) * nv + velten_slot(t[u], T)];
+#pragma unroll
+      for (int u = 0; u < UN; ++u) value += a[u];                            // :188-190
+    }
+    for (; k < ns; ++k, h += kVeltenHead) {
+      const float e = velten_sqdist(h[0], h[1], h[2], qx, qy, qz);
+      const int t = velten_bin(e, h[4], g.w, g.off);
+      value += base[k * nv + velten_slot(t, T)];
+    }
+    if (STAGED) {
+      __syncthreads();  // these rows are no longer read, the next are written
+      cur ^= 1;
     }
   }
   if (ok) vol[(size_t)b * nvox + v] = value;                                 // :192
@@ -398,153 +327,99 @@ __global__ __launch_bounds__(256) void velten_confocal_kernel(
 // (backprojection_cuda.cu:228-287)
 //
 // The path length D is computed as the reference does (correctly rounded
-// roots, sums in its order).  Its bin floor((D - off) / w + 0.5) is a
-// non-decreasing function of D, the same for every pair, so one table of
-// thresholds D_k = min{D : bin(D) >= k} (bisection over the float bit
-// patterns) turns the division into an estimate a = floor(fma(D, 1/w,
-// 0.5 - off/w)), within one bin where D/w stays below 2^16 bins, and its
-// correction a - [D < D_a] + [D >= D_(a+1)].  The pair's constant terms
-// (the points and their origin distances) are computed once per pair.
+// roots, sums in its order).  Its two roots belong to the voxel and one
+// point each, so a lane computes |p_s - q| once per scan point, and keeps the
+// distances to up to sixteen laser points in registers for the whole call.
+// A pair is then two sums, a difference, the correctly rounded division by
+// the bin width as four multiply-adds (DivConst), + 0.5, floor and one
+// gather: about 13 vector instructions, which set its time.  64^3 voxels,
+// 256 x 16 points, 512 bins: 0.60 ms, against 1.76 ms with two roots and a
+// table correction (three gathers) per pair.
 // ---------------------------------------------------------------------------
 
-// One row of floats per (scan point, laser point) pair r = s * L + l, 16-byte
-// aligned parts:
-//   [0, 4)    p_s, |p_s - o_s|        [4, 8)  p_l, |p_l - o_l|
-//   [8, 12)   1 where the estimate's bound holds for the pair (else 0),
-//             1 where both points keep every squared distance to the box in
-//             [2^-64, 2^64] (the short correctly rounded root serves), 0, 0
-//   [12, 12 + nv)  its bins, vals[1 + t] = bin t, zeros at 0 and T + 1
-//                  (nv = T + 2 rounded up to a multiple of 4)
-struct ExRow {
-  int nv, len;
-};
+// Workspace of A3: headers of 8 floats per scan point, then per laser point,
+//   {x, y, z, |p - o|, reach, mid, 0, 0}: reach bounds |p - o| + |p - q| over
+//   the box (+inf for NaN), mid is 1 where every squared distance to the box
+//   lies in [2^-64, 2^64] (the short correctly rounded root serves),
+// then one row per pair r = s * L + l as in A2 (velten_row).
 
-__host__ __device__ __forceinline__ ExRow ex_row(int T) {
-  ExRow r;
-  r.nv = (T + 5) & ~3;
-  r.len = 12 + r.nv;
-  return r;
-}
-
-// Thread (b, r): the pair's constants and the zero pads of its bins.  The
-// estimate's error: the reference chain rounds the difference, the quotient
-// and + 0.5, the estimate 1/w, off/w, the constant and the FMA; under
-// 8 * 2^-24 * M bins for M = (D_max + |off|) / w + 1, D_max bounding D over
-// the box (origin terms plus the largest distances to the box's corners).
-// M < 2^16 keeps that far below one bin.
-__global__ __launch_bounds__(256) void velten_ex_rows_kernel(
+// Thread i of batch b: header i (scan points, then laser points), and the
+// zero slot of row i.
+__global__ __launch_bounds__(256) void velten_ex_head_kernel(
     const float* __restrict__ scan, const float* __restrict__ laser,
-    const float* __restrict__ sorig, const float* __restrict__ lorig, BoxGeom g, int S,
-    int L, int So, int Lo, float* __restrict__ rows) {
-  const ExRow xr = ex_row(g.T);
-  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (size_t)g.B * S * L) return;
-  const int b = (int)(id / ((size_t)S * L));
-  const int r = (int)(id - (size_t)b * S * L);
-  const int s = r / L, l = r - s * L;
-  const float* ps = scan + ((size_t)b * S + s) * 3;
-  const float* pl = laser + ((size_t)b * L + l) * 3;
-  const float px = ps[0], py = ps[1], pz = ps[2];
-  const float lx = pl[0], ly = pl[1], lz = pl[2];
-  float dso = 0.f, dlo = 0.f;
-  if (So > 0) {
-    const float* o = sorig + ((size_t)b * So + s) * 3;
-    dso = dist3(px, py, pz, o[0], o[1], o[2]);                               // :256-261
+    const float* __restrict__ sorig, const float* __restrict__ lorig, BoxGeom g, int S, int L,
+    int So, int Lo, float* __restrict__ head, float* __restrict__ rows) {
+  const int nv = velten_row(g.T);
+  const int b = blockIdx.y;
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < (size_t)S * L) rows[((size_t)b * S * L + i) * nv + g.T] = 0.f;
+  if (i >= (size_t)S + L) return;
+  const bool is_scan = i < (size_t)S;
+  const size_t k = is_scan ? (size_t)b * S + i : (size_t)b * L + (i - S);
+  const float* p = (is_scan ? scan : laser) + k * 3;
+  const float px = p[0], py = p[1], pz = p[2];
+  float o = 0.f;
+  if ((is_scan ? So : Lo) > 0) {
+    const float* q = (is_scan ? sorig : lorig) + k * 3;
+    o = dist3(px, py, pz, q[0], q[1], q[2]);                                 // :256-261,269-274
   }
-  if (Lo > 0) {
-    const float* o = lorig + ((size_t)b * Lo + l) * 3;
-    dlo = dist3(lx, ly, lz, o[0], o[1], o[2]);                               // :269-274
-  }
-  float ds = 0.f, dl = 0.f;
-  for (int c = 0; c < 8; ++c) {
-    const float cx = (c & 1) ? g.ex : g.sx, cy = (c & 2) ? g.ey : g.sy,
-                cz = (c & 4) ? g.ez : g.sz;
-    ds = fmaxf(ds, dist3(px, py, pz, cx, cy, cz));
-    dl = fmaxf(dl, dist3(lx, ly, lz, cx, cy, cz));
-  }
-  const float m = (dso + dlo + ds + dl + fabsf(g.off)) / g.w + 1.f;
-  const bool est = g.w > 0.f && m < kVeltenMaxBins;  // false for NaN or inf
+  float d = 0.f;
+  bool nan = !(px == px) || !(py == py) || !(pz == pz);
+  for (int c = 0; c < 8; ++c)
+    d = fmaxf(d, dist3(px, py, pz, (c & 1) ? g.ex : g.sx, (c & 2) ? g.ey : g.sy,
+                       (c & 4) ? g.ez : g.sz));
+  const float reach = o + d;
+  nan = nan || !(reach == reach);
   // at least 2^-20 from the box and at most 2^30 from its far corners
-  const float bs = box_sqdist(px, py, pz, g.sx, g.sy, g.sz, g.ex, g.ey, g.ez);
-  const float bl = box_sqdist(lx, ly, lz, g.sx, g.sy, g.sz, g.ex, g.ey, g.ez);
-  const bool mid = bs >= 0x1p-40f && bl >= 0x1p-40f && ds <= 0x1p30f && dl <= 0x1p30f;
-  float4* h = (float4*)(rows + id * xr.len);
-  h[0] = make_float4(px, py, pz, dso);
-  h[1] = make_float4(lx, ly, lz, dlo);
-  h[2] = make_float4(est ? 1.f : 0.f, mid ? 1.f : 0.f, 0.f, 0.f);
-  rows[id * xr.len + 12] = 0.f;
-  rows[id * xr.len + 12 + g.T + 1] = 0.f;
+  const float lo = box_sqdist(px, py, pz, g.sx, g.sy, g.sz, g.ex, g.ey, g.ez);
+  const bool mid = !nan && lo >= 0x1p-40f && d <= 0x1p30f;
+  float4* h = (float4*)(head + ((size_t)b * (S + L) + i) * kVeltenHead);
+  h[0] = make_float4(px, py, pz, o);
+  h[1] = make_float4(nan ? INFINITY : reach, mid ? 1.f : 0.f, 0.f, 0.f);
 }
 
-// Thread j in [0, T + 3): the path-length thresholds
-// {-inf, D_0, ..., D_T, NaN}, D_k = +inf when no finite D reaches bin k.
-__global__ __launch_bounds__(256) void velten_ex_table_kernel(BoxGeom g,
-                                                              float* __restrict__ tab) {
-  const int n = g.T + 3;
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  float d;
-  if (j == 0) {
-    d = -INFINITY;
-  } else if (j == n - 1) {
-    d = __builtin_nanf("");
+// |p - q| of N points with headers at h (uniform), every stride-th float: one
+// uniform test for all, so that the header loads are in flight together.
+template <int N, typename At>
+__device__ __forceinline__ void ex_head_dists(At at, float qx, float qy, float qz, float (&d)[N]) {
+  float mid = 1.f;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    d[j] = velten_sqdist(at(j)[0], at(j)[1], at(j)[2], qx, qy, qz);
+    mid = fminf(mid, at(j)[5]);
+  }
+  if (mid != 0.f) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) d[j] = sqrt_rn_mid(d[j]);                    // :255,268
   } else {
-    const int k = j - 1;
-    unsigned lo = 0u, hi = 0x7f800000u;
-    if (nearest_bin(0.f, g.w, g.off) >= k) {
-      hi = 0u;
-    } else {
-      while (hi - lo > 1u) {
-        const unsigned mid = lo + (hi - lo) / 2u;
-        if (nearest_bin(__uint_as_float(mid), g.w, g.off) >= k)
-          hi = mid;
-        else
-          lo = mid;
-      }
-    }
-    d = __uint_as_float(hi);
+#pragma unroll
+    for (int j = 0; j < N; ++j) d[j] = sqrt_rn(d[j]);
   }
-  tab[j] = d;
 }
 
-// Bin of one (voxel, pair): D as the reference computes it (MID: with the
-// short correctly rounded root, the same values), then the corrected estimate
-// (EST) or the reference's division; clamped to [-1, T].
-template <bool EST, bool MID>
-__device__ __forceinline__ int velten_ex_bin(const float* row, const float* tab, float qx,
-                                             float qy, float qz, float rw, float c0,
-                                             const BoxGeom& g) {
-  const float4 hs = *(const float4*)row, hl = *(const float4*)(row + 4);
-  const float dsv = MID ? sqrt_rn_mid(sqdist3(hs.x, hs.y, hs.z, qx, qy, qz))
-                        : dist3(hs.x, hs.y, hs.z, qx, qy, qz);                // :255
-  const float dlv = MID ? sqrt_rn_mid(sqdist3(hl.x, hl.y, hl.z, qx, qy, qz))
-                        : dist3(hl.x, hl.y, hl.z, qx, qy, qz);                // :268
-  float dist = hs.w + dsv;                                                   // :276-277
-  dist = dist + dlv;
-  dist = dist + hl.w;
-  if (EST) {
-    int a = (int)floorf(__builtin_fmaf(dist, rw, c0));
-    a = min(max(a, -1), g.T);
-    return a + (dist < tab[a + 1] ? -1 : 0) + (dist >= tab[a + 2] ? 1 : 0);
-  }
-  const int t = nearest_bin(dist, g.w, g.off);                               // :279
-  return min(max(t, -1), g.T);
+// A unit of the exhaustive walk: SG scan points and a tile of KT laser points,
+// up to sixteen pairs whose decisions and gathers overlap (eight: 0.79 ms at
+// the size above), or up to eight where the stage does not hold sixteen rows.  Several scan points only where
+// one tile holds all laser points (KT = L).
+__host__ __device__ constexpr int ex_scan_group(int KT, int pairs) {
+  return KT <= 6 ? (pairs / KT > 1 ? pairs / KT : 1) : 1;
 }
 
-// One lane per voxel, flat over [D][H][W]; rows as laid out above, the
-// threshold table in LDS.  Rows are staged in LDS as in A2 (STAGED), or read
-// from global memory (long rows).  Sums run over pairs in the reference's
-// order (scan point outer, laser point inner).
-template <bool STAGED>
-__global__ __launch_bounds__(256) void velten_exhaustive_kernel(
-    const float* __restrict__ rows, const float* __restrict__ gtab, float* __restrict__ vol,
-    BoxGeom g, int NR, int R, float rw, float c0) {
+// One lane per voxel, flat over [D][H][W].  The rows of U consecutive units
+// are staged in LDS (STAGED), or read from global memory (long rows).  NTL:
+// tiles whose distances stay in registers (L <= NTL * KT), or 0 (computed per
+// unit).  Sums run over pairs in the reference's order (scan point outer,
+// laser point inner).
+template <int KT, int NTL, int SG, bool STAGED, int NTH>
+__global__ __launch_bounds__(NTH) void velten_exhaustive_kernel(
+    const float* __restrict__ head, const float* __restrict__ rows, float* __restrict__ vol,
+    BoxGeom g, int S, int L, int U, int cap, DivConst dw) {
   extern __shared__ float4 lds4[];
   const int T = g.T;
-  const ExRow xr = ex_row(T);
+  const int nv = velten_row(T);
   const int b = blockIdx.y;
   const int nvox = g.D * g.H * g.W;
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  const int v = blockIdx.x * NTH + threadIdx.x;
   const bool ok = v < nvox;
   const int vv = ok ? v : 0;
   const int x = vv % g.W;
@@ -553,82 +428,130 @@ __global__ __launch_bounds__(256) void velten_exhaustive_kernel(
   const float qx = inclusive_coord(x, g.W, g.sx, g.ex);
   const float qy = inclusive_coord(y, g.H, g.sy, g.ey);
   const float qz = inclusive_coord(z, g.D, g.sz, g.ez);
-  const size_t bR = (size_t)b * NR;
-  // LDS: the threshold table (T + 3 floats, rounded to float4s), then the stage
-  const int ntab4 = (T + 6) / 4;
-  float* tab = (float*)lds4;
-  float* stage = (float*)(lds4 + ntab4);
-  const float* tb = gtab;
+  const float* hs = head + (size_t)b * (S + L) * kVeltenHead;
+  const float* hl = hs + (size_t)S * kVeltenHead;
+  const float* rb = rows + (size_t)b * S * L * nv;
+  const int NT = (L + KT - 1) / KT;  // 1 where SG > 1
+  const int n_units = (S + SG - 1) / SG * NT;
+  // first row of unit u <= n_units
+  auto unit_row = [&](int u) { return min(u / NT * SG, S) * L + u % NT * KT; };
+
+  float dl[NTL > 0 ? NTL : 1][KT];
+  float reach[NTL > 0 ? NTL : 1];
+  auto laser_tile = [&](int k, float (&d)[KT], float& rch) {
+    rch = 0.f;
+    auto at = [&](int j) { return hl + min(k * KT + j, L - 1) * kVeltenHead; };
+    ex_head_dists<KT>(at, qx, qy, qz, d);
+#pragma unroll
+    for (int j = 0; j < KT; ++j) rch = fmaxf(rch, at(j)[4]);
+  };
+#pragma unroll
+  for (int k = 0; k < NTL; ++k) laser_tile(k, dl[k], reach[k]);
+
+  float* stage = (float*)lds4;
+  RowStage<NTH> next;
+  auto unit_n4 = [&](int u0) { return (unit_row(min(u0 + U, n_units)) - unit_row(u0)) * nv / 4; };
+  auto load = [&](int u0) { next.load(rb + (size_t)unit_row(u0) * nv, unit_n4(u0)); };
   if (STAGED) {
-    for (int e = threadIdx.x; e < T + 3; e += blockDim.x) tab[e] = gtab[e];
-    tb = tab;
+    load(0);
+    next.store(stage, unit_n4(0));
+    if (U < n_units) load(U);
+    __syncthreads();
   }
-  float4 buf[kVeltenCopy4];
-  if (STAGED) {
-    const int n4 = min(R, NR) * xr.len / 4;
-    const float4* src = (const float4*)(rows + bR * xr.len);
+
+  float value = 0.f, as[SG], rs = 0.f;
+  // One unit: scan points s .. s + SG - 1 (as: |p - o| + |p - q| of each, rs:
+  // their largest reach), tile k, its rows at base.
+  auto unit = [&](const float* base, int s, int k, const float (&d)[KT], float rch) {
+    const int ns = min(SG, S - s), nl = min(KT, L - k * KT);
+    const float* h = hl + k * KT * kVeltenHead;
+    float lo[KT];
 #pragma unroll
-    for (int i = 0; i < kVeltenCopy4; ++i) {
-      const int e = i * 256 + (int)threadIdx.x;
-      buf[i] = e < n4 ? src[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  }
-  float value = 0.f;
-  for (int r0 = 0; r0 < NR; r0 += R) {
-    const int nr = min(R, NR - r0);
-    const float* base = rows + (bR + r0) * xr.len;
-    if (STAGED) {
-      __syncthreads();  // the previous group is no longer read
-      const int n4 = nr * xr.len / 4;
+    for (int j = 0; j < KT; ++j) lo[j] = h[min(j, nl - 1) * kVeltenHead + 3];
+    float dist[SG][KT];
 #pragma unroll
-      for (int i = 0; i < kVeltenCopy4; ++i) {
-        const int e = i * 256 + (int)threadIdx.x;
-        if (e < n4) ((float4*)stage)[e] = buf[i];
+    for (int i = 0; i < SG; ++i)
+#pragma unroll
+      for (int j = 0; j < KT; ++j) {
+        dist[i][j] = as[i] + d[j];                                           // :276-277
+        dist[i][j] = dist[i][j] + lo[j];
       }
-      __syncthreads();
-      if (r0 + R < NR) {
-        const int n4n = min(R, NR - r0 - R) * xr.len / 4;
-        const float4* src = (const float4*)(rows + (bR + r0 + R) * xr.len);
+    // false for NaN or inf; uniform
+    if (dw.ok && (rs + rch + fabsf(g.off)) * dw.hi < kVeltenMaxBins) {
+      unsigned at[SG][KT];
 #pragma unroll
-        for (int i = 0; i < kVeltenCopy4; ++i) {
-          const int e = i * 256 + (int)threadIdx.x;
-          buf[i] = e < n4n ? src[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-      }
-      base = stage;
-    }
-    // groups of kVeltenUnroll pairs, as in A2
-    for (int k = 0; k < nr; k += kVeltenUnroll) {
-      const int nu = min(kVeltenUnroll, nr - k);
-      bool est = true;
+      for (int i = 0; i < SG; ++i)
 #pragma unroll
-      for (int u = 0; u < kVeltenUnroll; ++u) {
-        const float* r = base + (k + min(u, nu - 1)) * xr.len;
-        est = est && r[8] != 0.f && r[9] != 0.f;
-      }
-      if (est) {
-        float a[kVeltenUnroll];
+        for (int j = 0; j < KT; ++j)
+          at[i][j] = velten_slot(floor_to_int(div_const(dist[i][j] - g.off, dw) + 0.5f), T);  // :279
+      if (ns == SG && nl == KT) {
+        float a[SG][KT];
+        const float* row = base;
 #pragma unroll
-        for (int u = 0; u < kVeltenUnroll; ++u) {
-          const float* r = base + (k + min(u, nu - 1)) * xr.len;
-          a[u] = r[12 + velten_ex_bin<true, true>(r, tb, qx, qy, qz, rw, c0, g) + 1];
-        }
-        if (nu == kVeltenUnroll) {
+        for (int i = 0; i < SG; ++i)
 #pragma unroll
-          for (int u = 0; u < kVeltenUnroll; ++u) value += a[u];            // :280-282
-        } else {
+          for (int j = 0; j < KT; ++j, row += nv) a[i][j] = row[at[i][j]];
 #pragma unroll
-          for (int u = 0; u < kVeltenUnroll; ++u)
-            if (u < nu) value += a[u];
-        }
+        for (int i = 0; i < SG; ++i)
+#pragma unroll
+          for (int j = 0; j < KT; ++j) value += a[i][j];                     // :280-282
       } else {
-        for (int u = 0; u < nu; ++u) {
-          const float* r = base + (k + u) * xr.len;
-          const int t = r[8] != 0.f ? velten_ex_bin<true, false>(r, tb, qx, qy, qz, rw, c0, g)
-                                    : velten_ex_bin<false, false>(r, tb, qx, qy, qz, rw, c0, g);
-          value += r[12 + t + 1];  // bins -1 and T read the zero pads (:280-282)
+#pragma unroll
+        for (int i = 0; i < SG; ++i)
+#pragma unroll
+          for (int j = 0; j < KT; ++j)
+            if (i < ns && j < nl) value += base[(i * nl + j) * nv + at[i][j]];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < SG; ++i)
+#pragma unroll
+        for (int j = 0; j < KT; ++j)
+          if (i < ns && j < nl)
+            value += base[(i * nl + j) * nv +
+                          velten_slot(nearest_bin(dist[i][j], g.w, g.off), T)];
+    }
+  };
+
+  int s = 0, k = 0;  // the next unit's first scan point and tile
+  int cur = 0;
+  for (int u0 = 0; u0 < n_units; u0 += U) {
+    const int ue = min(u0 + U, n_units);
+    const float* base = STAGED ? stage + cur * cap : rb + (size_t)unit_row(u0) * nv;
+    if (STAGED && ue < n_units) {
+      next.store(stage + (cur ^ 1) * cap, unit_n4(ue));
+      if (ue + U < n_units) load(ue + U);
+    }
+    for (int u = u0; u < ue; ++u) {
+      if (k == 0) {
+        rs = 0.f;
+        auto at = [&](int i) { return hs + (size_t)min(s + i, S - 1) * kVeltenHead; };
+        ex_head_dists<SG>(at, qx, qy, qz, as);
+#pragma unroll
+        for (int i = 0; i < SG; ++i) {
+          as[i] = at(i)[3] + as[i];                                          // :276-277
+          rs = fmaxf(rs, at(i)[4]);
         }
       }
+      if constexpr (NTL == 0) {
+        laser_tile(k, dl[0], reach[0]);
+        unit(base, s, k, dl[0], reach[0]);
+      } else if constexpr (NTL == 1) {
+        unit(base, s, 0, dl[0], reach[0]);
+      } else {
+#pragma unroll
+        for (int c = 0; c < NTL; ++c)
+          if (k == c) unit(base, s, c, dl[c], reach[c]);
+      }
+      base += (size_t)(min(SG, S - s) * min(KT, L - k * KT)) * nv;
+      if (++k == NT) {
+        k = 0;
+        s += SG;
+      }
+    }
+    if (STAGED) {
+      __syncthreads();  // these rows are no longer read, the next are written
+      cur ^= 1;
     }
   }
   if (ok) vol[(size_t)b * nvox + v] = value;                                 // :285
@@ -853,9 +776,12 @@ using namespace totri_hip;
 namespace totri_hip {
 namespace {
 
-// Workspace of A2: one row per scan point (velten_row), [B][S][len] floats.
+// Scratch that A2 asks for, per scan point: room for two floats per bin,
+// which bounds what the allocation-free entry point takes.  Its headers and
+// rows need about half of it.
 size_t velten_bytes(int64_t B, int64_t T, int64_t S) {
-  return align256((size_t)B * S * velten_row((int)T).len * sizeof(float));
+  const size_t len = 4 + (((size_t)T + 5) & ~(size_t)3) + (((size_t)T + 6) & ~(size_t)3);
+  return align256((size_t)B * S * len * sizeof(float));
 }
 
 }  // namespace
@@ -901,31 +827,37 @@ int velten_confocal(const float* transient, int64_t B, int64_t T, int64_t S,
                 workspace_bytes);
   TOTRI_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace & 15) == 0,
                   "workspace must be a non-null, 16-byte aligned device pointer");
-  float* rows = (float*)workspace;
-  const VeltenRow vr = velten_row((int)T);
-  rc = transpose_strided(transient, rows, (int)B, (int)T, (int)S, vr.len, 5, st);
+  // headers, then rows: 8 + nv floats per scan point, of the 4 + nv + nt
+  // (nt >= 4) asked for
+  float* head = (float*)workspace;
+  float* rows = head + (size_t)B * S * kVeltenHead;
+  const int nv = velten_row((int)T);
+  rc = transpose_strided(transient, rows, (int)B, (int)T, (int)S, nv, 0, st);
   if (rc) return rc;
   const float rw = 1.f / bin_width;
-  const size_t nthr = (size_t)B * S * (T + 3);
-  hipLaunchKernelGGL(velten_bins_kernel, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st,
-                     scan_points, scan_origin, g, (int)S, (int)So, rw, rows);
-  rc = check_launch("velten_bins_kernel");
+  hipLaunchKernelGGL(velten_head_kernel, dim3((unsigned)((B * S + 255) / 256)), dim3(256), 0, st,
+                     scan_points, scan_origin, g, (int)S, (int)So, rw, head, rows);
+  rc = check_launch("velten_head_kernel");
   if (rc) return rc;
-  // Scan points per LDS stage.  Where fewer than four rows fit (T above
-  // about 1020 bins) the stage's barriers would come every few points: the
-  // rows are then read from global memory, through the caches.
-  int R = (int)std::min<int64_t>(S, kVeltenStage / vr.len);
-  if (R < 4 && R < S) R = 0;
+  // Scan points per LDS stage: whole groups of eight, or four.  Where fewer
+  // rows fit (T above about 2550) the stage's barriers would come every few
+  // points: the rows are then read from global memory, through the caches.
+  const StagePlan sp = stage_plan(B, (int64_t)nvox);
+  int R = sp.cap / nv;
+  R = R >= 8 ? R & ~7 : R & ~3;
   const float k2 = 2.f * rw;
-  const dim3 grid(blocks_for(nvox), (unsigned)B);
-  if (R > 0) {
-    hipLaunchKernelGGL(velten_confocal_kernel<true>, grid, dim3(256),
-                       (size_t)R * vr.len * sizeof(float), st, rows, scan_origin, volume, g,
-                       (int)S, (int)So, R, k2);
-  } else {
-    hipLaunchKernelGGL(velten_confocal_kernel<false>, grid, dim3(256), 0, st, rows,
-                       scan_origin, volume, g, (int)S, (int)So, (int)S, k2);
-  }
+  const bool wide = sp.threads == 1024;
+  auto kernel = R >= 8  ? (wide ? velten_confocal_kernel<true, 8, 1024>
+                                : velten_confocal_kernel<true, 8, 256>)
+                : R > 0 ? (wide ? velten_confocal_kernel<true, 4, 1024>
+                                : velten_confocal_kernel<true, 4, 256>)
+                        : velten_confocal_kernel<false, 8, 256>;
+  const int threads = R > 0 ? sp.threads : 256;
+  rc = allow_stage(kernel);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(nvox, threads), (unsigned)B), dim3(threads),
+                     R > 0 ? 2 * (size_t)sp.cap * sizeof(float) : 0, st, head, rows, volume, g,
+                     (int)S, R > 0 ? R : (int)S, sp.cap, k2, make_div_const(g.w));
   return check_launch("velten_confocal_kernel");
 }
 
@@ -1003,16 +935,83 @@ extern "C" int totri_backprojection_confocal_velten_forward_noalloc(
 namespace totri_hip {
 namespace {
 
-// Workspace of A3: the pair rows [B][S*L][len], then the threshold table.
+// Workspace of A3: the point headers, then the pair rows [B][S*L][nv].
 struct ExLayout {
-  size_t tab_off, end;
+  size_t rows_off, end;
 };
 
 ExLayout ex_layout(int64_t B, int64_t T, int64_t S, int64_t L) {
   ExLayout l;
-  l.tab_off = align256((size_t)B * S * L * ex_row((int)T).len * sizeof(float));
-  l.end = align256(l.tab_off + (size_t)(T + 3) * sizeof(float));
+  l.rows_off = align256((size_t)B * (S + L) * kVeltenHead * sizeof(float));
+  l.end = l.rows_off + align256((size_t)B * S * L * velten_row((int)T) * sizeof(float));
   return l;
+}
+
+template <int KT, int NTL, int SG>
+int launch_velten_ex(const float* head, const float* rows, float* volume, const BoxGeom& g,
+                     int64_t S, int64_t L, const StagePlan& sp, hipStream_t st) {
+  const int nv = velten_row(g.T);
+  const int64_t NT = (L + KT - 1) / KT;
+  // Units per LDS stage: whole scan points, else one tile of a scan point.
+  int64_t U = 1;
+  if (SG * L * nv <= sp.cap)
+    U = std::min<int64_t>((S + SG - 1) / SG, sp.cap / (SG * L * nv)) * NT;
+  auto kernel = sp.threads == 1024 ? velten_exhaustive_kernel<KT, NTL, SG, true, 1024>
+                                   : velten_exhaustive_kernel<KT, NTL, SG, true, 256>;
+  const int rc = allow_stage(kernel);
+  if (rc) return rc;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for((size_t)g.D * g.H * g.W, sp.threads), (unsigned)g.B),
+                     dim3(sp.threads), 2 * (size_t)sp.cap * sizeof(float), st, head, rows, volume,
+                     g, (int)S, (int)L, (int)U, sp.cap, make_div_const(g.w));
+  return check_launch("velten_exhaustive_kernel");
+}
+
+// The tile size for L laser points, tiles of at most 16 points and `most`
+// rows: tiles of equal size, rounded up to one that is compiled.  A tile
+// that is not full masks its last points, so all laser points of a call with
+// several scan points per unit (L <= 6) make exactly one tile.
+int velten_ex_tile(int64_t L, int64_t most) {
+  static const int sizes[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
+  int top = 0;
+  for (int k : sizes)
+    if (k <= most) top = k;
+  if (top == 0 || (L > top && top < 7)) return 0;
+  const int64_t nt = (L + top - 1) / top, kt = (L + nt - 1) / nt;
+  for (int k : sizes)
+    if (k >= kt) return k;
+  return 0;
+}
+
+int velten_ex(const float* head, const float* rows, float* volume, const BoxGeom& g, int64_t S,
+              int64_t L, hipStream_t st) {
+  const size_t nvox = (size_t)g.D * g.H * g.W;
+  const StagePlan sp = stage_plan(g.B, (int64_t)nvox);
+  const int64_t fit = sp.cap / velten_row(g.T);
+  int kt = velten_ex_tile(L, fit);
+  const int pairs = ex_scan_group(kt > 0 ? kt : 1, 16) * (int64_t)kt <= fit ? 16 : 8;
+  if (kt > 0 && ex_scan_group(kt, pairs) * (int64_t)kt > fit) kt = 0;
+  if (kt == 0) {  // rows longer than the stage: read from global memory
+    const int64_t nt = (L + 7) / 8;
+    hipLaunchKernelGGL((velten_exhaustive_kernel<8, 0, 1, false, 256>),
+                       dim3(blocks_for(nvox), (unsigned)g.B), dim3(256), 0, st, head, rows,
+                       volume, g, (int)S, (int)L, (int)(S * nt), 0, make_div_const(g.w));
+    return check_launch("velten_exhaustive_kernel");
+  }
+  const int64_t nt = (L + kt - 1) / kt;
+#define TOTRI_EX(KT, NTL) \
+  if (kt == KT && (nt > 3 ? 0 : nt) == NTL) \
+    return launch_velten_ex<KT, NTL, 1>(head, rows, volume, g, S, L, sp, st);
+#define TOTRI_EX4(KT) TOTRI_EX(KT, 1) TOTRI_EX(KT, 2) TOTRI_EX(KT, 3) TOTRI_EX(KT, 0)
+#define TOTRI_EX1(KT) \
+  if (kt == KT) \
+    return pairs == 16 ? launch_velten_ex<KT, 1, ex_scan_group(KT, 16)>(head, rows, volume, g, S, L, sp, st) \
+                       : launch_velten_ex<KT, 1, ex_scan_group(KT, 8)>(head, rows, volume, g, S, L, sp, st);
+  TOTRI_EX1(1) TOTRI_EX1(2) TOTRI_EX1(3) TOTRI_EX1(4) TOTRI_EX1(5) TOTRI_EX1(6)
+  TOTRI_EX4(7) TOTRI_EX4(8) TOTRI_EX4(10) TOTRI_EX4(12) TOTRI_EX4(14) TOTRI_EX4(16)
+#undef TOTRI_EX1
+#undef TOTRI_EX4
+#undef TOTRI_EX
+  return fail(TOTRI_EINVAL, "no kernel for tiles of %d laser points", kt);
 }
 
 }  // namespace
@@ -1054,38 +1053,18 @@ extern "C" int totri_backprojection_exhaustive_velten_forward(
                 workspace_bytes);
   TOTRI_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace & 15) == 0,
                   "workspace must be a non-null, 16-byte aligned device pointer");
-  float* rows = (float*)workspace;
-  float* tab = (float*)((char*)workspace + lay.tab_off);
-  const ExRow xr = ex_row((int)T);
-  const int NR = (int)(S * L);
-  rc = transpose_strided(transient, rows, (int)B, (int)T, NR, xr.len, 13, st);
+  float* head = (float*)workspace;
+  float* rows = (float*)((char*)workspace + lay.rows_off);
+  const int nv = velten_row((int)T);
+  rc = transpose_strided(transient, rows, (int)B, (int)T, (int)(S * L), nv, 0, st);
   if (rc) return rc;
-  const size_t npairs = (size_t)B * NR;
-  hipLaunchKernelGGL(velten_ex_rows_kernel, dim3((unsigned)((npairs + 255) / 256)), dim3(256),
-                     0, st, scan_points, laser_points, scan_origin, laser_origin, g, (int)S,
-                     (int)L, (int)So, (int)Lo, rows);
-  rc = check_launch("velten_ex_rows_kernel");
+  const int64_t n_head = std::max<int64_t>(S * L, S + L);
+  hipLaunchKernelGGL(velten_ex_head_kernel, dim3((unsigned)((n_head + 255) / 256), (unsigned)B),
+                     dim3(256), 0, st, scan_points, laser_points, scan_origin, laser_origin, g,
+                     (int)S, (int)L, (int)So, (int)Lo, head, rows);
+  rc = check_launch("velten_ex_head_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(velten_ex_table_kernel, dim3((unsigned)((T + 3 + 255) / 256)), dim3(256), 0,
-                     st, g, tab);
-  rc = check_launch("velten_ex_table_kernel");
-  if (rc) return rc;
-  const float rw = 1.f / bin_width;
-  const float c0 = -bin_offset * rw + 0.5f;
-  // pairs per LDS stage (beside the table); with fewer than four per stage
-  // the rows and the table are read from global memory
-  int R = (int)std::min<int64_t>(NR, kVeltenStage / xr.len);
-  if (R < 4 && R < NR) R = 0;
-  const dim3 grid(blocks_for(nvox), (unsigned)B);
-  if (R > 0) {
-    const size_t lds = ((size_t)(T + 6) / 4 * 4 + (size_t)R * xr.len) * sizeof(float);
-    hipLaunchKernelGGL(velten_exhaustive_kernel<true>, grid, dim3(256), lds, st, rows, tab,
-                       volume, g, NR, R, rw, c0);
-  } else {
-    hipLaunchKernelGGL(velten_exhaustive_kernel<false>, grid, dim3(256), 0, st, rows, tab,
-                       volume, g, NR, NR, rw, c0);
-  }
-  return check_launch("velten_exhaustive_kernel");
+  return velten_ex(head, rows, volume, g, S, L, st);
 }
 
 namespace totri_hip {

@@ -82,6 +82,34 @@ __device__ __forceinline__ float sqrt_fast(float x) {
   return __builtin_amdgcn_sqrtf(x);
 }
 
+// Division of many values by one w, correctly rounded, in four operations
+// (the compiler's division takes eleven).  With hi = RN(1/w) and lo the rest
+// of 1/w, q = fma(x, hi, x lo) lies within one ulp of x / w, the residual
+// r = x - q w is exact, and RN(q + r hi) is the correctly rounded quotient
+// (Markstein's theorem, which asks for a correctly rounded hi and such a q).
+// `ok` is false where an exponent could leave the range this holds in; x must
+// be finite and below 2^60 in magnitude.  Quotients that underflow are
+// not exact, which no bin decision sees.
+struct DivConst {
+  float w, hi, lo;
+  int ok;
+};
+
+inline DivConst make_div_const(float w) {
+  DivConst d;
+  d.w = w;
+  d.hi = 1.f / w;
+  d.lo = (float)(1.0 / (double)w - (double)d.hi);
+  d.ok = w >= 0x1p-40f && w <= 0x1p40f ? 1 : 0;
+  return d;
+}
+
+__device__ __forceinline__ float div_const(float x, const DivConst& d) {
+  const float q = __builtin_fmaf(x, d.hi, x * d.lo);
+  const float r = __builtin_fmaf(-q, d.w, x);
+  return __builtin_fmaf(r, d.hi, q);
+}
+
 // tc = t * w + off, rounded after the product and after the sum
 // (src/render/volume_cuda.cu:23).
 __device__ __forceinline__ float bin_distance(int t, float w, float off) {
