@@ -1,0 +1,82 @@
+"""Exhaustive render adjoint (A5) against the FP64-summed oracle at the edges of
+its forms: laser tiles of 1 to 8 points and several, scan points with and
+without a remainder, spans of at most 2 and 6 bins (masked reads) and of
+dozens (running sums), histograms that cut voxels off at both ends, rows too
+long for a stage, 256 and 1024 lanes, and a gradient with an infinity.
+
+Tolerance 1e-6 relative L2, that of the existing adjoint test: the oracle's
+weights are the same FP32 numbers to an ulp of frac, summed in double; here a
+voxel sums a few hundred pairs in float (2^-24 each, random signs)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.cases import rel_l2
+
+VS, VE = (-1.0, -1.0, 0.5), (1.0, 1.0, 2.5)
+
+
+def t(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def adjoint(G, res, scan, laser, w, off):
+    from totrilib_amd.totri_cpp.render import volume_render_exhaustive_grad_volume
+    B = G.shape[0]
+    out = torch.empty((B,) + res, device="cuda")
+    empty = torch.empty(B, 3, 0, device="cuda")
+    volume_render_exhaustive_grad_volume(t(G), t(scan), t(laser), empty, empty, out, VS, VE, w, off)
+    return out.cpu().numpy()
+
+
+def points(rng, B, n):
+    return np.concatenate([rng.uniform(-1, 1, (B, 2, n)), np.zeros((B, 1, n))], 1).astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [1, 2, 3, 4, 5, 7, 8, 9, 17])
+@pytest.mark.parametrize("T,w,off,D", [
+    (40, 0.2, 0.0, 20),      # spans within 2 bins
+    (150, 0.05, 0.0, 20),    # within 6 bins
+    (60, 0.05, 3.0, 20),     # cut off at both ends
+    (700, 0.0115, 0.0, 6),   # dozens of bins
+    (200, 0.0115, 3.5, 6),   # dozens, cut off
+])
+def test_adjoint_tiles(L, T, w, off, D):
+    rng = np.random.default_rng(L + T)
+    B, S, res = 2, 9, (D, 5, 7)
+    scan, laser = points(rng, B, S), points(rng, B, L)
+    G = rng.standard_normal((B, T, S, L)).astype(np.float32)
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, off, mode=O.PINNED64)
+    assert ref.any()
+    assert rel_l2(adjoint(G, res, scan, laser, w, off), ref) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("res", [(64, 48, 65), (5, 6, 7)])     # 1024 and 256 lanes
+@pytest.mark.parametrize("T", [64, 1100, 2600, 9000])
+def test_adjoint_stages(res, T):
+    rng = np.random.default_rng(T)
+    w = 8.0 / T
+    scan, laser = points(rng, 1, 3), points(rng, 1, 2)
+    G = rng.standard_normal((1, T, 3, 2)).astype(np.float32)
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64)
+    assert rel_l2(adjoint(G, res, scan, laser, w, 0.0), ref) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D", [(150, 20), (700, 6)])
+def test_adjoint_infinite_gradient(T, D):
+    """An infinity reaches the voxels whose spans hold its bin, and no others."""
+    rng = np.random.default_rng(T)
+    res, w = (D, 5, 7), 8.0 / T
+    scan, laser = points(rng, 1, 3), points(rng, 1, 2)
+    G = rng.standard_normal((1, T, 3, 2)).astype(np.float32)
+    G[0, T // 2, 1, 1] = np.inf
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64)
+    got = adjoint(G, res, scan, laser, w, 0.0)
+    fine = np.isfinite(ref)
+    assert 0 < np.count_nonzero(~fine) < fine.size
+    assert np.array_equal(np.isfinite(got), fine)
+    assert rel_l2(got[fine], ref[fine]) < 1e-6

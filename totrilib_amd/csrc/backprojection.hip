@@ -29,6 +29,7 @@
 
 #include "common.h"
 #include "compact.h"
+#include "stage.h"
 
 namespace totri_hip {
 namespace {
@@ -173,58 +174,6 @@ __device__ __forceinline__ bool velten_near(float r, float half) {
 // Slot of bin t: bins outside [0, T) read the zero at T.
 __device__ __forceinline__ unsigned velten_slot(int t, int T) {
   return min((unsigned)t, (unsigned)T);
-}
-
-// Staged rows (A2, A3): two LDS buffers of `cap` floats.  A workgroup writes
-// the next rows, loaded into registers one stage earlier, into one buffer
-// while its waves read the other, so a stage costs one barrier.  Every
-// workgroup reads all rows, so L2 traffic falls with the voxels per workgroup:
-// at 64^3 and 4096 pairs of 512 bins, 1024 lanes (one workgroup per CU) read
-// 2.1 GB where 256 lanes read 8.6 GB (A3: 0.85 -> 0.79 ms).  Volumes that
-// would leave a quarter of the CUs without a workgroup of 1024 keep 256 lanes.
-// Floats per buffer, at most: 72 KiB where a workgroup has a CU to itself,
-// else 40 KiB.
-constexpr int stage_max(int threads) { return threads == 1024 ? 18432 : 10240; }
-
-template <int NTH>
-struct RowStage {
-  static constexpr int kCopy4 = (stage_max(NTH) / 4 + NTH - 1) / NTH;
-  float4 buf[kCopy4];
-  // n4 float4s, 0 <= n4 <= stage_max(NTH) / 4
-  __device__ __forceinline__ void load(const float* src, int n4) {
-#pragma unroll
-    for (int i = 0; i < kCopy4; ++i) {
-      const int e = i * NTH + (int)threadIdx.x;
-      buf[i] = e < n4 ? ((const float4*)src)[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  }
-  __device__ __forceinline__ void store(float* dst, int n4) const {
-#pragma unroll
-    for (int i = 0; i < kCopy4; ++i) {
-      const int e = i * NTH + (int)threadIdx.x;
-      if (e < n4) ((float4*)dst)[e] = buf[i];
-    }
-  }
-};
-
-// Lets a kernel take both buffers (launches get 64 KiB by default).
-template <typename K>
-int allow_stage(K kernel) {
-  TOTRI_CHECK_HIP(hipFuncSetAttribute((const void*)kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      2 * stage_max(1024) * (int)sizeof(float)));
-  return TOTRI_OK;
-}
-
-// Workgroup size and floats per buffer for B volumes of nvox voxels.
-struct StagePlan {
-  int threads, cap;
-};
-
-StagePlan stage_plan(int64_t B, int64_t nvox) {
-  if (B * ((nvox + 1023) / 1024) >= 192) return {1024, stage_max(1024)};
-  // up to two workgroups per CU take full buffers, more of them half
-  return {256, B * ((nvox + 255) / 256) <= 512 ? stage_max(256) : stage_max(256) / 2};
 }
 
 // One lane per voxel, flat over [D][H][W].  The rows of R scan points at a

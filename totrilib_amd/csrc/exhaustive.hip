@@ -24,8 +24,12 @@
 // IEEE correctly rounded square roots and divisions.
 #include <math.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "compact.h"
+#include "stage.h"
 
 namespace totri_hip {
 namespace {
@@ -35,7 +39,8 @@ constexpr int kR2Waves = 4;
 // KiB of LDS.  Longer transients take several tiles (grid z), each pass
 // recomputing the voxel spans and keeping the bins of its tile.
 constexpr int kR2Tile = 64 * 1024 / (kR2Waves * (int)sizeof(long long));
-constexpr int kStage = 8192;  // floats of staged gradient rows (32 KiB)
+
+size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct ExGeom {
   int B, D, H, W, T;
@@ -63,24 +68,11 @@ struct Span {
   float wf, wm, wl;     // weights of the first, inner and last bins
 };
 
-// Bin span and weights of one voxel for one (scan, laser) pair
-// (volume_cuda.cu:339-374).  With first == last the whole occupancy goes to
+// Bin span and weights of one voxel whose faces have path lengths d0 and d1
+// (volume_cuda.cu:341-374).  With first == last the whole occupancy goes to
 // that bin (wf = occ).
-// MID: every radicand lies in [2^-64, 2^64] (both points keep a distance
-// from the box, sqrt_mid_range), so the short correctly rounded root serves.
-template <bool MID>
-__device__ __forceinline__ float ex_dist(float ax, float ay, float az, float bx, float by,
-                                         float bz) {
-  return MID ? sqrt_rn_mid(sqdist3(ax, ay, az, bx, by, bz)) : dist3(ax, ay, az, bx, by, bz);
-}
-
-template <bool MID>
-__device__ __forceinline__ Span voxel_span(const ExGeom& g, float occ, float xf, float yf,
-                                           float zf0, float zf1, float spx, float spy,
-                                           float spz, float lpx, float lpy, float lpz) {
+__device__ __forceinline__ Span span_of(const ExGeom& g, float occ, float d0, float d1) {
   Span r;
-  float d0 = ex_dist<MID>(spx, spy, spz, xf, yf, zf0) + ex_dist<MID>(lpx, lpy, lpz, xf, yf, zf0);
-  float d1 = ex_dist<MID>(spx, spy, spz, xf, yf, zf1) + ex_dist<MID>(lpx, lpy, lpz, xf, yf, zf1);
   if (d1 < d0) {
     const float t = d0;
     d0 = d1;
@@ -116,10 +108,28 @@ __device__ __forceinline__ Span voxel_span(const ExGeom& g, float occ, float xf,
   return r;
 }
 
-// Flag of each point of a [B][3][N] array: 1 where every squared distance
-// from it to a point of the volume box lies in [2^-64, 2^64] (it is at least
-// 2^-20 from the box and at most 2^30 from its far corner), so that the
-// exhaustive kernels may take the short correctly rounded root for it.
+// MID: every radicand lies in [2^-64, 2^64] (both points keep a distance
+// from the box, sqrt_mid_range), so the short correctly rounded root serves.
+template <bool MID>
+__device__ __forceinline__ float ex_dist(float ax, float ay, float az, float bx, float by,
+                                         float bz) {
+  return MID ? sqrt_rn_mid(sqdist3(ax, ay, az, bx, by, bz)) : dist3(ax, ay, az, bx, by, bz);
+}
+
+template <bool MID>
+__device__ __forceinline__ Span voxel_span(const ExGeom& g, float occ, float xf, float yf,
+                                           float zf0, float zf1, float spx, float spy,
+                                           float spz, float lpx, float lpy, float lpz) {
+  const float d0 =
+      ex_dist<MID>(spx, spy, spz, xf, yf, zf0) + ex_dist<MID>(lpx, lpy, lpz, xf, yf, zf0);
+  const float d1 =
+      ex_dist<MID>(spx, spy, spz, xf, yf, zf1) + ex_dist<MID>(lpx, lpy, lpz, xf, yf, zf1);
+  return span_of(g, occ, d0, d1);
+}
+// Whether every squared distance from a point to the volume box lies in
+// [2^-64, 2^64] (it is at least 2^-20 from the box and at most 2^30 from its
+// far corner), so that the exhaustive kernels may take the short correctly
+// rounded root for it.
 __device__ __forceinline__ bool ex_point_mid(const ExGeom& g, float px, float py, float pz) {
   const float lo = box_sqdist(px, py, pz, g.sx, g.sy, g.sz, g.ex, g.ey, g.ez);
   float hi = 0.f;
@@ -129,14 +139,22 @@ __device__ __forceinline__ bool ex_point_mid(const ExGeom& g, float px, float py
   return lo >= 0x1p-40f && hi <= 0x1p60f;  // false for NaN
 }
 
-__global__ __launch_bounds__(256) void ex_point_flags_kernel(const float* __restrict__ pts,
-                                                             int N, ExGeom g,
-                                                             int* __restrict__ flags) {
+// Headers {x, y, z, flag} of each batch's scan points, then laser points; and
+// a zero per batch.
+__global__ __launch_bounds__(256) void ex_point_head_kernel(const float* __restrict__ scan,
+                                                            const float* __restrict__ laser,
+                                                            int S, int L, ExGeom g,
+                                                            float4* __restrict__ head,
+                                                            int* __restrict__ zero) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= g.B * N) return;
-  const int b = i / N, k = i - b * N;
-  const float* p = pts + (size_t)b * 3 * N;
-  flags[i] = ex_point_mid(g, p[k], p[N + k], p[2 * N + k]) ? 1 : 0;
+  const int n = S + L;
+  if (i < g.B) zero[i] = 0;
+  if (i >= g.B * n) return;
+  const int b = i / n, k = i - b * n;
+  const int N = k < S ? S : L, at = k < S ? k : k - S;
+  const float* p = (k < S ? scan : laser) + (size_t)b * 3 * N;
+  const float x = p[at], y = p[N + at], z = p[2 * N + at];
+  head[i] = make_float4(x, y, z, ex_point_mid(g, x, y, z) ? 1.f : 0.f);
 }
 
 // ---- R2 -------------------------------------------------------------------
@@ -292,93 +310,353 @@ __global__ __launch_bounds__(kR2Waves * 64) void r2_forward_kernel(
 }
 
 // ---- A5 -------------------------------------------------------------------
-// Float4s per thread of one stage copy (kStage floats, 256 lanes).
-constexpr int kA5Copy4 = kStage / 4 / 256;
+// A voxel's share of a pair is wf g[first] + wm (g between) + wl g[last].
+// Short spans (K > 0: first and last at most K bins apart) read the K - 1
+// bins after the first at fixed offsets and mask them, without a loop.  For
+// longer ones (K = 0) the rows are kept as running sums
+// C[t] = g[0] + .. + g[t - 1] in double as well: three differences of four
+// neighbouring entries give g[first], the sum between and g[last] for spans
+// of any length, more exactly than adding the bins in float.  A batch with an
+// infinite or NaN gradient, which running sums would spread, adds the bins.
 
-// Row stride of the transposed gradient: T rounded up to whole float4s.
-__host__ __device__ __forceinline__ int a5_stride(int T) { return (T + 3) & ~3; }
+// Row stride of the transposed gradient: whole float4s.
+__host__ __device__ __forceinline__ int a5_row(int T) { return (T + 3) & ~3; }
 
-// One lane per voxel.  gT holds one row of a5_stride(T) floats per
-// (scan point, laser point) pair.  A workgroup stages R rows in LDS
-// (STAGED), loading the next R into registers while it works on the current
-// ones, or reads them from global memory (rows longer than the stage).
-template <bool STAGED>
-__global__ __launch_bounds__(256) void r2_adjoint_kernel(
-    const float* __restrict__ gT,      // [B][S*L][a5_stride(T)]
-    const float* __restrict__ scan, const float* __restrict__ laser,
-    const int* __restrict__ sflag, const int* __restrict__ lflag,  // [B][S], [B][L]
-    float* __restrict__ grad,          // [B][D][H][W]
-    ExGeom g, int S, int L, int R) {
-  extern __shared__ float4 stage4[];
+// Row stride of the running sums: T + 1 rounded up to whole pairs.
+__host__ __device__ __forceinline__ int a5_stride(int T) { return (T + 2) & ~1; }
+
+struct A5Rows {
+  const float* g;     // [B][S*L][a5_row(T)] the transposed gradient
+  const double* c;    // [B][S*L][a5_stride(T)] its running sums
+  const int* bad;     // [B] whether the batch holds an infinity or a NaN
+};
+
+struct A5Layout {
+  size_t prefix, head, bad, end;
+};
+
+A5Layout a5_layout(int64_t B, int64_t T, int64_t S, int64_t L) {
+  A5Layout l;
+  l.prefix = align256((size_t)B * S * L * a5_row((int)T) * sizeof(float));
+  l.head = l.prefix + align256((size_t)B * S * L * a5_stride((int)T) * sizeof(double));
+  l.bad = l.head + align256((size_t)B * (S + L) * sizeof(float4));
+  l.end = l.bad + align256((size_t)B * sizeof(int));
+  return l;
+}
+
+// One wave per row, eight bins per lane and step.
+__global__ __launch_bounds__(256) void a5_prefix_kernel(const float* __restrict__ gT,
+                                                        double* __restrict__ c,
+                                                        int* __restrict__ bad, ExGeom g,
+                                                        int rows) {
+  const int lane = threadIdx.x & 63;
+  const size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= (size_t)g.B * rows) return;
+  const float* src = gT + r * a5_row(g.T);
+  double* dst = c + r * a5_stride(g.T);
+  double base = 0.0;
+  bool finite = true;
+  for (int t0 = 0; t0 < g.T; t0 += 512) {
+    double s[8], sum = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int t = t0 + lane * 8 + k;
+      const float v = t < g.T ? src[t] : 0.f;
+      finite = finite && fabsf(v) < INFINITY;
+      s[k] = sum;
+      sum += (double)v;
+    }
+    double up = sum;  // inclusive sum over the lanes
+    for (int m = 1; m < 64; m <<= 1) {
+      const double o = __shfl_up(up, m, 64);
+      if (lane >= m) up += o;
+    }
+    const double before = base + (up - sum);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int t = t0 + lane * 8 + k;
+      if (t < g.T) dst[t] = before + s[k];
+    }
+    base += __shfl(up, 63, 64);
+  }
+  if (lane == 0) dst[g.T] = base;
+  if (!finite) atomicOr(bad + r / rows, 1);
+}
+
+__global__ void zero_f32_kernel(float* __restrict__ out, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[(size_t)blockIdx.y * n + i] = 0.f;
+}
+
+// Gradient of one (voxel, pair) from its two path lengths, bin by bin, in the
+// reference's arithmetic (volume_cuda.cu:341-374), unit occupancy.
+__device__ __forceinline__ float a5_pair_any(const ExGeom& g, float d0, float d1,
+                                             const float* row) {
+  const Span sp = span_of(g, 1.f, d0, d1);
+  if (sp.first > sp.last) return 0.f;
+  if (sp.first == sp.last) return sp.wf * row[sp.first];
+  float m = 0.f;
+  for (int bn = sp.first + 1; bn < sp.last; ++bn) m += row[bn];
+  return sp.wf * row[sp.first] + sp.wm * m + sp.wl * row[sp.last];
+}
+
+constexpr int kA5Pairs = 8;  // (scan, laser) pairs of a unit, at most
+constexpr int kA5Slack = 8;  // floats past the staged rows that masked reads may touch
+
+// One lane per voxel.  For each tile of KT laser points a lane keeps the
+// tile's distances to the voxel's two faces in registers and walks the scan
+// points in units of SG, so a pair costs two sums where each pair's four
+// correctly rounded roots had taken a third of the kernel; the bin positions
+// are exact divisions by a constant (DivConst).  A unit's rows lie in LDS
+// (STAGED, U units per stage) or in global memory (long rows).  Units with a
+// span that is clipped at the histogram's ends, or longer than K, take a
+// second form (per wave).
+//
+// VALU issue bounds it.  64^3 voxels, 256 x 16 pairs, 512 bins (spans up to 6
+// bins): 1.37 ms a call with K = 6 and 1.50 with running sums, against 5.3 ms
+// with four roots and a loop over the bins per pair; 16 x 64 x 64 voxels,
+// 144 x 16 pairs, 1000 bins (spans up to 34 bins), render included: 0.91 ms
+// with running sums, 4.03 with the loop as the second form, 4.46 before.
+template <int K, int KT, bool STAGED, int NTH>
+__global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
+    A5Rows rows, const float4* __restrict__ head,  // [B][S + L]
+    float* __restrict__ grad,                      // [B][D][H][W]
+    ExGeom g, int S, int L, int U, int cap, DivConst dw) {
+  extern __shared__ float4 lds4[];
+  constexpr int SG = kA5Pairs / KT > 1 ? kA5Pairs / KT : 1;
   const int b = blockIdx.y;
   const int nvox = g.D * g.H * g.W;
-  const int P = a5_stride(g.T);
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  const int P = K > 0 ? a5_row(g.T) : 2 * a5_stride(g.T);  // floats of a staged row
+  const int v = blockIdx.x * NTH + threadIdx.x;
   const bool ok = v < nvox;
   const int vv = ok ? v : 0;
   const int xi = vv % g.W, yi = (vv / g.W) % g.H, zi = vv / (g.W * g.H);
   float xf, yf, zf0, zf1;
   voxel_faces(g, xi, yi, zi, &xf, &yf, &zf0, &zf1);
-  const float* sb = scan + (size_t)b * 3 * S;
-  const float* lb = laser + (size_t)b * 3 * L;
-  const int* sf = sflag + (size_t)b * S;
-  const int* lf = lflag + (size_t)b * L;
-  const int nrows = S * L;
-  const float* gb = gT + (size_t)b * nrows * P;
-  float4 buf[kA5Copy4];
-  if (STAGED) {
-    const int n4 = min(R, nrows) * P / 4;
+  const float4* hs = head + (size_t)b * (S + L);
+  const float4* hl = hs + S;
+  const float* gb = rows.g + (size_t)b * S * L * a5_row(g.T);
+  const float* cb = K > 0 ? gb : (const float*)(rows.c + (size_t)b * S * L * a5_stride(g.T));
+  const bool fast = dw.ok && (K > 0 || !rows.bad[b]);  // uniform
+  float* stage = (float*)lds4;
+  const int n_units = (S + SG - 1) / SG;
+  // distances of n points (uniform) to the voxel's faces
+  auto faces = [&](auto at, auto& d0, auto& d1, auto n) {
+    float mid = 1.f;
 #pragma unroll
-    for (int i = 0; i < kA5Copy4; ++i) {
-      const int e = i * 256 + (int)threadIdx.x;
-      buf[i] = e < n4 ? ((const float4*)gb)[e] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int j = 0; j < n; ++j) mid = fminf(mid, at(j).w);
+    if (mid != 0.f) {
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        d0[j] = ex_dist<true>(at(j).x, at(j).y, at(j).z, xf, yf, zf0);
+        d1[j] = ex_dist<true>(at(j).x, at(j).y, at(j).z, xf, yf, zf1);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < n; ++j) {
+        d0[j] = ex_dist<false>(at(j).x, at(j).y, at(j).z, xf, yf, zf0);
+        d1[j] = ex_dist<false>(at(j).x, at(j).y, at(j).z, xf, yf, zf1);
+      }
     }
-  }
+  };
+  // The weighted bins of a span; x0 <= x1 are the clipped bin positions of
+  // the faces, f = floor(x0), l = floor(x1), range their unclipped difference.
+  auto weigh = [&](const float* row, float x0, float x1, int f, int l, float range) {
+    float first, in, last;
+    if constexpr (K > 0) {
+      const float* r = row + f;
+      const int m = l - f;
+      first = r[0];
+      last = r[m];
+      in = 0.f;
+#pragma unroll
+      for (int k = 1; k < K; ++k) {
+        const float val = r[k];
+        in += k < m ? val : 0.f;
+      }
+    } else {
+      const double* c = (const double*)row;
+      const double c0 = c[f], c1 = c[f + 1], c2 = c[l], c3 = c[l + 1];
+      first = (float)(c1 - c0);
+      in = (float)(c2 - c1);
+      last = (float)(c3 - c2);
+    }
+    float frac = __builtin_amdgcn_rcpf(range);
+    frac = fmaf(fmaf(-range, frac, 1.f), frac, frac);
+    const float wf = 1.f - (x0 - (float)f), wl = x1 - (float)l;
+    const float sum = fmaf(wf, first, fmaf(wl, last, in)) * frac;
+    return f == l ? first : sum;
+  };
+
   float acc = 0.f;
-  for (int r0 = 0; r0 < nrows; r0 += R) {
-    const int nr = min(R, nrows - r0);
-    const float* src = gb + (size_t)r0 * P;
+  for (int l0 = 0; l0 < L; l0 += KT) {
+    const int nl = min(KT, L - l0);
+    float dl0[KT], dl1[KT];
+    faces([&](int j) { return hl[min(l0 + j, L - 1)]; }, dl0, dl1,
+          std::integral_constant<int, KT>{});
+    // rows of scan points s0 .. : nl consecutive rows each, L rows apart,
+    // packed in the stage
+    RowStage<NTH> next;
+    const int n4s = nl * P / 4;  // float4s per scan point
+    auto points = [&](int u) { return min(U * SG, S - u * SG); };
+    auto load = [&](int u) {
+      next.load_pieces(cb + ((size_t)u * SG * L + l0) * P, points(u) * n4s, n4s, L * P / 4);
+    };
+    auto put = [&](int u, int buf) { next.store(stage + buf * cap, points(u) * n4s); };
     if (STAGED) {
-      __syncthreads();  // the previous rows are no longer read
-      const int n4 = nr * P / 4;
-#pragma unroll
-      for (int i = 0; i < kA5Copy4; ++i) {
-        const int e = i * 256 + (int)threadIdx.x;
-        if (e < n4) stage4[e] = buf[i];
-      }
+      load(0);
+      put(0, 0);
+      if (U < n_units) load(U);
       __syncthreads();
-      if (r0 + R < nrows) {
-        const int n4n = min(R, nrows - r0 - R) * P / 4;
-        const float4* nx = (const float4*)(gb + (size_t)(r0 + R) * P);
-#pragma unroll
-        for (int i = 0; i < kA5Copy4; ++i) {
-          const int e = i * 256 + (int)threadIdx.x;
-          buf[i] = e < n4n ? nx[e] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-      }
-      src = (const float*)stage4;
     }
-    for (int k = 0; k < nr; ++k) {
-      const int r = r0 + k;
-      const int s = r / L, l = r - s * L;
-      const Span sp =
-          sf[s] & lf[l]
-              ? voxel_span<true>(g, 1.f, xf, yf, zf0, zf1, sb[s], sb[S + s], sb[2 * S + s],
-                                 lb[l], lb[L + l], lb[2 * L + l])
-              : voxel_span<false>(g, 1.f, xf, yf, zf0, zf1, sb[s], sb[S + s], sb[2 * S + s],
-                                  lb[l], lb[L + l], lb[2 * L + l]);
-      if (sp.first > sp.last) continue;
-      const float* row = src + k * P;
-      if (sp.first == sp.last) {
-        acc += sp.wf * row[sp.first];
-      } else {
-        acc += sp.wf * row[sp.first];
-        for (int bn = sp.first + 1; bn < sp.last; ++bn) acc += sp.wm * row[bn];
-        acc += sp.wl * row[sp.last];
+    int cur = 0;
+    for (int u0 = 0; u0 < n_units; u0 += U) {
+      const int ue = min(u0 + U, n_units);
+      if (STAGED && ue < n_units) {
+        put(ue, cur ^ 1);
+        if (ue + U < n_units) load(ue + U);
+      }
+      for (int u = u0; u < ue; ++u) {
+        const int s0 = u * SG, ns = min(SG, S - s0);
+        // row of pair (s0 + i, l0 + j)
+        const float* base = STAGED ? stage + cur * cap + (u - u0) * SG * nl * P
+                                   : cb + ((size_t)s0 * L + l0) * P;
+        const int si = (STAGED ? nl : L) * P;
+        float ds0[SG], ds1[SG];
+        faces([&](int i) { return hs[min(s0 + i, S - 1)]; }, ds0, ds1,
+              std::integral_constant<int, SG>{});
+        if (fast) {
+          float x0[SG][KT], x1[SG][KT];
+          int f[SG][KT], l[SG][KT];
+          bool clipped = ns < SG || nl < KT, odd = false;
+#pragma unroll
+          for (int i = 0; i < SG; ++i)
+#pragma unroll
+            for (int j = 0; j < KT; ++j) {
+              const float a = ds0[i] + dl0[j], c = ds1[i] + dl1[j];
+              x0[i][j] = div_const(fminf(a, c) - g.off, dw);                  // :341-347
+              x1[i][j] = div_const(fmaxf(a, c) - g.off, dw);
+              f[i][j] = floor_to_int(x0[i][j]);                               // :349-350
+              l[i][j] = floor_to_int(x1[i][j]);
+              clipped |= f[i][j] < 0 | l[i][j] >= g.T;
+              if (K > 0) clipped |= l[i][j] - f[i][j] > K;
+              odd |= !(x1[i][j] - x0[i][j] < 0x1p60f);  // NaN or infinite
+            }
+          if (!__any(clipped | odd)) {
+#pragma unroll
+            for (int i = 0; i < SG; ++i)
+#pragma unroll
+              for (int j = 0; j < KT; ++j)
+                acc += weigh(base + i * si + j * P, x0[i][j], x1[i][j], f[i][j], l[i][j],
+                             x1[i][j] - x0[i][j]);
+            continue;
+          }
+          if (K == 0 && !__any(odd)) {
+#pragma unroll
+            for (int i = 0; i < SG; ++i)
+#pragma unroll
+              for (int j = 0; j < KT; ++j)
+                if (i < ns && j < nl) {
+                  const bool empty = l[i][j] < 0 || f[i][j] >= g.T;           // :351-364
+                  const float range = x1[i][j] - x0[i][j];
+                  const float e1 = l[i][j] >= g.T ? (float)(g.T - 1) : x1[i][j];
+                  const float sum = weigh(base + i * si + j * P, fmaxf(x0[i][j], 0.f), e1,
+                                          min(max(f[i][j], 0), g.T - 1),
+                                          min(max(l[i][j], 0), g.T - 1), range);
+                  acc += empty ? 0.f : sum;
+                }
+            continue;
+          }
+        }
+        const float* any = K > 0 ? base : gb + ((size_t)s0 * L + l0) * a5_row(g.T);
+        const int ai = K > 0 ? si : L * a5_row(g.T);
+#pragma unroll
+        for (int i = 0; i < SG; ++i)
+#pragma unroll
+          for (int j = 0; j < KT; ++j)
+            if (i < ns && j < nl)
+              acc += a5_pair_any(g, ds0[i] + dl0[j], ds1[i] + dl1[j],
+                                 any + (size_t)i * ai + j * a5_row(g.T));
+      }
+      if (STAGED) {
+        __syncthreads();
+        cur ^= 1;
       }
     }
   }
   if (ok) grad[(size_t)b * nvox + v] = acc;
+}
+
+template <int K, int KT>
+int a5_launch_tile(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g,
+                   int64_t S, int64_t L, const StagePlan& sp, int64_t P, hipStream_t st) {
+  constexpr int SG = kA5Pairs / KT > 1 ? kA5Pairs / KT : 1;
+  const int64_t n = (int64_t)SG * std::min<int64_t>(KT, L);  // rows of a unit
+  // masked reads may touch K floats past the last row
+  const int64_t U = std::min<int64_t>((S + SG - 1) / SG, (sp.cap - kA5Slack) / (n * P));
+  auto kernel = sp.threads == 1024 ? r2_adjoint_kernel<K, KT, true, 1024>
+                                   : r2_adjoint_kernel<K, KT, true, 256>;
+  const int rc = allow_stage(kernel);
+  if (rc) return rc;
+  const unsigned blocks = (unsigned)(((size_t)g.D * g.H * g.W + sp.threads - 1) / sp.threads);
+  hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)g.B), dim3(sp.threads),
+                     2 * (size_t)sp.cap * sizeof(float), st, rows, head, grad, g, (int)S, (int)L,
+                     (int)U, sp.cap, make_div_const(g.w));
+  return check_launch("r2_adjoint_kernel");
+}
+
+template <int K>
+int a5_launch_span(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g,
+                   int64_t S, int64_t L, hipStream_t st) {
+  const int64_t nvox = (int64_t)g.D * g.H * g.W;
+  const int64_t P = K > 0 ? a5_row(g.T) : 2 * a5_stride(g.T);
+  if (K == 0) {
+    const int64_t waves = g.B * S * L;
+    hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st,
+                       rows.g, (double*)rows.c, (int*)rows.bad, g, (int)(S * L));
+    const int rc = check_launch("a5_prefix_kernel");
+    if (rc) return rc;
+  }
+  StagePlan sp = stage_plan(g.B, nvox);
+  // fewer, larger buffers rather than rows from global memory
+  if (kA5Pairs * P > sp.cap - kA5Slack) sp.cap = kStageMax;
+  const int64_t fit = (sp.cap - kA5Slack) / P;
+  // The tile with the least work: every slot of a tile costs a pair (about
+  // 50 instructions), every scan point of a tile two roots (about 35).
+  static const int sizes[] = {1, 2, 3, 4, 6, 8};
+  int kt = 0;
+  int64_t least = 0;
+  for (int k : sizes) {
+    if ((int64_t)(kA5Pairs / k) * std::min<int64_t>(k, L) > fit) continue;
+    const int64_t cost = (L + k - 1) / k * (50 * k + 35);
+    if (kt == 0 || cost <= least) {
+      kt = k;
+      least = cost;
+    }
+  }
+  if (kt == 1) return a5_launch_tile<K, 1>(rows, head, grad, g, S, L, sp, P, st);
+  if (kt == 2) return a5_launch_tile<K, 2>(rows, head, grad, g, S, L, sp, P, st);
+  if (kt == 3) return a5_launch_tile<K, 3>(rows, head, grad, g, S, L, sp, P, st);
+  if (kt == 4) return a5_launch_tile<K, 4>(rows, head, grad, g, S, L, sp, P, st);
+  if (kt == 6) return a5_launch_tile<K, 6>(rows, head, grad, g, S, L, sp, P, st);
+  if (kt == 8) return a5_launch_tile<K, 8>(rows, head, grad, g, S, L, sp, P, st);
+  if (K > 0) return a5_launch_span<0>(rows, head, grad, g, S, L, st);
+  // rows too long for the stage: running sums in global memory
+  hipLaunchKernelGGL((r2_adjoint_kernel<0, 8, false, 256>),
+                     dim3((unsigned)((nvox + 255) / 256), (unsigned)g.B), dim3(256), 0, st, rows,
+                     head, grad, g, (int)S, (int)L, (int)S, 0, make_div_const(g.w));
+  return check_launch("r2_adjoint_kernel");
+}
+
+// A voxel's faces are at most 2 dz / w bins apart (each leg of a path changes
+// by at most the voxel's height), so their bins at most floor(2 dz / w) + 1.
+// A wrong guess costs the second form, no error.
+int a5_launch(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g, int64_t S,
+              int64_t L, hipStream_t st) {
+  const double bins = 2.0 * fabs((double)g.ez - g.sz) / g.D / (double)g.w;
+  if (bins < 1.99) return a5_launch_span<2>(rows, head, grad, g, S, L, st);
+  if (bins < 5.95) return a5_launch_span<6>(rows, head, grad, g, S, L, st);
+  return a5_launch_span<0>(rows, head, grad, g, S, L, st);
 }
 
 ExGeom ex_geom(int64_t B, int64_t D, int64_t H, int64_t W, int64_t T, const float* vs,
@@ -399,8 +677,6 @@ ExGeom ex_geom(int64_t B, int64_t D, int64_t H, int64_t W, int64_t T, const floa
   g.off = off;
   return g;
 }
-
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 int check_sizes(int64_t B, int64_t D, int64_t H, int64_t W, int64_t T, int64_t S, int64_t L) {
   for (int64_t d : {B, D, H, W, T, S, L})
@@ -505,9 +781,7 @@ extern "C" int totri_volume_render_exhaustive_forward(
 extern "C" size_t totri_volume_render_exhaustive_grad_volume_workspace(int64_t B, int64_t T,
                                                                        int64_t S, int64_t L) {
   if (B <= 0 || T < 0 || S <= 0 || L <= 0) return 0;
-  // the transposed gradient rows, then the point flags of the scan and laser points
-  return align256((size_t)B * S * L * a5_stride((int)T) * sizeof(float)) +
-         align256((size_t)B * (S + L) * sizeof(int));
+  return a5_layout(B, T, S, L).end;
 }
 
 extern "C" int totri_volume_render_exhaustive_grad_volume(
@@ -527,10 +801,8 @@ extern "C" int totri_volume_render_exhaustive_grad_volume(
   const ExGeom g = ex_geom(B, D, H, W, T, volume_start, volume_end, bin_width, bin_offset);
   const dim3 grid((unsigned)((nvox + 255) / 256), (unsigned)B);
   if (T == 0 || S == 0 || L == 0) {  // no bins or no pairs: a zero gradient
-    hipLaunchKernelGGL(r2_adjoint_kernel<false>, grid, dim3(256), 0, st, (const float*)nullptr,
-                       scan_points, laser_points, (const int*)nullptr, (const int*)nullptr,
-                       volume_grad, g, 0, 1, 1);
-    return check_launch("r2_adjoint_kernel");
+    hipLaunchKernelGGL(zero_f32_kernel, grid, dim3(256), 0, st, volume_grad, (int)nvox);
+    return check_launch("zero_f32_kernel");
   }
   TOTRI_CHECK_ARG(transient_grad && scan_points && laser_points, "null input");
   const size_t need = totri_volume_render_exhaustive_grad_volume_workspace(B, T, S, L);
@@ -539,32 +811,22 @@ extern "C" int totri_volume_render_exhaustive_grad_volume(
                 workspace_bytes);
   TOTRI_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace & 15) == 0,
                   "workspace must be a non-null, 16-byte aligned device pointer");
-  float* gT = (float*)workspace;
-  const int P = a5_stride((int)T);
-  int* sflag = (int*)((char*)workspace + align256((size_t)B * S * L * P * sizeof(float)));
-  int* lflag = sflag + B * S;
-  // [B][T][S*L] -> [B][S*L][P]
-  rc = transpose_strided(transient_grad, gT, (int)B, (int)T, (int)(S * L), P, 0, st);
+  const A5Layout lay = a5_layout(B, T, S, L);
+  char* ws = (char*)workspace;
+  A5Rows rows;
+  rows.g = (float*)ws;
+  rows.c = (double*)(ws + lay.prefix);
+  rows.bad = (int*)(ws + lay.bad);
+  float4* head = (float4*)(ws + lay.head);
+  // [B][T][S*L] -> [B][S*L][a5_row(T)]
+  rc = transpose_strided(transient_grad, (float*)ws, (int)B, (int)T, (int)(S * L),
+                         a5_row((int)T), 0, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(ex_point_flags_kernel, dim3((unsigned)((B * S + 255) / 256)), dim3(256), 0,
-                     st, scan_points, (int)S, g, sflag);
-  rc = check_launch("ex_point_flags_kernel");
+  hipLaunchKernelGGL(ex_point_head_kernel, dim3((unsigned)((B * (S + L) + 255) / 256)), dim3(256),
+                     0, st, scan_points, laser_points, (int)S, (int)L, g, head, (int*)rows.bad);
+  rc = check_launch("ex_point_head_kernel");
   if (rc) return rc;
-  hipLaunchKernelGGL(ex_point_flags_kernel, dim3((unsigned)((B * L + 255) / 256)), dim3(256), 0,
-                     st, laser_points, (int)L, g, lflag);
-  rc = check_launch("ex_point_flags_kernel");
-  if (rc) return rc;
-  // rows per LDS stage; rows longer than the stage are read from global memory
-  const int R = (int)std::min<int64_t>(S * L, kStage / P);
-  if (R > 0) {
-    hipLaunchKernelGGL(r2_adjoint_kernel<true>, grid, dim3(256), (size_t)R * P * sizeof(float),
-                       st, gT, scan_points, laser_points, sflag, lflag, volume_grad, g, (int)S,
-                       (int)L, R);
-  } else {
-    hipLaunchKernelGGL(r2_adjoint_kernel<false>, grid, dim3(256), 0, st, gT, scan_points,
-                       laser_points, sflag, lflag, volume_grad, g, (int)S, (int)L, (int)(S * L));
-  }
-  return check_launch("r2_adjoint_kernel");
+  return a5_launch(rows, head, volume_grad, g, S, L, st);
 }
 
 namespace totri_hip {
