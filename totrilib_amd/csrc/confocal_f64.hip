@@ -13,10 +13,9 @@
 //     arithmetic and the sum are double (backprojection_cuda.cu:167-190).
 // pow(x, 2) and pow(x, 4) are written as products.
 //
-// These are plain one-thread-per-output kernels in the reference's loop
-// order (columns, scan points and bins in order), so each sum is the
-// reference's sequence of double operations; FP64 is the accuracy form, the
-// FP32 kernels are the fast path.
+// Each output's sum is the reference's sequence of double operations (columns,
+// scan points and bins in order); FP64 is the accuracy form, the FP32 kernels
+// are the fast path.
 #include <math.h>
 
 #include "common.h"
@@ -28,6 +27,27 @@ __device__ __forceinline__ double cell_centre_d(int i, float o, float sz, int n)
   double a = ((double)i + 0.5) * (double)sz;  // volume_cuda.cu:35
   a = a / (double)n;
   return (double)o + a;
+}
+
+// Correctly rounded square root without the library form's scaling and special
+// values: one Newton step on the hardware's reciprocal root, then two residual
+// steps, of which the last decides the rounding (Markstein).  For positive x in
+// [2^-500, 2^500], which every active sample's d2 is: its terms are a square
+// of a float radius and a difference from it, so a positive one is at least
+// 2^-460 and at most 2^256.  Other x give NaN.
+__device__ __forceinline__ double sqrt_mid_f64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// x is positive and finite.
+__device__ __forceinline__ bool positive_f64(double x) {
+  return __builtin_amdgcn_class(x, 0x180);
 }
 
 struct SampleD {
@@ -70,6 +90,7 @@ struct GeomD {
 };
 
 // R1: one thread per (scan point, bin); columns in order (volume_cuda.cu:33-63).
+// The form for transients of few bins: r1_tiles_f64_kernel takes the others.
 __global__ __launch_bounds__(256) void r1_f64_kernel(const double* __restrict__ vol,
                                                      const double* __restrict__ mp,
                                                      double* __restrict__ tr, GeomD g) {
@@ -95,11 +116,136 @@ __global__ __launch_bounds__(256) void r1_f64_kernel(const double* __restrict__ 
   tr[e] = value;
 }
 
+// The same sums, 64 bins of one scan point to a workgroup: three producer waves
+// take eight columns each, leave the samples' terms in LDS, and a fourth wave,
+// a lane per bin, adds the previous round's in column order (a lane that walks
+// its own columns waits for every sample's chain: 32^3 voxels, 256 points, 256
+// bins are one wave per SIMD).  An inactive sample's term is +0, which leaves
+// a sum that began at +0 unchanged.  Where bins and rows rise together (w > 0,
+// off >= 0, size_z > 0) the rows of a column's first and last bin tell whether
+// any bin between is active; columns with none leave zeros.  The bin's square
+// is the lane's own, so depth / t2 is a division by a constant (see DivConst).
+// Bound by the double-precision issue rate of the square roots and quotients.
+// 32^3 voxels, 256 points, 256 bins: 287 -> 105 us (four waves, so that
+// a workgroup loads the SIMDs evenly; with five, 178).
+constexpr int kProdR1F64 = 3, kColsR1F64 = 8;
+// Of fewer bins a tile has too many idle lanes: 32^2 x 16 voxels take 420 us
+// with 4,096 points of 8 bins (r1_f64_kernel: 276), and with 16 bins the gain
+// (275 -> 128 us, 1,024 points) is gone once r1_f64_kernel fills the chip.
+constexpr int kMinBinsF64 = 32;
+
+__global__ __launch_bounds__(64 * (kProdR1F64 + 1)) void r1_tiles_f64_kernel(
+    const double* __restrict__ vol, const double* __restrict__ mp, double* __restrict__ tr,
+    GeomD g, int n_tiles, int rising) {
+  constexpr int P = kProdR1F64, U = kColsR1F64, H = 4;
+  __shared__ double terms[2][P][U][64];
+  __shared__ double2 lateral[P][64];  // squared x and y offsets of a wave's next columns
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const double o = (double)g.oz;
+  const double s = (double)g.Z / (double)g.sz;
+  const int n_cols = g.X * g.Y;
+  const int rounds = (n_cols + P * U - 1) / (P * U);
+  const long long n_blocks = (long long)g.N * n_tiles;
+  for (long long blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
+    // Neighbouring workgroups (on different XCDs) take the same bins: the near
+    // bins are active in fewer columns.
+    const int i = (int)(blk % g.N);
+    const int tile = (int)(blk / g.N) * 64;
+    const double wx = mp[i], wy = mp[g.N + i], wz = mp[2 * g.N + i];
+    const int ti = min(tile + lane, g.T - 1);
+    auto bin_square = [&](int t) {
+      const double tc = (double)bin_distance(t, g.w, g.off);
+      return tc * tc;
+    };
+    auto row_of = [&](double d2, double* depth, double* zh) {
+      *depth = sqrt_mid_f64(d2);
+      const double z = wz + *depth;
+      *zh = (z - o) * s;
+      *zh = *zh - 0.5;
+      return (int)floorf((float)*zh);  // floorf narrows to float
+    };
+    const double t2 = bin_square(ti);
+    const double t2a = bin_square(tile), t2b = bin_square(min(tile + 63, g.T - 1));
+    const double hi = 1.0 / t2;
+    const double lo = __builtin_fma(-hi, t2, 1.0) * hi;
+    double value = 0.0;
+    unsigned long long some = 0;  // bit: lateral[wave][bit]'s column has an active bin
+    for (int r = 0; r <= rounds; ++r) {
+      if (wave < P && r < rounds) {
+        if (r % 8 == 0) {
+          const int c = (r + (lane >> 3)) * (P * U) + wave * U + (lane & 7);
+          const int cc = min(c, n_cols - 1);
+          const int xi = cc / g.Y, yi = cc - xi * g.Y;
+          const double dx = wx - cell_centre_d(xi, g.ox, g.sx, g.X);
+          const double dy = wy - cell_centre_d(yi, g.oy, g.sy, g.Y);
+          const double dx2 = dx * dx, dy2 = dy * dy;
+          lateral[wave][lane] = make_double2(dx2, dy2);
+          bool a = c < n_cols && g.Z > 1;
+          if (rising) {
+            double d2a = t2a - dx2, d2b = t2b - dx2, depth, zh;
+            d2a = d2a - dy2;
+            d2b = d2b - dy2;
+            const bool past = positive_f64(d2a) && row_of(d2a, &depth, &zh) >= g.Z - 1;
+            const bool before = !(d2b > 0.0) ||
+                                (positive_f64(d2b) && row_of(d2b, &depth, &zh) < 0);
+            a = a && !past && !before;
+          }
+          some = __ballot(a);
+        }
+        const int k = (r & 7) * U;
+        const int c0 = r * (P * U) + wave * U;
+#pragma unroll
+        for (int h = 0; h < U; h += H) {
+          double(*out)[64] = &terms[r & 1][wave][h];
+          if (((some >> (k + h)) & ((1u << H) - 1u)) == 0) {
+#pragma unroll
+            for (int u = 0; u < H; ++u) out[u][lane] = 0.0;
+            continue;
+          }
+          double depth[H], alpha[H], v0[H], v1[H];
+          bool act[H];
+#pragma unroll
+          for (int u = 0; u < H; ++u) {
+            const double2 l = lateral[wave][k + h + u];
+            double d2 = t2 - l.x;
+            d2 = d2 - l.y;
+            double zh;
+            const int zu = row_of(d2, &depth[u], &zh);
+            // no short circuits: a branch per sample would serialise the chains
+            act[u] = positive_f64(d2) & (zu >= 0) & (zu < g.Z - 1) & (c0 + h + u < n_cols);
+            const unsigned zi = act[u] ? zu : 0;
+            alpha[u] = zh - (double)zu;
+            const double* p = vol + (size_t)min(c0 + h + u, n_cols - 1) * g.Z;
+            v0[u] = p[zi];
+            v1[u] = p[zi + 1];
+          }
+#pragma unroll
+          for (int u = 0; u < H; ++u) {
+            double q = __builtin_fma(depth[u], hi, depth[u] * lo);
+            q = __builtin_fma(__builtin_fma(-q, t2, depth[u]), hi, q);
+            q = q * q;
+            const double f2 = q * q;
+            const double f1 = (1.0 - alpha[u]) * v0[u] + alpha[u] * v1[u];
+            out[u][lane] = act[u] ? f1 * f2 : 0.0;
+          }
+        }
+      } else if (wave == P && r > 0) {
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+          for (int u = 0; u < U; ++u) value = value + terms[(r - 1) & 1][p][u][lane];
+      }
+      __syncthreads();
+    }
+    if (wave == P && tile + lane < g.T) tr[(size_t)i * g.T + tile + lane] = value;
+  }
+}
+
 // A1 as the exact transpose of r1_f64_kernel: one thread per voxel; over scan
 // points and bins in order, a sample flooring to z adds (1 - alpha) f2 G and
-// one flooring to z - 1 adds alpha f2 G.  Only bins whose radius may put
-// z_hat within two voxels of [z - 1, z + 1) are visited (the decision itself
-// is taken exactly for each of them).
+// one flooring to z - 1 adds alpha f2 G.  The general form: a1_rows_f64_kernel
+// takes the calls with w > 0, off >= 0 and size_z > 0.
 __global__ __launch_bounds__(256) void a1_f64_kernel(double* __restrict__ vol,
                                                      const double* __restrict__ mp,
                                                      const double* __restrict__ G, GeomD g) {
@@ -143,6 +289,162 @@ __global__ __launch_bounds__(256) void a1_f64_kernel(double* __restrict__ vol,
     }
   }
   vol[e] = value;
+}
+
+// The same sums where bins and rows rise together (w > 0, off >= 0, size_z >
+// 0).  A voxel's samples are then the bins of two neighbouring rows, so a
+// workgroup takes one column's tile of 64 voxels and computes each sample of
+// it once (a1_f64_kernel computes a sample for about seven voxels): three
+// producer waves take three units -- a unit is a scan point and up to kBinsF64
+// of its bins -- and leave in LDS each sample's two contributions and the bin
+// at which each row starts; the fourth wave, a lane per voxel, adds the
+// previous round's contributions in scan point and bin order.  Inactive
+// samples hold +0, which leaves a sum that began at +0 unchanged.  Bound by
+// the double-precision issue rate of the samples' square root and division.
+// 32^3 voxels, 256 points, 256 bins: 1575 -> 197 us (with four
+// producers, five waves: 277).
+constexpr int kBinsF64 = 256, kProdF64 = 3, kTileF64 = 64;
+// Of fewer rows a tile has too few voxels for a unit's samples: 256 x 256
+// columns, 64 points, 128 bins take 2.42 ms with 8 rows (a1_f64_kernel: 3.09)
+// and 3.59 ms with 4 (2.69).
+constexpr int kMinRowsF64 = 8;
+struct UnitF64 {
+  double2 c[kBinsF64];        // alpha f2 G (row zi + 1), (1 - alpha) f2 G (row zi)
+  double2 zero;               // c[kBinsF64].x = +0
+  int start[kTileF64 + 2];    // first bin of the unit at or past row z0 - 1 + i
+};
+
+// The value lane `l` (uniform) holds.
+__device__ __forceinline__ double lane_f64(double v, int l) {
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
+  return __longlong_as_double(((unsigned long long)hi << 32) | lo);
+}
+
+__global__ __launch_bounds__(64 * (kProdF64 + 1)) void a1_rows_f64_kernel(
+    double* __restrict__ vol, const double* __restrict__ mp, const double* __restrict__ G,
+    GeomD g, int n_tiles, int chunks) {
+  __shared__ UnitF64 buf[2][kProdF64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = blockIdx.x / n_tiles;
+  const int z0 = (blockIdx.x - col * n_tiles) * kTileF64;
+  const int xi = col / g.Y, yi = col - (col / g.Y) * g.Y;
+  const double x = cell_centre_d(xi, g.ox, g.sx, g.X);
+  const double y = cell_centre_d(yi, g.oy, g.sy, g.Y);
+  const double o = (double)g.oz;
+  const double s = (double)g.Z / (double)g.sz;
+  const int z_last = min(z0 + kTileF64, g.Z) - 1;
+  const unsigned units = (unsigned)g.N * (unsigned)chunks;  // < 2^32: N T < 2^31
+  const unsigned rounds = units / kProdF64 + (units % kProdF64 != 0);
+  if (threadIdx.x < 2 * kProdF64)
+    buf[threadIdx.x / kProdF64][threadIdx.x % kProdF64].zero = make_double2(0.0, 0.0);
+  __syncthreads();
+  double value = 0.0;
+  // Producers: lane r % 64 holds its wave's unit of round r: squared lateral
+  // offsets, the wall's z, the scan point and the bins [first, last].
+  double dx2l = 0.0, dy2l = 0.0, wzl = 0.0;
+  int il = 0, t0l = 0, t1l = -1;
+  for (unsigned r = 0; r <= rounds; ++r) {
+    if (wave < kProdF64) {
+      if ((r & 63u) == 0) {
+        const unsigned u = min((r + lane) * kProdF64 + wave, units - 1u);
+        il = (int)(u / (unsigned)max(chunks, 1));
+        if (r < rounds) {
+          const double wx = mp[il], wy = mp[g.N + il];
+          wzl = mp[2 * g.N + il];
+          const double dx = wx - x, dy = wy - y;
+          dx2l = dx * dx;
+          dy2l = dy * dy;
+          // The tile's bins: rows max(z0 - 1, 0) .. min(z_last, Z - 2), a
+          // quarter row wider (2^20 rows round to 1/16 when narrowed).
+          t0l = 0;
+          t1l = -1;
+          const double row_lo = (double)max(z0 - 1, 0), row_hi = (double)min(z_last + 1, g.Z - 1);
+          const double dlo = fmax((row_lo + 0.25) / s + o - wzl, 0.0);
+          const double dhi = (row_hi + 0.75) / s + o - wzl;
+          if (dhi > 0.0) {
+            const double rho2 = dx2l + dy2l;
+            const double rlo = sqrt(rho2 + dlo * dlo) * (1.0 - 1e-6);
+            const double rhi = sqrt(rho2 + dhi * dhi) * (1.0 + 1e-6);
+            const double ta = floor((rlo - (double)g.off) / (double)g.w) - 2.0;
+            const double tb = ceil((rhi - (double)g.off) / (double)g.w) + 2.0;
+            t0l = ta < 0.0 ? 0 : (ta > (double)g.T ? g.T : (int)ta);
+            t1l = tb > (double)(g.T - 1) ? g.T - 1 : (tb < -1.0 ? -1 : (int)tb);
+          }
+          t0l += (int)(u - (unsigned)il * (unsigned)chunks) * kBinsF64;
+        }
+      }
+      const int rl = (int)(r & 63u);
+      if (r * kProdF64 + wave < units) {
+        UnitF64& b = buf[r & 1][wave];
+        const double dx2 = lane_f64(dx2l, rl), dy2 = lane_f64(dy2l, rl);
+        const double wz = lane_f64(wzl, rl);
+        const int t0 = __builtin_amdgcn_readlane(t0l, rl);
+        const int t1 = __builtin_amdgcn_readlane(t1l, rl);
+        const double* gi = G + (size_t)__builtin_amdgcn_readlane(il, rl) * g.T;
+        const int cnt = min(t1 + 1 - t0, kBinsF64);
+        if (cnt <= 0) {
+          for (int k = lane; k < kTileF64 + 2; k += 64) b.start[k] = 0;
+        } else {
+          int prev = 0;  // row of the bin before this lane's
+          for (int j = 0; j < cnt; j += 64) {
+            const int k = j + lane;
+            const int t = min(t0 + k, t1);
+            const double gt = gi[t];
+            const double tc = (double)bin_distance(t, g.w, g.off);
+            const double t2 = tc * tc;
+            double d2 = t2 - dx2;
+            d2 = d2 - dy2;
+            const double depth = sqrt_mid_f64(d2);
+            const double z = wz + depth;
+            double zh = (z - o) * s;
+            zh = zh - 0.5;
+            const int zi = (int)floorf((float)zh);  // floorf narrows to float
+            const bool below = !positive_f64(d2) | (zi < 0);
+            const bool act = !below & (zi < g.Z - 1);
+            const double alpha = zh - (double)zi;
+            const double q = -depth / t2;
+            const double q2 = q * q;
+            const double fg = (q2 * q2) * gt;
+            b.c[k] = make_double2(act ? alpha * fg : 0.0, act ? (1.0 - alpha) * fg : 0.0);
+            const int row = below ? -1 : min(max(min(zi, g.Z) - (z0 - 1), -1), kTileF64 + 1);
+            if (j == 0) {
+              prev = __builtin_amdgcn_readfirstlane(row);
+              for (int m = lane; m < kTileF64 + 2; m += 64) b.start[m] = m <= prev ? 0 : cnt;
+            }
+            const int up = __shfl_up(row, 1);
+            const int before = lane == 0 ? prev : up;
+            if (k < cnt)
+              for (int m = before + 1; m <= row; ++m) b.start[m] = k;
+            prev = __builtin_amdgcn_readlane(row, 63);
+          }
+        }
+      }
+    } else if (r > 0) {
+      const unsigned u0 = (r - 1) * kProdF64;
+      const int nu = (int)min(units - u0, (unsigned)kProdF64);
+      for (int p = 0; p < nu; ++p) {
+        const UnitF64& b = buf[(r - 1) & 1][p];
+        const double* c = (const double*)b.c;
+        // bins [ka, kb) are on row z - 1, [kb, kc) on row z: in halves of c
+        const int ka = 2 * b.start[lane], kb = 2 * b.start[lane + 1], kc = 2 * b.start[lane + 2];
+        for (int k = ka; __ballot(k < kc) != 0; k += 8) {
+          double v[4];
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            const int e = k + 2 * m + (k + 2 * m >= kb ? 1 : 0);
+            v[m] = c[k + 2 * m < kc ? e : 2 * kBinsF64];
+          }
+#pragma unroll
+          for (int m = 0; m < 4; ++m) value += v[m];
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (wave == kProdF64 && z0 + lane < g.Z) vol[(size_t)col * g.Z + z0 + lane] = value;
 }
 
 // The reference's window-form A1 in double (volume_cuda.cu:95-160): one
@@ -267,6 +569,18 @@ GeomD geom_d(int64_t X, int64_t Y, int64_t Z, int64_t N, int64_t T, const float*
   return g;
 }
 
+// Units per scan point that cover every tile's bins: a tile's radii span at
+// most its depth (64 voxels and 3 on either side), and the window's margins
+// are relative to radii that a bin can have.
+int unit_chunks_f64(const GeomD& g) {
+  const double far = (double)g.T * g.w + g.off;
+  const double depth = ((double)(g.Z < kTileF64 ? g.Z : kTileF64) + 6.0) * g.sz / g.Z;
+  const double span = depth * (1.0 + 1e-6) + 3e-6 * far +
+                      1e-11 * (far + fabs((double)g.oz) + (double)g.sz);
+  const double bins = fmin(span / g.w + 10.0, (double)g.T);
+  return (int)((bins + kBinsF64 - 1.0) / kBinsF64);
+}
+
 }  // namespace
 }  // namespace totri_hip
 
@@ -282,6 +596,15 @@ extern "C" int totri_volume_confocal_forward_f64(
   TOTRI_CHECK_ARG(transient && measurement_points && (X * Y * Z == 0 || volume),
                   "null pointer");
   const GeomD g = geom_d(X, Y, Z, N, T, volume_origin, volume_size, bin_width, bin_offset);
+  if (T >= kMinBinsF64) {
+    const long long n_tiles = (T + 63) / 64;
+    const long long blocks = N * n_tiles;
+    const int rising = bin_width > 0.f && bin_offset >= 0.f && volume_size[2] > 0.f;
+    hipLaunchKernelGGL(r1_tiles_f64_kernel, dim3((unsigned)(blocks < (1 << 22) ? blocks : 1 << 22)),
+                       dim3(64 * (kProdR1F64 + 1)), 0, (hipStream_t)stream, volume,
+                       measurement_points, transient, g, (int)n_tiles, rising);
+    return check_launch("r1_tiles_f64_kernel");
+  }
   hipLaunchKernelGGL(r1_f64_kernel, dim3(blocks_for(N * T)), dim3(256), 0,
                      (hipStream_t)stream, volume, measurement_points, transient, g);
   return check_launch("r1_f64_kernel");
@@ -302,6 +625,15 @@ extern "C" int totri_volume_confocal_grad_volume_f64(
     hipLaunchKernelGGL(a1_window_f64_kernel, dim3(blocks_for(nv)), dim3(256), 0,
                        (hipStream_t)stream, volume, measurement_points, transient, g);
     return check_launch("a1_window_f64_kernel");
+  }
+  const long long n_tiles = (Z + kTileF64 - 1) / kTileF64;
+  const long long blocks = X * Y * n_tiles;
+  if (bin_width > 0.f && bin_offset >= 0.f && volume_size[2] > 0.f && Z >= kMinRowsF64 &&
+      Z <= (1 << 20) && blocks < (1ll << 23)) {
+    hipLaunchKernelGGL(a1_rows_f64_kernel, dim3((unsigned)blocks), dim3(64 * (kProdF64 + 1)), 0,
+                       (hipStream_t)stream, volume, measurement_points, transient, g,
+                       (int)n_tiles, N * T == 0 ? 0 : unit_chunks_f64(g));
+    return check_launch("a1_rows_f64_kernel");
   }
   hipLaunchKernelGGL(a1_f64_kernel, dim3(blocks_for(nv)), dim3(256), 0, (hipStream_t)stream,
                      volume, measurement_points, transient, g);
