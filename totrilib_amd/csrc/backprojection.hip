@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "compact.h"
@@ -543,8 +544,25 @@ __device__ __forceinline__ EllPair ell_pair(const float* sb, const float* lb,
   return e;
 }
 
+// The value lane `l` (uniform) holds.
+__device__ __forceinline__ float readlane_f(float v, int l) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l));
+}
+
 // One wave: columns tile*64 .. tile*64+63 of batch b, list chunk `chunk` of
 // n_chunks.  dst is the chunk's partial volume [B][D][H][W] (written).
+//
+// Bound by the VALU issue of the per-column formula and the latency of its
+// chain (the column accumulators in LDS leave two waves per SIMD at 64 rows).
+// What depends on the bin alone -- its index split, value, radii, one root, one
+// quotient and its pair's geometry -- is computed for 64 list entries at once, a
+// lane each, and handed out by readlane; entries whose ellipsoid misses the
+// wave's columns are left out there; two entries of one scan/laser pair then
+// go together, so their chains overlap.  Roots and quotients of values in the
+// middle of the range take the short correctly rounded forms; other values
+// send the entry through the full ones (same results).  16^2 scan and 4^2
+// laser points, 512 bins, 5 % positive, 64^3 voxels: 2.04 -> 0.87 ms (1.27
+// without leaving entries out).
 template <bool IN_LDS>
 __global__ __launch_bounds__(64) void arellano_kernel(
     const float* __restrict__ trT,     // [B][S][L][T]
@@ -583,51 +601,45 @@ __global__ __launch_bounds__(64) void arellano_kernel(
   const float* lb = laser + (size_t)b * 3 * L;
   const float* sob = sorig + (size_t)b * 3 * So;
   const float* lob = lorig + (size_t)b * 3 * Lo;
-  int cur_pair = -1;
-  EllPair e;
-  float rsx = 0.f, rsy = 0.f, rsz = 0.f, rex = 0.f, rey = 0.f, rez = 0.f, dps = 0.f, dpe = 0.f;
-  for (int k = k0; k < k1; ++k) {
-    const int idx = uniform_i32(lb_list[k]);
-    const int pair = idx / g.T;                                              // s * L + l
-    const int ti = idx - pair * g.T;
-    if (pair != cur_pair) {
-      cur_pair = pair;
-      const int s = pair / L, l = pair - s * L;
-      e = ell_pair(sb, lb, sob, lob, S, L, So, Lo, s, l);
-      rsx = xf - e.cx;                                                       // :72
-      rsy = yf - e.cy;
-      rsz = g.sz - e.cz;
-      rex = xf - e.cx;                                                       // :74
-      rey = yf - e.cy;
-      rez = g.ez - e.cz;
-      dps = rsx * e.nx;
-      dps = dps + rsy * e.ny;
-      dps = dps + rsz * e.nz;
-      dpe = rex * e.nx;
-      dpe = dpe + rey * e.ny;
-      dpe = dpe + rez * e.nz;
-    }
-    const float value = tb[idx];                                             // > 0 (:77)
-    float tc = (float)ti * g.w;                                              // :79-80
-    tc = tc + g.off;
-    tc = tc - e.sd;
-    tc = tc - e.ld;
-    if (!(tc > e.len)) continue;                                             // :81
-    const float r0 = tc / 2.f;                                               // :83
-    float r1s = r0 * r0;
-    r1s = r1s - (e.len * e.len) / 4.f;                                       // :84
-    const float r1 = sqrt_rn(r1s);
-    const float sc = r1 / r0;                                                // :85
-    const float ks = (sc - 1.f) * dps;                                       // :87
-    const float stx = rsx + ks * e.nx, sty = rsy + ks * e.ny, stz = rsz + ks * e.nz;
-    const float ke = (sc - 1.f) * dpe;                                       // :88
-    const float etx = rex + ke * e.nx, ety = rey + ke * e.ny, etz = rez + ke * e.nz;
+  const float depth = (float)g.D;
+  // The box of this wave's columns, a row longer at either end (a hit's row is
+  // rounded to the nearest, and row 0 takes what lies up to a row before it).
+  float bx0 = ok ? xf : INFINITY, bx1 = ok ? xf : -INFINITY;
+  float by0 = ok ? yf : INFINITY, by1 = ok ? yf : -INFINITY;
+  for (int m = 1; m < 64; m <<= 1) {
+    bx0 = fminf(bx0, __shfl_xor(bx0, m));
+    bx1 = fmaxf(bx1, __shfl_xor(bx1, m));
+    by0 = fminf(by0, __shfl_xor(by0, m));
+    by1 = fmaxf(by1, __shfl_xor(by1, m));
+  }
+  const float row_z = 2.f * fabsf(g.ez - g.sz) / depth;
+  const float bz0 = fminf(g.sz, g.ez) - row_z, bz1 = fmaxf(g.sz, g.ez) + row_z;
+  // Smallest and largest distance of (px, py, pz) to the box, added.
+  auto box_reach = [&](float px, float py, float pz, float* lo, float* hi) {
+    const float ax = fmaxf(fmaxf(bx0 - px, px - bx1), 0.f), cx = fmaxf(px - bx0, bx1 - px);
+    const float ay = fmaxf(fmaxf(by0 - py, py - by1), 0.f), cy = fmaxf(py - by0, by1 - py);
+    const float az = fmaxf(fmaxf(bz0 - pz, pz - bz1), 0.f), cz = fmaxf(pz - bz0, bz1 - pz);
+    *lo += sqrt_fast(ax * ax + ay * ay + az * az);
+    *hi += sqrt_fast(cx * cx + cy * cy + cz * cz);
+  };
+  float nx = 0.f, ny = 0.f, nz = 0.f;
+  float rsx = 0.f, rsy = 0.f, rsz = 0.f, rez = 0.f, dps = 0.f, dpe = 0.f;
+
+  // The row of one entry in this lane's column, -1 for none; k1m = r1/r0 - 1
+  // and r1q = r1^2 are the entry's.  MID: *out tells that a root or quotient
+  // leaves the range of the short forms.
+  auto row_of = [&](float k1m, float r1q, auto mid, bool* out) {
+    constexpr bool MID = decltype(mid)::value;
+    const float ks = k1m * dps;                                              // :87
+    const float stx = rsx + ks * nx, sty = rsy + ks * ny, stz = rsz + ks * nz;
+    const float ke = k1m * dpe;                                              // :88
+    const float etx = rsx + ke * nx, ety = rsy + ke * ny, etz = rez + ke * nz;
     float dx = etx - stx, dy = ety - sty, dz = etz - stz;                    // :89
     float rl = dx * dx;
     rl = rl + dy * dy;
     rl = rl + dz * dz;
-    const float rlen = sqrt_rn(rl);                                          // :90
-    const float ir = 1.f / rlen;                                             // :91
+    const float rlen = MID ? sqrt_rn_mid(rl) : sqrt_rn(rl);                  // :90
+    const float ir = MID ? recip_rn_mid(rlen) : 1.f / rlen;                  // :91
     dx = ir * dx;
     dy = ir * dy;
     dz = ir * dz;
@@ -637,22 +649,107 @@ __global__ __launch_bounds__(64) void arellano_kernel(
     float ss = stx * stx;
     ss = ss + sty * sty;
     ss = ss + stz * stz;
-    float v1 = v0 * v0 - (ss - r1 * r1);                                     // :94
-    if (!(v1 > 0.f) || !ok) continue;                                        // :95
-    v1 = sqrt_rn(v1);
+    float v1 = v0 * v0 - (ss - r1q);                                         // :94
+    const bool hit = (v1 > 0.f) & ok;                                        // :95
+    if (MID) {
+      const float other = hit ? v1 : rl;
+      *out = !(fminf(rl, other) >= 0x1p-64f && fmaxf(rl, other) <= 0x1p64f);
+    }
+    v1 = MID ? sqrt_rn_mid(v1) : sqrt_rn(v1);
     float d = -v0 - v1;
-    if (d < 0.f) d = -v0 + v1;                                               // :97-100
-    float bf = d / rlen;
-    bf = bf * (float)g.D;
+    d = d < 0.f ? -v0 + v1 : d;                                              // :97-100
+    float bf = MID ? div_recip_mid(d, rlen, ir) : d / rlen;
+    bf = bf * depth;
     bf = bf + 0.5f;
-    const int bini = (int)bf;                                                // :101-102
-    // :103-109: the interpolation weight is int - int = 0, so only bini
-    // receives the value.
-    if (bini >= 0 && bini < g.D) {
-      if (IN_LDS)
-        colacc[bini * 64 + lane] += value;
-      else
-        gcol[(size_t)bini * ncol] += value;
+    const int row = (int)bf;                                                 // :101-102
+    return hit & (row >= 0) & (row < g.D) ? row : -1;
+  };
+
+  for (int base = k0; base < k1; base += 64) {
+    const int n = min(64, k1 - base);
+    // lane j: entry base + j
+    const int idx = lb_list[base + min(lane, n - 1)];
+    const float value = tb[idx];                                             // > 0 (:77)
+    const int pair = idx / g.T;                                              // s * L + l
+    const int s = pair / L;
+    const EllPair e = ell_pair(sb, lb, sob, lob, S, L, So, Lo, s, pair - s * L);
+    float tc = (float)(idx - pair * g.T) * g.w;                              // :79-80
+    tc = tc + g.off;
+    tc = tc - e.sd;
+    tc = tc - e.ld;
+    const float r0 = tc / 2.f;                                               // :83
+    float r1s = r0 * r0;
+    r1s = r1s - (e.len * e.len) / 4.f;                                       // :84
+    const float r1 = sqrt_rn(r1s);
+    const float k1m = r1 / r0 - 1.f;                                         // :85
+    const float r1q = tc > e.len ? r1 * r1 : -INFINITY;                      // :81: no hit
+    // An ellipsoid that stays clear of the box hits no column of it.  Its points
+    // have distance sums tc; rounding of the sphere it is scaled to moves that
+    // by a part in 10^3 at most where the sphere is not small (r1^2 no less
+    // than 10^-3 of the box's largest sum, squared): 4 parts are left.
+    float lo = 0.f, hi = 0.f;
+    const int l = pair - s * L;
+    box_reach(sb[s], sb[S + s], sb[2 * S + s], &lo, &hi);
+    box_reach(lb[l], lb[L + l], lb[2 * L + l], &lo, &hi);
+    const bool clear = !(tc > e.len) || (r1q >= 1e-3f * hi * hi &&
+                                         (tc < lo - 4e-3f * hi || tc > hi * 1.004f));
+    unsigned long long todo = __ballot(lane < n && !clear);
+    auto entries = [&](const int* j, auto count) {
+      constexpr int U = decltype(count)::value;
+      int row[U];
+      bool out = false;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        bool o;
+        row[u] = row_of(readlane_f(k1m, j[u]), readlane_f(r1q, j[u]), std::true_type{}, &o);
+        out |= o;
+      }
+      if (__ballot(out) != 0) {
+        for (int u = 0; u < U; ++u)
+          row[u] = row_of(readlane_f(k1m, j[u]), readlane_f(r1q, j[u]), std::false_type{},
+                          nullptr);
+      }
+      // :103-109: the interpolation weight is int - int = 0, so only the row
+      // itself receives the value.
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float add = readlane_f(value, j[u]);
+        if (row[u] >= 0) {
+          if (IN_LDS)
+            colacc[row[u] * 64 + lane] += add;
+          else
+            gcol[(size_t)row[u] * ncol] += add;
+        }
+      }
+    };
+    int cur = -1;
+    while (todo != 0) {
+      int j[2];
+      j[0] = (int)__builtin_ctzll(todo);
+      todo &= todo - 1;
+      const int p = __builtin_amdgcn_readlane(pair, j[0]);
+      if (p != cur) {
+        cur = p;
+        nx = readlane_f(e.nx, j[0]);
+        ny = readlane_f(e.ny, j[0]);
+        nz = readlane_f(e.nz, j[0]);
+        const float cz = readlane_f(e.cz, j[0]);
+        rsx = xf - readlane_f(e.cx, j[0]);                                   // :72, :74
+        rsy = yf - readlane_f(e.cy, j[0]);
+        rsz = g.sz - cz;
+        rez = g.ez - cz;
+        dps = rsx * nx;
+        dps = dps + rsy * ny;
+        dpe = dps + rez * nz;
+        dps = dps + rsz * nz;
+      }
+      j[1] = todo != 0 ? (int)__builtin_ctzll(todo) : 63;
+      if (todo != 0 && __builtin_amdgcn_readlane(pair, j[1]) == p) {
+        todo &= todo - 1;
+        entries(j, std::integral_constant<int, 2>{});
+      } else {
+        entries(j, std::integral_constant<int, 1>{});
+      }
     }
   }
   if (IN_LDS && ok)

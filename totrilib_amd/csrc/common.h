@@ -110,6 +110,27 @@ __device__ __forceinline__ float div_const(float x, const DivConst& d) {
   return __builtin_fmaf(r, d.hi, q);
 }
 
+// Correctly rounded 1 / b for b in [2^-60, 2^60]: the hardware's reciprocal
+// (within 1 ulp) and two Newton steps, which leave the one mantissa that is
+// all ones to its known result, (1/2 + 2^-24) 2^-e.  Checked over every
+// mantissa and every start within 2 ulp.
+__device__ __forceinline__ float recip_rn_mid(float b) {
+  float y = __builtin_amdgcn_rcpf(b);
+  y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+  y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+  const unsigned u = __float_as_uint(b);
+  return (u | 0xff800000u) == 0xffffffffu ? __uint_as_float(0x7f000000u - u) : y;
+}
+
+// Correctly rounded a / b from y = RN(1 / b): a y is within 1.5 ulp, one
+// residual step makes it faithful, the second rounds it (Markstein).  For b as
+// in recip_rn_mid and quotients that neither overflow nor underflow.
+__device__ __forceinline__ float div_recip_mid(float a, float b, float y) {
+  float q = a * y;
+  q = __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), y, q);
+}
+
 // tc = t * w + off, rounded after the product and after the sum
 // (src/render/volume_cuda.cu:23).
 __device__ __forceinline__ float bin_distance(int t, float w, float off) {
