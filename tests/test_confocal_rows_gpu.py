@@ -6,6 +6,8 @@
 * A1's row walks settle a sample exactly only at the end of its row where one
   bin moves it by more than four guard widths, and at every sample otherwise:
   bin widths on both sides of that line, bit for bit against the oracle.
+* Calls too small to fill the chip are split down to one mirror quad (pair) of
+  scan points per range and to small column chunks: sizes around the limits.
 """
 import numpy as np
 import pytest
@@ -112,3 +114,31 @@ def test_a1_bins_within_the_guard(w, T, scan):
         assert np.abs(got - want).max() <= 2.6e-3 * want.max()
         n += int(act.sum())
     assert n > 0
+
+
+@pytest.mark.parametrize("shape,n,T", [
+    ((8, 8, 8), 2, 64),       # one quad
+    ((6, 4, 70), 4, 100),     # four quads, a partial tile, 9 slabs
+    ((32, 32, 32), 16, 256),  # one quad per range
+    ((20, 20, 20), 24, 200),  # 144 quads: ranges of one and two
+    ((18, 7, 24), 8, 150),    # odd Y: pairs
+    ((16, 16, 160), 8, 300),  # deep: chunks of few columns
+])
+def test_small_splits(shape, n, T):
+    from totrilib_amd.totri_cpp.render import (volume_confocal_forward,
+                                               volume_confocal_grad_volume)
+    X, Y, Z = shape
+    w = 3.0 / T
+    rng = np.random.default_rng(n + T)
+    mp = wall_grid(n)
+    vol = rng.random(shape).astype(np.float32)
+    G = rng.random((n * n, T)).astype(np.float32)
+    m = torch.from_numpy(np.ascontiguousarray(mp)).to(dev())
+    out = torch.full((n * n, T), float("nan"), device=dev())
+    volume_confocal_forward(torch.from_numpy(vol).to(dev()), m, out, ORIGIN, SIZE, w, 0.0)
+    gv = torch.full(shape, float("nan"), device=dev())
+    volume_confocal_grad_volume(gv, m, torch.from_numpy(G).to(dev()), ORIGIN, SIZE, w, 0.0)
+    ref = O.r1_forward(vol, mp, T, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64)
+    refv = O.a1_transpose(G, mp, X, Y, Z, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64)
+    assert rel_l2(out.cpu().numpy(), ref) < TOL
+    assert rel_l2(gv.cpu().numpy(), refv) < TOL

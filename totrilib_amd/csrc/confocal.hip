@@ -170,6 +170,13 @@ __device__ __forceinline__ int2 sample_rows(const ConfGeom& g, int col) {
   return g.rows ? g.rows[col] : make_int2(0, g.Z - 2);
 }
 
+// g without the row ranges, known to the compiler as such (the batched kernels
+// have none, and spend their registers elsewhere).
+__device__ __forceinline__ ConfGeom all_rows(ConfGeom g) {
+  g.rows = nullptr;
+  return g;
+}
+
 // One wave per column.
 __global__ __launch_bounds__(256) void sample_rows_kernel(const float* __restrict__ vol,
                                                           ConfGeom g, int2* __restrict__ rows) {
@@ -622,19 +629,32 @@ __global__ __launch_bounds__(64) void scan_mirror_kernel(const float* __restrict
   scan_mirror_item(mp, N, partner, (int)blockIdx.x);
 }
 
-// Inclusive scan of one int per thread over a 1024-thread workgroup.
-__device__ __forceinline__ int block_scan_1024(int v, int* s_cnt) {
-  const int tid = threadIdx.x;
-  __syncthreads();
-  s_cnt[tid] = v;
-  __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int u = tid >= off ? s_cnt[tid - off] : 0;
-    __syncthreads();
-    s_cnt[tid] += u;
-    __syncthreads();
+// Inclusive sum of one int per lane over each `width` lanes.  A rolled loop: the
+// batched detection shares CUs with running walks, and a workgroup of 16
+// waves waits until its registers fit beside theirs.
+__device__ __forceinline__ int lane_scan(int v, int width) {
+  const int lane = threadIdx.x & (width - 1);
+#pragma unroll 1
+  for (int off = 1; off < width; off <<= 1) {
+    const int u = __shfl_up(v, off, width);
+    if (lane >= off) v += u;
   }
-  return s_cnt[tid];
+  return v;
+}
+
+// Inclusive scan of one int per thread over a 1024-thread workgroup; *total is
+// its last value.  Within each wave by lane shuffles, then over the 16 waves'
+// sums: two barriers (a scan through LDS alone takes twenty).
+__device__ __forceinline__ int block_scan_1024(int v, int* s_cnt, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  v = lane_scan(v, 64);
+  __syncthreads();
+  if (lane == 63) s_cnt[wave] = v;
+  __syncthreads();
+  const int sums = lane_scan(s_cnt[lane & 15], 16);
+  *total = __shfl(sums, 15);
+  const int before = __shfl(sums, wave - (wave > 0));
+  return wave > 0 ? v + before : v;
 }
 
 // One workgroup: checks whether the mirror relation splits all N scan
@@ -647,7 +667,7 @@ __device__ __forceinline__ void scan_quads_block(const int* __restrict__ partner
                                                  int* __restrict__ quads,
                                                  int* __restrict__ pairs,
                                                  int* __restrict__ info) {
-  __shared__ int s_cnt[1024];
+  __shared__ int s_cnt[16];
   __shared__ int s_bad[2];
   const int tid = threadIdx.x;
   if (tid < 2) s_bad[tid] = 0;
@@ -678,10 +698,9 @@ __device__ __forceinline__ void scan_quads_block(const int* __restrict__ partner
   }
   if (qbad) atomicOr(&s_bad[0], 1);
   if (pbad) atomicOr(&s_bad[1], 1);
-  const int q_incl = block_scan_1024(qc, s_cnt);
-  const int n_quads = s_cnt[1023];
-  const int p_incl = block_scan_1024(pc, s_cnt);
-  const int n_pairs = s_cnt[1023];
+  int n_quads, n_pairs;
+  const int q_incl = block_scan_1024(qc, s_cnt, &n_quads);
+  const int p_incl = block_scan_1024(pc, s_cnt, &n_pairs);
   const bool quads_ok = s_bad[0] == 0;
   const bool pairs_ok = s_bad[1] == 0;
   if (quads_ok) {
@@ -1341,6 +1360,23 @@ void a6_pair_kernel(
                          chunks_per_group, lds2);
 }
 
+// Sum over p < n_parts of part[p * stride], in order, sixteen loads at a time (a
+// small call has few elements and many parts): 64 parts of 32^3 voxels 28 -> 9 us,
+// the benchmark step's 7 parts of 128^3 46 -> 30 us.
+__device__ __forceinline__ float sum_parts_at(const float* __restrict__ part, size_t stride,
+                                              int n_parts) {
+  constexpr int U = 16;
+  float v = part[0];
+  for (int p = 1; p < n_parts; p += U) {
+    float x[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) x[k] = part[(size_t)min(p + k, n_parts - 1) * stride];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v = p + k < n_parts ? v + x[k] : v;
+  }
+  return v;
+}
+
 // Sum of partials in a fixed order where the number of parts depends on
 // which path ran: the xy-mirror one (info[0] set and n_sym given), else the
 // x-pair one (info[2] set and n_pair given), else the general one.
@@ -1352,9 +1388,7 @@ __global__ void sum_partials_flag_kernel(const float* __restrict__ part,
   const int n_parts = (n_sym && info[0]) ? n_sym : (n_pair && info[2]) ? n_pair : n_gen;
   for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
        e += (size_t)gridDim.x * blockDim.x) {
-    float v = part[e];
-    for (int p = 1; p < n_parts; ++p) v += part[(size_t)p * n + e];
-    store_elem(out + e, v);
+    store_elem(out + e, sum_parts_at(part + e, n, n_parts));
   }
 }
 
@@ -1369,9 +1403,7 @@ __device__ __forceinline__ float a1_boundary(const float* __restrict__ bnd, size
   if (z == 0 || z % slab_h) return 0.f;
   const size_t ncol = n / (size_t)Z, col = e / (size_t)Z;
   const int sb = z / slab_h - 1;
-  float b = bnd[col * n_slabs + sb];
-  for (int p = 1; p < n_parts; ++p) b += bnd[((size_t)p * ncol + col) * n_slabs + sb];
-  return b;
+  return sum_parts_at(bnd + col * n_slabs + sb, ncol * n_slabs, n_parts);
 }
 
 // A1 partial sums: the xy-mirror kernel ran when quad_on and info[0] (its
@@ -1396,8 +1428,7 @@ __global__ void sum_partials_a1_kernel(const float* __restrict__ part,
   const int slabs = (quad || pair) ? n_slabs : n_slabs_gen;
   for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
        e += (size_t)gridDim.x * blockDim.x) {
-    float v = part[e];
-    for (int p = 1; p < n_parts; ++p) v += part[(size_t)p * n + e];
+    float v = sum_parts_at(part + e, n, n_parts);
     if (b) v += a1_boundary(b, e, n, Z, slabs, n_parts, slab_h);
     out[e] = v;
   }
@@ -1551,9 +1582,7 @@ __global__ void sum_partials_kernel(const float* __restrict__ part, int n_parts,
                                     size_t n, OutT* __restrict__ out) {
   for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n;
        e += (size_t)gridDim.x * blockDim.x) {
-    float v = part[e];
-    for (int p = 1; p < n_parts; ++p) v += part[(size_t)p * n + e];
-    store_elem(out + e, v);
+    store_elem(out + e, sum_parts_at(part + e, n, n_parts));
   }
 }
 
@@ -2936,6 +2965,19 @@ R1Plan plan_r1(int64_t X, int64_t Y, int64_t Z, int64_t N, int64_t T, int wg_per
   return p;
 }
 
+// Column groups per chunk, at most rpc, that give every CU kFillR1 workgroups of
+// `blocks` scan blocks times the chunks of n_reps column groups; never fewer than
+// kMinRepsR1.  32^3 voxels, 16^2 points, 256 bins: 144 workgroups took 50 us, 512
+// take 22; 32^3, 32^2 points, 512 bins, render and gradient: 356 -> 273 us (with
+// 4 and 4 instead of 2 and 8, 288: more partial sums).
+constexpr int kFillR1 = 2, kMinRepsR1 = 8;
+int64_t fill_chunk(int64_t rpc, int64_t n_reps, int64_t blocks) {
+  const int64_t chunks = (kFillR1 * (int64_t)device_cu_count() + blocks - 1) / blocks;
+  const int64_t fill = n_reps / chunks;
+  if (rpc > fill) rpc = fill < kMinRepsR1 ? (rpc < kMinRepsR1 ? rpc : kMinRepsR1) : fill;
+  return rpc;
+}
+
 R1SymPlan plan_r1_sym(int64_t X, int64_t Y, int64_t Z, int64_t N, int64_t T,
                       const R1Plan& gen) {
   R1SymPlan p;
@@ -2948,9 +2990,11 @@ R1SymPlan plan_r1_sym(int64_t X, int64_t Y, int64_t Z, int64_t N, int64_t T,
   const int64_t n_reps = (X / 2) * (Y / 2);
   int64_t rpc = kChunkVoxels / (4 * (Z + 1));  // column quads plus a zero row each
   if (rpc > 64) rpc = 64;
+  const int64_t quad_blocks = (N / 4 + kWaves - 1) / kWaves;
+  // Too few chunks to give every CU kFillR1 workgroups: smaller ones
+  rpc = fill_chunk(rpc, n_reps, quad_blocks);
   p.reps_per_chunk = (int)rpc;
   const int64_t total_chunks = (n_reps + rpc - 1) / rpc;
-  const int64_t quad_blocks = (N / 4 + kWaves - 1) / kWaves;
   // four workgroups per CU and pass (two run at a time): smaller items
   // shorten the tail of the last wave of workgroups
   const int64_t target = 4 * (int64_t)device_cu_count();
@@ -2981,9 +3025,10 @@ R1SymPlan plan_r1_pair(int64_t X, int64_t Y, int64_t Z, int64_t N, int64_t T,
   const int64_t n_reps = (X / 2) * Y;
   int64_t rpc = kChunkVoxels / (2 * (Z + 1));  // column pairs plus a zero row each
   if (rpc > 64) rpc = 64;
+  const int64_t pair_blocks = (N / 2 + kWaves - 1) / kWaves;
+  rpc = fill_chunk(rpc, n_reps, pair_blocks);
   p.reps_per_chunk = (int)rpc;
   const int64_t total_chunks = (n_reps + rpc - 1) / rpc;
-  const int64_t pair_blocks = (N / 2 + kWaves - 1) / kWaves;
   const int64_t target = 4 * (int64_t)device_cu_count();
   int64_t G = 1;
   if (pair_blocks < target) G = (target + pair_blocks - 1) / pair_blocks;
@@ -3315,6 +3360,18 @@ struct A1QuadPlan {
   int tiles_x, tiles_y, n_slabs, n_ranges;
 };
 
+// At most R scan ranges of n scan groups: ranges of `least` groups or more, of
+// fewer only as far as every SIMD gets one wave.  32^3 voxels, 64 quads: 256
+// items took 97 us, 1,024 take 49; where the chip is full, shorter ranges only
+// add partial volumes.
+int64_t limit_ranges(int64_t R, int64_t items, int64_t n, int64_t least) {
+  const int64_t simds = 4 * (int64_t)device_cu_count();
+  int64_t fill = (simds + items - 1) / items;
+  if (fill > n) fill = n;
+  const int64_t most = n / least > fill ? n / least : fill;
+  return R < most ? R : most;
+}
+
 A1QuadPlan plan_a1_quad(int64_t X, int64_t Y, int64_t Z, int64_t N) {
   A1QuadPlan p;
   memset(&p, 0, sizeof(p));
@@ -3329,18 +3386,18 @@ A1QuadPlan plan_a1_quad(int64_t X, int64_t Y, int64_t Z, int64_t N) {
   // times with the geometry, and with only one or two rounds the slots that
   // draw two costly items set the kernel's time.  Partial volumes then take
   // at most 64 x CU x 2048 voxels of floats (128 MiB on 256 CUs) at any
-  // volume size.  Ranges keep at least 4 quads.
+  // volume size (see limit_ranges for short ranges).
   const int64_t target = 64 * (int64_t)device_cu_count();
   int64_t R = 1;
   if (items < target) R = (target + items - 1) / items;
-  if (R > N / 16) R = N / 16;
+  R = limit_ranges(R, items, N / 4, 4);
   if (R < 1) R = 1;
   p.n_ranges = (int)R;
   return p;
 }
 
 // Plan of the x-pair row walk: tiles of 8x8 columns of the half grid
-// x < 0, 8-row slabs, pair ranges as in plan_a1_quad (at least 4 pairs each).
+// x < 0, 8-row slabs, pair ranges as in plan_a1_quad.
 A1QuadPlan plan_a1_pair_rows(int64_t X, int64_t Y, int64_t Z, int64_t N) {
   A1QuadPlan p;
   memset(&p, 0, sizeof(p));
@@ -3353,7 +3410,7 @@ A1QuadPlan plan_a1_pair_rows(int64_t X, int64_t Y, int64_t Z, int64_t N) {
   const int64_t target = 64 * (int64_t)device_cu_count();
   int64_t R = 1;
   if (items < target) R = (target + items - 1) / items;
-  if (R > N / 8) R = N / 8;
+  R = limit_ranges(R, items, N / 2, 4);
   if (R < 1) R = 1;
   p.n_ranges = (int)R;
   return p;
