@@ -60,3 +60,38 @@ def test_velten_stages(res, S, T):
     got = BackprojectionExhaustiveVelten.apply(t(tr), t(scan), t(laser), vd, bd).cpu().numpy()
     ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, w, off, mode=O.FP32)
     assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [9, 10, 11, 12, 16, 17, 36])
+@pytest.mark.parametrize("T", [1600, 1900, 2200, 2500])   # 11, 9, 8 and 7 rows to a stage
+def test_velten_exhaustive_few_rows_per_stage(L, T):
+    """Laser points in several tiles where a stage holds few rows."""
+    from totrilib_amd.reconstruct import BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(L + T)
+    S, res = 5, (5, 6, 11)
+    scan, laser = points(rng, 1, S), points(rng, 1, L)
+    tr = rng.random((1, T, S, L)).astype(np.float32)
+    got = BackprojectionExhaustiveVelten.apply(
+        t(tr), t(scan), t(laser), VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T)).cpu().numpy()
+    ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
+    assert ref.any()
+    assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("res,T,L", [((56, 56, 56), 640, 9), ((56, 56, 56), 700, 16),
+                                     ((48, 48, 48), 1024, 9)])
+def test_velten_exhaustive_smaller_stages(res, T, L):
+    """Volumes of several workgroups per CU, whose stages are smaller."""
+    from totrilib_amd.reconstruct import BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(T)
+    scan, laser = points(rng, 1, 3), points(rng, 1, L)
+    tr = rng.random((1, T, 3, L)).astype(np.float32)
+    got = BackprojectionExhaustiveVelten.apply(
+        t(tr), t(scan), t(laser), VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T)).cpu().numpy()
+    ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
+    assert ref.any()
+    assert np.array_equal(got.astype(np.float64), ref)

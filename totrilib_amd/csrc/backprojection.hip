@@ -1014,15 +1014,19 @@ int launch_velten_ex(const float* head, const float* rows, float* volume, const 
 
 // The tile size for L laser points, tiles of at most 16 points and `most`
 // rows: tiles of equal size, rounded up to one that is compiled.  A tile
-// that is not full masks its last points, so all laser points of a call with
-// several scan points per unit (L <= 6) make exactly one tile.
+// that is not full masks its last points.  Tiles of up to six points belong to
+// calls whose laser points make exactly one (their units take several scan
+// points); several tiles have seven points or more, also where that masks more
+// of the last.
 int velten_ex_tile(int64_t L, int64_t most) {
   static const int sizes[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
   int top = 0;
   for (int k : sizes)
     if (k <= most) top = k;
   if (top == 0 || (L > top && top < 7)) return 0;
-  const int64_t nt = (L + top - 1) / top, kt = (L + nt - 1) / nt;
+  const int64_t nt = (L + top - 1) / top;
+  int64_t kt = (L + nt - 1) / nt;
+  if (nt > 1 && kt < 7) kt = 7;  // top >= 7 here
   for (int k : sizes)
     if (k >= kt) return k;
   return 0;
@@ -1049,7 +1053,7 @@ int velten_ex(const float* head, const float* rows, float* volume, const BoxGeom
     return launch_velten_ex<KT, NTL, 1>(head, rows, volume, g, S, L, sp, st);
 #define TOTRI_EX4(KT) TOTRI_EX(KT, 1) TOTRI_EX(KT, 2) TOTRI_EX(KT, 3) TOTRI_EX(KT, 0)
 #define TOTRI_EX1(KT) \
-  if (kt == KT) \
+  if (kt == KT && nt == 1) \
     return pairs == 16 ? launch_velten_ex<KT, 1, ex_scan_group(KT, 16)>(head, rows, volume, g, S, L, sp, st) \
                        : launch_velten_ex<KT, 1, ex_scan_group(KT, 8)>(head, rows, volume, g, S, L, sp, st);
   TOTRI_EX1(1) TOTRI_EX1(2) TOTRI_EX1(3) TOTRI_EX1(4) TOTRI_EX1(5) TOTRI_EX1(6)
@@ -1057,7 +1061,7 @@ int velten_ex(const float* head, const float* rows, float* volume, const BoxGeom
 #undef TOTRI_EX1
 #undef TOTRI_EX4
 #undef TOTRI_EX
-  return fail(TOTRI_EINVAL, "no kernel for tiles of %d laser points", kt);
+  return fail(TOTRI_EINVAL, "no kernel for %lld tiles of %d laser points", (long long)nt, kt);
 }
 
 }  // namespace
