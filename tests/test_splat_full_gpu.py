@@ -96,3 +96,22 @@ def test_full_splat_zero_sigma():
     assert np.isnan(vol[0, :, at]).all()
     assert np.isfinite(vol[0, :, ~at]).all()
     assert rel_l2(vol[0][:, ~at], want[0][:, ~at]) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ws", [True, False])
+@pytest.mark.parametrize("at", [0, 300, 1499])
+def test_full_splat_zero_sigma_split(at, ws):
+    """The same where the RBFs are split over workgroups, in any split's chunks."""
+    rng = np.random.default_rng(4)
+    res = (13, 11, 9)
+    rbf = _rbf(rng, 1, 1500, 1)
+    rbf[0, at] = (0.0, 0.0, 1.5, 0.0, 1.0)      # the grid's middle voxel
+    G = np.zeros((1, 2) + res, np.float32)
+    vol, _, nf, _ = _calls(rbf, res, G, ws)
+    assert (nf > 0) == ws
+    want = O.splat_forward(np.delete(rbf, at, 1), res, VS, VE, mode=O.PURE64)
+    mid = np.zeros(res, bool)
+    mid[6, 5, 4] = True
+    assert np.isnan(vol[0][:, mid]).all()
+    assert rel_l2(vol[0][:, ~mid], want[0][:, ~mid]) < 1e-5

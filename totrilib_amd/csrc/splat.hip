@@ -625,21 +625,25 @@ __global__ __launch_bounds__(kSepWaves * 64) void splat_sep_kernel(
   const int col = col0 + 16 * (wave % kSepNT) + r;
   const int zr = z0 + 16 * (wave / kSepNT) + 4 * q;
   if (col >= HW) return;
-  if (any_degenerate && split == 0) {
+  if (any_degenerate) {  // of this split's RBFs
     const float xc = splat_coord(col % g.W, g.W, g.sx, g.ex);
     const float yc = splat_coord(col / g.W, g.H, g.sy, g.ey);
-    for (int i = 0; i < g.N; ++i) {
-      const float* p = rb + (size_t)i * RC;
-      const float k = gauss_k(p[3]);
-      if (!sep_degenerate(k)) continue;
+    constexpr int G = kSepWaves * kSepChunk;
+    for (int64_t i0 = (int64_t)split * G; i0 < g.N; i0 += (int64_t)n_split * G) {
+      const int end = (int)(i0 + G < g.N ? i0 + G : g.N);
+      for (int i = (int)i0; i < end; ++i) {
+        const float* p = rb + (size_t)i * RC;
+        const float k = gauss_k(p[3]);
+        if (!sep_degenerate(k)) continue;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float zc = splat_coord(min(zr + u, g.D - 1), g.D, g.sz, g.ez);
-        const float w = gauss_exp2(rbf_r2(xc, yc, zc, p[0], p[1], p[2]), k);
-        sum[0][u] += w;
+        for (int u = 0; u < 4; ++u) {
+          const float zc = splat_coord(min(zr + u, g.D - 1), g.D, g.sz, g.ez);
+          const float w = gauss_exp2(rbf_r2(xc, yc, zc, p[0], p[1], p[2]), k);
+          sum[0][u] += w;
 #pragma unroll
-        for (int c = 1; c < C; ++c)
-          if (a0 + c - 1 < g.A) sum[c][u] += w * p[4 + a0 + c - 1];
+          for (int c = 1; c < C; ++c)
+            if (a0 + c - 1 < g.A) sum[c][u] += w * p[4 + a0 + c - 1];
+        }
       }
     }
   }
