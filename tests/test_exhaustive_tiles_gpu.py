@@ -80,3 +80,50 @@ def test_adjoint_infinite_gradient(T, D):
     assert 0 < np.count_nonzero(~fine) < fine.size
     assert np.array_equal(np.isfinite(got), fine)
     assert rel_l2(got[fine], ref[fine]) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("big", [1e8, 1e10, 1e14, 1e20, 3e38])
+@pytest.mark.parametrize("T,D", [(150, 20), (700, 6), (2600, 6), (9000, 6)])
+def test_adjoint_large_gradient(T, D, big):
+    """A large finite bin costs the voxels whose spans do not hold it no accuracy."""
+    rng = np.random.default_rng(T)
+    res, w = (D, 5, 7), 8.0 / T
+    scan, laser = points(rng, 1, 3), points(rng, 1, 2)
+    G = rng.standard_normal((1, T, 3, 2)).astype(np.float32)
+    G[0, T // 2, 1, 1] = np.inf
+    clear = np.isfinite(O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64))
+    G[0, T // 2, 1, 1] = big
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64)
+    got = adjoint(G, res, scan, laser, w, 0.0)
+    assert 0 < np.count_nonzero(~clear) < clear.size
+    assert rel_l2(got[clear], ref[clear]) < 1e-6
+    assert rel_l2(got, ref) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [700, 2600])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 48])      # bin widths past DivConst's range
+def test_adjoint_marked_rows(T, scale):
+    """Batches without, with a few and with many rows of large range."""
+    from totrilib_amd.totri_cpp.render import volume_render_exhaustive_grad_volume
+    rng = np.random.default_rng(T)
+    res, w = (6, 5, 7), 8.0 / T * scale
+    VS, VE = ((-scale, -scale, 0.5 * scale), (scale, scale, 2.5 * scale))
+    scan, laser = (points(rng, 3, n) * np.float32(scale) for n in (9, 5))
+    G = rng.standard_normal((3, T, 9, 5)).astype(np.float32)
+    clear = np.ones((3,) + res, bool)
+    for b, pairs in ((1, [(8, 4)]), (2, [(s, l) for s in range(9) for l in range(3)])):
+        for s, l in pairs:
+            G[b, T // 2, s, l] = np.inf
+    clear = np.isfinite(O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64))
+    G[np.isinf(G)] = 1e15
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64)
+    out = torch.empty((3,) + res, device="cuda")
+    empty = torch.empty(3, 3, 0, device="cuda")
+    volume_render_exhaustive_grad_volume(t(G), t(scan), t(laser), empty, empty, out, VS, VE, w, 0.0)
+    got = out.cpu().numpy()
+    for b in range(3):
+        assert clear[b].any()
+        assert rel_l2(got[b][clear[b]], ref[b][clear[b]]) < 1e-6
+        assert rel_l2(got[b], ref[b]) < 1e-6

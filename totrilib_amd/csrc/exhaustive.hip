@@ -316,8 +316,13 @@ __global__ __launch_bounds__(kR2Waves * 64) void r2_forward_kernel(
 // longer ones (K = 0) the rows are kept as running sums
 // C[t] = g[0] + .. + g[t - 1] in double as well: three differences of four
 // neighbouring entries give g[first], the sum between and g[last] for spans
-// of any length, more exactly than adding the bins in float.  A batch with an
-// infinite or NaN gradient, which running sums would spread, adds the bins.
+// of any length.  The sums are formed in two doubles and rounded once, so a
+// difference is off by at most 2^-52 of the row's largest |C|, and exact over
+// empty bins.  A row where that exceeds 2^-24 of its smallest nonzero bin, or
+// that holds an infinity or a NaN, is marked: its running sums are zeros, and
+// its pairs add the bins (a5_marked_kernel).  Of rows of 1,000 normal deviates
+// about one in 5,000 is marked; a batch of many marked rows takes the short
+// form, which adds the bins of long spans from LDS.
 
 // Row stride of the transposed gradient: whole float4s.
 __host__ __device__ __forceinline__ int a5_row(int T) { return (T + 3) & ~3; }
@@ -327,60 +332,96 @@ __host__ __device__ __forceinline__ int a5_stride(int T) { return (T + 2) & ~1; 
 
 struct A5Rows {
   const float* g;     // [B][S*L][a5_row(T)] the transposed gradient
-  const double* c;    // [B][S*L][a5_stride(T)] its running sums
-  const int* bad;     // [B] whether the batch holds an infinity or a NaN
+  double* c;          // [B][S*L][a5_stride(T)] its running sums
+  int* marked;        // [B][S*L] whether a row's running sums are left out
+  int* count;         // [B] marked rows
 };
 
+// The batches a launch takes, by their marked rows.
+enum A5Take { kA5All, kA5Few, kA5Many };
+
+// Adding bins in the short form takes about as long as everything else at one
+// marked row in 32.
+__device__ __forceinline__ bool a5_many(int count, int rows) { return count > rows / 32; }
+
 struct A5Layout {
-  size_t prefix, head, bad, end;
+  size_t prefix, head, marked, count, end;
 };
 
 A5Layout a5_layout(int64_t B, int64_t T, int64_t S, int64_t L) {
   A5Layout l;
   l.prefix = align256((size_t)B * S * L * a5_row((int)T) * sizeof(float));
   l.head = l.prefix + align256((size_t)B * S * L * a5_stride((int)T) * sizeof(double));
-  l.bad = l.head + align256((size_t)B * (S + L) * sizeof(float4));
-  l.end = l.bad + align256((size_t)B * sizeof(int));
+  l.marked = l.head + align256((size_t)B * (S + L) * sizeof(float4));
+  l.count = l.marked + align256((size_t)B * S * L * sizeof(int));
+  l.end = l.count + align256((size_t)B * sizeof(int));
   return l;
 }
 
+// An unevaluated sum of two doubles, |lo| at most half an ulp of hi.
+struct Sum2 {
+  double hi, lo;
+};
+
+__device__ __forceinline__ Sum2 add2(const Sum2& a, const Sum2& b) {
+  const double s = a.hi + b.hi, v = s - a.hi;
+  const double e = ((a.hi - (s - v)) + (b.hi - v)) + (a.lo + b.lo);
+  Sum2 r;
+  r.hi = s + e;
+  r.lo = e - (r.hi - s);
+  return r;
+}
+
 // One wave per row, eight bins per lane and step.
-__global__ __launch_bounds__(256) void a5_prefix_kernel(const float* __restrict__ gT,
-                                                        double* __restrict__ c,
-                                                        int* __restrict__ bad, ExGeom g,
-                                                        int rows) {
+__global__ __launch_bounds__(256) void a5_prefix_kernel(A5Rows rows, ExGeom g, int n_rows) {
   const int lane = threadIdx.x & 63;
   const size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= (size_t)g.B * rows) return;
-  const float* src = gT + r * a5_row(g.T);
-  double* dst = c + r * a5_stride(g.T);
-  double base = 0.0;
+  if (r >= (size_t)g.B * n_rows) return;
+  const float* src = rows.g + r * a5_row(g.T);
+  double* dst = rows.c + r * a5_stride(g.T);
+  Sum2 base = {0.0, 0.0};
   bool finite = true;
+  float least = INFINITY;  // smallest nonzero |bin|
+  double most = 0.0;       // largest |running sum|
   for (int t0 = 0; t0 < g.T; t0 += 512) {
-    double s[8], sum = 0.0;
+    Sum2 s[8], sum = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int t = t0 + lane * 8 + k;
-      const float v = t < g.T ? src[t] : 0.f;
-      finite = finite && fabsf(v) < INFINITY;
+      const float v = t < g.T ? src[t] : 0.f, m = fabsf(v);
+      finite = finite && m < INFINITY;
+      least = m > 0.f ? fminf(least, m) : least;
       s[k] = sum;
-      sum += (double)v;
+      sum = add2(sum, Sum2{(double)v, 0.0});
     }
-    double up = sum;  // inclusive sum over the lanes
+    Sum2 up = sum;  // inclusive sum over the lanes
     for (int m = 1; m < 64; m <<= 1) {
-      const double o = __shfl_up(up, m, 64);
-      if (lane >= m) up += o;
+      const Sum2 o = {__shfl_up(up.hi, m, 64), __shfl_up(up.lo, m, 64)};
+      if (lane >= m) up = add2(up, o);
     }
-    const double before = base + (up - sum);
+    Sum2 before = {__shfl_up(up.hi, 1, 64), __shfl_up(up.lo, 1, 64)};
+    before = lane > 0 ? add2(base, before) : base;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int t = t0 + lane * 8 + k;
-      if (t < g.T) dst[t] = before + s[k];
+      const double v = add2(before, s[k]).hi;
+      if (t < g.T) dst[t] = v;
+      most = fmax(most, fabs(v));
     }
-    base += __shfl(up, 63, 64);
+    base = add2(base, Sum2{__shfl(up.hi, 63, 64), __shfl(up.lo, 63, 64)});
   }
-  if (lane == 0) dst[g.T] = base;
-  if (!finite) atomicOr(bad + r / rows, 1);
+  if (lane == 0) dst[g.T] = base.hi;
+  most = fmax(most, fabs(base.hi));
+  for (int m = 32; m >= 1; m >>= 1) {
+    least = fminf(least, __shfl_xor(least, m, 64));
+    most = fmax(most, __shfl_xor(most, m, 64));
+  }
+  const bool mark = __any(!finite) || most > 0x1p28 * (double)least;
+  if (mark)
+    for (int t = lane; t <= g.T; t += 64) dst[t] = 0.0;
+  if (lane != 0) return;
+  rows.marked[r] = mark ? 1 : 0;
+  if (mark) atomicAdd(rows.count + r / n_rows, 1);
 }
 
 __global__ void zero_f32_kernel(float* __restrict__ out, int n) {
@@ -388,16 +429,56 @@ __global__ void zero_f32_kernel(float* __restrict__ out, int n) {
   if (i < n) out[(size_t)blockIdx.y * n + i] = 0.f;
 }
 
-// Gradient of one (voxel, pair) from its two path lengths, bin by bin, in the
-// reference's arithmetic (volume_cuda.cu:341-374), unit occupancy.
+// Gradient of one (voxel, pair) from its two path lengths, bin by bin (U at a
+// time), in the reference's arithmetic (volume_cuda.cu:341-374), unit
+// occupancy.  The bins between are added in double: in float, spans of hundreds
+// of bins lose two digits.
+template <int U>
 __device__ __forceinline__ float a5_pair_any(const ExGeom& g, float d0, float d1,
                                              const float* row) {
   const Span sp = span_of(g, 1.f, d0, d1);
   if (sp.first > sp.last) return 0.f;
   if (sp.first == sp.last) return sp.wf * row[sp.first];
-  float m = 0.f;
-  for (int bn = sp.first + 1; bn < sp.last; ++bn) m += row[bn];
-  return sp.wf * row[sp.first] + sp.wm * m + sp.wl * row[sp.last];
+  double m = 0.0;
+  for (int bn = sp.first + 1; bn < sp.last; bn += U) {
+    float v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = row[min(bn + k, sp.last)];
+#pragma unroll
+    for (int k = 0; k < U; ++k) m += bn + k < sp.last ? (double)v[k] : 0.0;
+  }
+  return sp.wf * row[sp.first] + sp.wm * (float)m + sp.wl * row[sp.last];
+}
+
+// The marked rows of batches with few, added to the running sums' result: a lane
+// per voxel, in row order.
+__global__ __launch_bounds__(64) void a5_marked_kernel(A5Rows rows,
+                                                       const float4* __restrict__ head,
+                                                       float* __restrict__ grad, ExGeom g, int S,
+                                                       int L) {
+  const int b = blockIdx.y, n_rows = S * L, lane = threadIdx.x;
+  const int n = rows.count[b];
+  if (n == 0 || a5_many(n, n_rows)) return;
+  const int nvox = g.D * g.H * g.W;
+  const int v = (int)blockIdx.x * 64 + lane;
+  const int vv = v < nvox ? v : 0;
+  float xf, yf, zf0, zf1;
+  voxel_faces(g, vv % g.W, (vv / g.W) % g.H, vv / (g.W * g.H), &xf, &yf, &zf0, &zf1);
+  const float4* hs = head + (size_t)b * (S + L);
+  const int* marked = rows.marked + (size_t)b * n_rows;
+  float acc = 0.f;
+  for (int r0 = 0; r0 < n_rows; r0 += 64) {
+    unsigned long long todo = __ballot(r0 + lane < n_rows && marked[r0 + lane] != 0);
+    for (; todo != 0; todo &= todo - 1) {
+      const int r = r0 + (int)__builtin_ctzll(todo);
+      const int s = r / L;
+      const float4 ps = hs[s], pl = hs[S + r - s * L];
+      const float d0 = dist3(ps.x, ps.y, ps.z, xf, yf, zf0) + dist3(pl.x, pl.y, pl.z, xf, yf, zf0);
+      const float d1 = dist3(ps.x, ps.y, ps.z, xf, yf, zf1) + dist3(pl.x, pl.y, pl.z, xf, yf, zf1);
+      acc += a5_pair_any<8>(g, d0, d1, rows.g + ((size_t)b * n_rows + r) * a5_row(g.T));
+    }
+  }
+  if (v < nvox) grad[(size_t)b * nvox + v] += acc;
 }
 
 constexpr int kA5Pairs = 8;  // (scan, laser) pairs of a unit, at most
@@ -421,10 +502,11 @@ template <int K, int KT, bool STAGED, int NTH>
 __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
     A5Rows rows, const float4* __restrict__ head,  // [B][S + L]
     float* __restrict__ grad,                      // [B][D][H][W]
-    ExGeom g, int S, int L, int U, int cap, DivConst dw) {
+    ExGeom g, int S, int L, int U, int cap, DivConst dw, int take) {
   extern __shared__ float4 lds4[];
   constexpr int SG = kA5Pairs / KT > 1 ? kA5Pairs / KT : 1;
   const int b = blockIdx.y;
+  if (take != kA5All && a5_many(rows.count[b], S * L) != (take == kA5Many)) return;
   const int nvox = g.D * g.H * g.W;
   const int P = K > 0 ? a5_row(g.T) : 2 * a5_stride(g.T);  // floats of a staged row
   const int v = blockIdx.x * NTH + threadIdx.x;
@@ -437,7 +519,6 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
   const float4* hl = hs + S;
   const float* gb = rows.g + (size_t)b * S * L * a5_row(g.T);
   const float* cb = K > 0 ? gb : (const float*)(rows.c + (size_t)b * S * L * a5_stride(g.T));
-  const bool fast = dw.ok && (K > 0 || !rows.bad[b]);  // uniform
   float* stage = (float*)lds4;
   const int n_units = (S + SG - 1) / SG;
   // distances of n points (uniform) to the voxel's faces
@@ -525,7 +606,7 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
         float ds0[SG], ds1[SG];
         faces([&](int i) { return hs[min(s0 + i, S - 1)]; }, ds0, ds1,
               std::integral_constant<int, SG>{});
-        if (fast) {
+        if (dw.ok && take != kA5Many) {  // (most units of those add the bins)
           float x0[SG][KT], x1[SG][KT];
           int f[SG][KT], l[SG][KT];
           bool clipped = ns < SG || nl < KT, odd = false;
@@ -574,8 +655,9 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
         for (int i = 0; i < SG; ++i)
 #pragma unroll
           for (int j = 0; j < KT; ++j)
-            if (i < ns && j < nl)
-              acc += a5_pair_any(g, ds0[i] + dl0[j], ds1[i] + dl1[j],
+            if (i < ns && j < nl &&
+                !(K == 0 && rows.marked[((size_t)b * S + s0 + i) * L + l0 + j]))
+              acc += a5_pair_any<1>(g, ds0[i] + dl0[j], ds1[i] + dl1[j],
                                  any + (size_t)i * ai + j * a5_row(g.T));
       }
       if (STAGED) {
@@ -589,7 +671,8 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
 
 template <int K, int KT>
 int a5_launch_tile(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g,
-                   int64_t S, int64_t L, const StagePlan& sp, int64_t P, hipStream_t st) {
+                   int64_t S, int64_t L, const StagePlan& sp, int64_t P, int take,
+                   hipStream_t st) {
   constexpr int SG = kA5Pairs / KT > 1 ? kA5Pairs / KT : 1;
   const int64_t n = (int64_t)SG * std::min<int64_t>(KT, L);  // rows of a unit
   // masked reads may touch K floats past the last row
@@ -601,26 +684,17 @@ int a5_launch_tile(const A5Rows& rows, const float4* head, float* grad, const Ex
   const unsigned blocks = (unsigned)(((size_t)g.D * g.H * g.W + sp.threads - 1) / sp.threads);
   hipLaunchKernelGGL(kernel, dim3(blocks, (unsigned)g.B), dim3(sp.threads),
                      2 * (size_t)sp.cap * sizeof(float), st, rows, head, grad, g, (int)S, (int)L,
-                     (int)U, sp.cap, make_div_const(g.w));
+                     (int)U, sp.cap, make_div_const(g.w), take);
   return check_launch("r2_adjoint_kernel");
 }
 
-template <int K>
-int a5_launch_span(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g,
-                   int64_t S, int64_t L, hipStream_t st) {
-  const int64_t nvox = (int64_t)g.D * g.H * g.W;
-  const int64_t P = K > 0 ? a5_row(g.T) : 2 * a5_stride(g.T);
-  if (K == 0) {
-    const int64_t waves = g.B * S * L;
-    hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st,
-                       rows.g, (double*)rows.c, (int*)rows.bad, g, (int)(S * L));
-    const int rc = check_launch("a5_prefix_kernel");
-    if (rc) return rc;
-  }
-  StagePlan sp = stage_plan(g.B, nvox);
+// The stage and the laser points per tile of rows of P floats; 0 where the
+// rows of a unit do not fit.
+int a5_tile(const ExGeom& g, int64_t L, int64_t P, StagePlan* sp) {
+  *sp = stage_plan(g.B, (int64_t)g.D * g.H * g.W);
   // fewer, larger buffers rather than rows from global memory
-  if (kA5Pairs * P > sp.cap - kA5Slack) sp.cap = kStageMax;
-  const int64_t fit = (sp.cap - kA5Slack) / P;
+  if (kA5Pairs * P > sp->cap - kA5Slack) sp->cap = kStageMax;
+  const int64_t fit = (sp->cap - kA5Slack) / P;
   // The tile with the least work: every slot of a tile costs a pair (about
   // 50 instructions), every scan point of a tile two roots (about 35).
   static const int sizes[] = {1, 2, 3, 4, 6, 8};
@@ -634,17 +708,32 @@ int a5_launch_span(const A5Rows& rows, const float4* head, float* grad, const Ex
       least = cost;
     }
   }
-  if (kt == 1) return a5_launch_tile<K, 1>(rows, head, grad, g, S, L, sp, P, st);
-  if (kt == 2) return a5_launch_tile<K, 2>(rows, head, grad, g, S, L, sp, P, st);
-  if (kt == 3) return a5_launch_tile<K, 3>(rows, head, grad, g, S, L, sp, P, st);
-  if (kt == 4) return a5_launch_tile<K, 4>(rows, head, grad, g, S, L, sp, P, st);
-  if (kt == 6) return a5_launch_tile<K, 6>(rows, head, grad, g, S, L, sp, P, st);
-  if (kt == 8) return a5_launch_tile<K, 8>(rows, head, grad, g, S, L, sp, P, st);
-  if (K > 0) return a5_launch_span<0>(rows, head, grad, g, S, L, st);
-  // rows too long for the stage: running sums in global memory
-  hipLaunchKernelGGL((r2_adjoint_kernel<0, 8, false, 256>),
+  return kt;
+}
+
+// Floats of a row that a stage holds, by form.
+template <int K>
+int64_t a5_floats(int T) {
+  return K > 0 ? a5_row(T) : 2 * (int64_t)a5_stride(T);
+}
+
+template <int K>
+int a5_launch_form(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g,
+                   int64_t S, int64_t L, int take, hipStream_t st) {
+  const int64_t P = a5_floats<K>(g.T);
+  StagePlan sp;
+  const int kt = a5_tile(g, L, P, &sp);
+  if (kt == 1) return a5_launch_tile<K, 1>(rows, head, grad, g, S, L, sp, P, take, st);
+  if (kt == 2) return a5_launch_tile<K, 2>(rows, head, grad, g, S, L, sp, P, take, st);
+  if (kt == 3) return a5_launch_tile<K, 3>(rows, head, grad, g, S, L, sp, P, take, st);
+  if (kt == 4) return a5_launch_tile<K, 4>(rows, head, grad, g, S, L, sp, P, take, st);
+  if (kt == 6) return a5_launch_tile<K, 6>(rows, head, grad, g, S, L, sp, P, take, st);
+  if (kt == 8) return a5_launch_tile<K, 8>(rows, head, grad, g, S, L, sp, P, take, st);
+  // rows too long for the stage: from global memory
+  const int64_t nvox = (int64_t)g.D * g.H * g.W;
+  hipLaunchKernelGGL((r2_adjoint_kernel<K, 8, false, 256>),
                      dim3((unsigned)((nvox + 255) / 256), (unsigned)g.B), dim3(256), 0, st, rows,
-                     head, grad, g, (int)S, (int)L, (int)S, 0, make_div_const(g.w));
+                     head, grad, g, (int)S, (int)L, (int)S, 0, make_div_const(g.w), take);
   return check_launch("r2_adjoint_kernel");
 }
 
@@ -654,9 +743,23 @@ int a5_launch_span(const A5Rows& rows, const float4* head, float* grad, const Ex
 int a5_launch(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g, int64_t S,
               int64_t L, hipStream_t st) {
   const double bins = 2.0 * fabs((double)g.ez - g.sz) / g.D / (double)g.w;
-  if (bins < 1.99) return a5_launch_span<2>(rows, head, grad, g, S, L, st);
-  if (bins < 5.95) return a5_launch_span<6>(rows, head, grad, g, S, L, st);
-  return a5_launch_span<0>(rows, head, grad, g, S, L, st);
+  StagePlan sp;
+  const bool staged = a5_tile(g, L, a5_floats<6>(g.T), &sp) > 0;
+  if (staged && bins < 1.99) return a5_launch_form<2>(rows, head, grad, g, S, L, kA5All, st);
+  if (staged && bins < 5.95) return a5_launch_form<6>(rows, head, grad, g, S, L, kA5All, st);
+  const int64_t waves = g.B * S * L;
+  hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, rows,
+                     g, (int)(S * L));
+  int rc = check_launch("a5_prefix_kernel");
+  if (rc) return rc;
+  rc = a5_launch_form<0>(rows, head, grad, g, S, L, kA5Few, st);
+  if (rc) return rc;
+  rc = a5_launch_form<6>(rows, head, grad, g, S, L, kA5Many, st);
+  if (rc) return rc;
+  const int64_t nvox = (int64_t)g.D * g.H * g.W;
+  hipLaunchKernelGGL(a5_marked_kernel, dim3((unsigned)((nvox + 63) / 64), (unsigned)g.B), dim3(64),
+                     0, st, rows, head, grad, g, (int)S, (int)L);
+  return check_launch("a5_marked_kernel");
 }
 
 ExGeom ex_geom(int64_t B, int64_t D, int64_t H, int64_t W, int64_t T, const float* vs,
@@ -816,14 +919,15 @@ extern "C" int totri_volume_render_exhaustive_grad_volume(
   A5Rows rows;
   rows.g = (float*)ws;
   rows.c = (double*)(ws + lay.prefix);
-  rows.bad = (int*)(ws + lay.bad);
+  rows.marked = (int*)(ws + lay.marked);
+  rows.count = (int*)(ws + lay.count);
   float4* head = (float4*)(ws + lay.head);
   // [B][T][S*L] -> [B][S*L][a5_row(T)]
   rc = transpose_strided(transient_grad, (float*)ws, (int)B, (int)T, (int)(S * L),
                          a5_row((int)T), 0, st);
   if (rc) return rc;
   hipLaunchKernelGGL(ex_point_head_kernel, dim3((unsigned)((B * (S + L) + 255) / 256)), dim3(256),
-                     0, st, scan_points, laser_points, (int)S, (int)L, g, head, (int*)rows.bad);
+                     0, st, scan_points, laser_points, (int)S, (int)L, g, head, rows.count);
   rc = check_launch("ex_point_head_kernel");
   if (rc) return rc;
   return a5_launch(rows, head, volume_grad, g, S, L, st);
