@@ -115,3 +115,39 @@ def test_full_splat_zero_sigma_split(at, ws):
     mid[6, 5, 4] = True
     assert np.isnan(vol[0][:, mid]).all()
     assert rel_l2(vol[0][:, ~mid], want[0][:, ~mid]) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A", [1, 3])
+@pytest.mark.parametrize("big", [1.0, 1e3, 1e7])
+def test_full_splat_grad_attribute_range(big, A):
+    """An RBF's gradient does not suffer from the attribute of one out of its
+    reach.  Tolerance per entry: 64 * 2^-24 of the sum of its terms' magnitudes
+    (a weight's exponent carries four roundings of |k r^2| < 27, at most 75 *
+    2^-24 and on average a few; products and sums the rest)."""
+    rng = np.random.default_rng(6)
+    res, N = (24, 20, 28), 30
+    rbf = np.concatenate([rng.uniform(-0.7, 0.2, (N, 2)), rng.uniform(0.7, 1.6, (N, 1)),
+                          rng.uniform(0.08, 0.12, (N, 1)), rng.uniform(0.5, 1.5, (N, A))], 1)
+    rbf[17] = [0.95, 0.95, 2.45, 0.05] + [big] * A
+    rbf = rbf.astype(np.float32)[None]
+    G = rng.standard_normal((1, 1 + A) + res).astype(np.float32)
+    vol, grad, _, _ = _calls(rbf, res, G, True)
+    v64 = vol.astype(np.float64)
+    ref = O.splat_grad(rbf, v64, G, VS, VE, mode=O.PURE64)[0]
+    z, y, x = np.meshgrid(*(np.linspace(VS[2 - k], VE[2 - k], res[k]) for k in range(3)),
+                          indexing="ij")
+    inv = 1.0 / np.where(v64[0, 0] < 1e-8, 1.0, v64[0, 0])
+    for i in range(N):
+        if i == 17:
+            continue
+        px, py, pz, s, *a = rbf[0, i].astype(np.float64)
+        d = np.stack([x - px, y - py, z - pz])
+        r2 = (d ** 2).sum(0)
+        g = np.exp(-0.5 * r2 / s ** 2)
+        mag = np.abs(G[0, 0]) + sum(
+            np.abs(G[0, 1 + k]) * inv * (abs(a[k]) + np.abs(v64[0, 1 + k])) for k in range(A))
+        bound = [(mag * g * np.abs(d[k])).sum() / s ** 2 for k in range(3)]
+        bound += [(mag * g * r2).sum() / s ** 3]
+        bound += [(np.abs(G[0, 1 + k]) * inv * g).sum() for k in range(A)]
+        assert (np.abs(grad[0, i] - ref[i]) <= 64 * 2.0 ** -24 * np.array(bound)).all(), i

@@ -708,7 +708,7 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
     const float* __restrict__ vgrad, float* __restrict__ out, SplatGeom g, int n_seg) {
   __shared__ float coord[kGradCoord + 16];
   __shared__ float red[kGradWaves][kGradRbf][4 + kMaxAttr];
-  __shared__ float mean[kMaxAttr];
+  __shared__ float common[kMaxAttr];
   const int lane = threadIdx.x & 63, wave = uniform_i32(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   const int i0 = blockIdx.x * kGradRbf, seg = blockIdx.y, b = blockIdx.z;
@@ -730,15 +730,21 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
     for (int e = threadIdx.x; e < ((W + 15) & ~15); e += blockDim.x)
       coord[g.D + g.H + e] = splat_coord(min(e, W - 1), W, g.sx, g.ex);
   }
-  // A common attribute value taken out of both terms of F0 + a Fa, which
+  // A common attribute value c taken out of both terms of F0 + a Fa, which
   // nearly cancel where one RBF stands alone (Va = a there): the mean of the
-  // workgroup's RBFs.
+  // workgroup's RBFs, no larger than twice the smallest magnitude among them.
+  // What is left of an RBF's own terms, a - c, is then no larger than about
+  // a itself, whatever its neighbours in the list hold (the plain mean of one
+  // attribute of 1e7 and 31 of about 1 cost those 31 six digits).
   if ((int)threadIdx.x < A) {
-    float m = 0.f;
-    for (int n = 0; n < kGradRbf; ++n)
-      m += rbf[((size_t)b * g.N + min(i0 + n, g.N - 1)) * RC + 4 + threadIdx.x];
+    float m = 0.f, least = INFINITY;
+    for (int n = 0; n < kGradRbf; ++n) {
+      const float a = rbf[((size_t)b * g.N + min(i0 + n, g.N - 1)) * RC + 4 + threadIdx.x];
+      m += a;
+      least = fminf(least, fabsf(a));
+    }
     m *= 1.f / kGradRbf;
-    mean[threadIdx.x] = fabsf(m) < INFINITY ? m : 0.f;
+    common[threadIdx.x] = fabsf(m) < INFINITY ? fminf(fmaxf(m, -2.f * least), 2.f * least) : 0.f;
   }
   __syncthreads();
 
@@ -764,7 +770,7 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
         const int i = min(i0 + 16 * n + r, g.N - 1);
         av[n][c] = c0 + c == 0 ? 1.f : 0.f;
         if (c0 + c >= 1 && c0 + c <= A)
-          av[n][c] = rbf[((size_t)b * g.N + i) * RC + 3 + c0 + c] - mean[c0 + c - 1];
+          av[n][c] = rbf[((size_t)b * g.N + i) * RC + 3 + c0 + c] - common[c0 + c - 1];
         ms[n][c] = 0.f;
       }
     for (int t = seg * kGradWaves + wave; t < n_tiles; t += kGradWaves * n_seg) {
@@ -811,7 +817,7 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
             }
             load4(v0b + (size_t)a * V, va);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) drift[u] = fmaf(dla[u], va[u] - mean[a - 1], drift[u]);
+            for (int u = 0; u < 4; ++u) drift[u] = fmaf(dla[u], va[u] - common[a - 1], drift[u]);
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) F[0][u] -= drift[u] * inv[u];
