@@ -127,3 +127,22 @@ def test_adjoint_marked_rows(T, scale):
         assert clear[b].any()
         assert rel_l2(got[b][clear[b]], ref[b][clear[b]]) < 1e-6
         assert rel_l2(got[b], ref[b]) < 1e-6
+
+
+@pytest.mark.gpu
+def test_adjoint_rows_past_two_to_the_31():
+    """Eight rows of 1.6e8 bins each, whose running sums lie more than 2^31
+    floats apart.  Row l holds l + 1 everywhere, so each of its spans averages
+    to l + 1 (1e-5: spans of 2e7 bins, positions in float to 16 bins)."""
+    from totrilib_amd.totri_cpp.render import volume_render_exhaustive_grad_volume
+    rng = np.random.default_rng(1)
+    T, L, res = 160_000_000, 8, (2, 2, 2)
+    scan, laser = points(rng, 1, 1), points(rng, 1, L)
+    G = torch.arange(1, L + 1, device="cuda", dtype=torch.float32).expand(1, T, 1, L).contiguous()
+    out = torch.empty((1,) + res, device="cuda")
+    empty = torch.empty(1, 3, 0, device="cuda")
+    volume_render_exhaustive_grad_volume(G, t(scan), t(laser), empty, empty, out, VS, VE, 8.0 / T,
+                                         0.0)
+    assert (out / 36 - 1).abs().max() < 1e-5
+    del G
+    torch.cuda.empty_cache()

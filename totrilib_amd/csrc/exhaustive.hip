@@ -373,10 +373,9 @@ __device__ __forceinline__ Sum2 add2(const Sum2& a, const Sum2& b) {
 }
 
 // One wave per row, eight bins per lane and step.
-__global__ __launch_bounds__(256) void a5_prefix_kernel(A5Rows rows, ExGeom g, int n_rows) {
+__device__ __forceinline__ void a5_prefix_row(const A5Rows& rows, const ExGeom& g, int n_rows,
+                                              size_t r) {
   const int lane = threadIdx.x & 63;
-  const size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= (size_t)g.B * n_rows) return;
   const float* src = rows.g + r * a5_row(g.T);
   double* dst = rows.c + r * a5_stride(g.T);
   Sum2 base = {0.0, 0.0};
@@ -422,6 +421,12 @@ __global__ __launch_bounds__(256) void a5_prefix_kernel(A5Rows rows, ExGeom g, i
   if (lane != 0) return;
   rows.marked[r] = mark ? 1 : 0;
   if (mark) atomicAdd(rows.count + r / n_rows, 1);
+}
+
+__global__ __launch_bounds__(256) void a5_prefix_kernel(A5Rows rows, ExGeom g, int n_rows) {
+  for (size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < (size_t)g.B * n_rows;
+       r += (size_t)gridDim.x * 4)
+    a5_prefix_row(rows, g, n_rows, r);
 }
 
 __global__ void zero_f32_kernel(float* __restrict__ out, int n) {
@@ -498,7 +503,11 @@ constexpr int kA5Slack = 8;  // floats past the staged rows that masked reads ma
 // with four roots and a loop over the bins per pair; 16 x 64 x 64 voxels,
 // 144 x 16 pairs, 1000 bins (spans up to 34 bins), render included: 0.91 ms
 // with running sums, 4.03 with the loop as the second form, 4.46 before.
-template <int K, int KT, bool STAGED, int NTH>
+//
+// Off holds the offsets between a unit's rows; 64 bits only where 32 do not
+// hold them (fewer loads are then in flight: 0.65 ms instead of 0.49 at 16 x 64
+// x 64 voxels, 144 x 16 pairs, 3,000 bins).
+template <int K, int KT, bool STAGED, int NTH, typename Off = int>
 __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
     A5Rows rows, const float4* __restrict__ head,  // [B][S + L]
     float* __restrict__ grad,                      // [B][D][H][W]
@@ -508,7 +517,7 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
   const int b = blockIdx.y;
   if (take != kA5All && a5_many(rows.count[b], S * L) != (take == kA5Many)) return;
   const int nvox = g.D * g.H * g.W;
-  const int P = K > 0 ? a5_row(g.T) : 2 * a5_stride(g.T);  // floats of a staged row
+  const Off P = K > 0 ? (Off)a5_row(g.T) : 2 * (Off)a5_stride(g.T);  // floats of a row
   const int v = blockIdx.x * NTH + threadIdx.x;
   const bool ok = v < nvox;
   const int vv = ok ? v : 0;
@@ -578,10 +587,11 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
     // rows of scan points s0 .. : nl consecutive rows each, L rows apart,
     // packed in the stage
     RowStage<NTH> next;
-    const int n4s = nl * P / 4;  // float4s per scan point
+    const int n4s = STAGED ? (int)(nl * P / 4) : 0;  // float4s per scan point
     auto points = [&](int u) { return min(U * SG, S - u * SG); };
     auto load = [&](int u) {
-      next.load_pieces(cb + ((size_t)u * SG * L + l0) * P, points(u) * n4s, n4s, L * P / 4);
+      next.load_pieces(cb + ((size_t)u * SG * L + l0) * P, points(u) * n4s, n4s,
+                       (int64_t)L * P / 4);
     };
     auto put = [&](int u, int buf) { next.store(stage + buf * cap, points(u) * n4s); };
     if (STAGED) {
@@ -602,7 +612,7 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
         // row of pair (s0 + i, l0 + j)
         const float* base = STAGED ? stage + cur * cap + (u - u0) * SG * nl * P
                                    : cb + ((size_t)s0 * L + l0) * P;
-        const int si = (STAGED ? nl : L) * P;
+        const Off si = SG > 1 ? (STAGED ? nl : L) * P : 0;
         float ds0[SG], ds1[SG];
         faces([&](int i) { return hs[min(s0 + i, S - 1)]; }, ds0, ds1,
               std::integral_constant<int, SG>{});
@@ -650,7 +660,7 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
           }
         }
         const float* any = K > 0 ? base : gb + ((size_t)s0 * L + l0) * a5_row(g.T);
-        const int ai = K > 0 ? si : L * a5_row(g.T);
+        const int64_t ai = K > 0 || SG == 1 ? (int64_t)si : (int64_t)L * a5_row(g.T);
 #pragma unroll
         for (int i = 0; i < SG; ++i)
 #pragma unroll
@@ -658,7 +668,7 @@ __global__ __launch_bounds__(NTH) void r2_adjoint_kernel(
             if (i < ns && j < nl &&
                 !(K == 0 && rows.marked[((size_t)b * S + s0 + i) * L + l0 + j]))
               acc += a5_pair_any<1>(g, ds0[i] + dl0[j], ds1[i] + dl1[j],
-                                 any + (size_t)i * ai + j * a5_row(g.T));
+                                 any + i * ai + j * (Off)a5_row(g.T));
       }
       if (STAGED) {
         __syncthreads();
@@ -731,9 +741,11 @@ int a5_launch_form(const A5Rows& rows, const float4* head, float* grad, const Ex
   if (kt == 8) return a5_launch_tile<K, 8>(rows, head, grad, g, S, L, sp, P, take, st);
   // rows too long for the stage: from global memory
   const int64_t nvox = (int64_t)g.D * g.H * g.W;
-  hipLaunchKernelGGL((r2_adjoint_kernel<K, 8, false, 256>),
-                     dim3((unsigned)((nvox + 255) / 256), (unsigned)g.B), dim3(256), 0, st, rows,
-                     head, grad, g, (int)S, (int)L, (int)S, 0, make_div_const(g.w), take);
+  auto kernel = 8 * P < (1ll << 31) ? r2_adjoint_kernel<K, 8, false, 256>
+                                    : r2_adjoint_kernel<K, 8, false, 256, int64_t>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((nvox + 255) / 256), (unsigned)g.B), dim3(256), 0,
+                     st, rows, head, grad, g, (int)S, (int)L, (int)S, 0, make_div_const(g.w),
+                     take);
   return check_launch("r2_adjoint_kernel");
 }
 
@@ -747,9 +759,9 @@ int a5_launch(const A5Rows& rows, const float4* head, float* grad, const ExGeom&
   const bool staged = a5_tile(g, L, a5_floats<6>(g.T), &sp) > 0;
   if (staged && bins < 1.99) return a5_launch_form<2>(rows, head, grad, g, S, L, kA5All, st);
   if (staged && bins < 5.95) return a5_launch_form<6>(rows, head, grad, g, S, L, kA5All, st);
-  const int64_t waves = g.B * S * L;
-  hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, rows,
-                     g, (int)(S * L));
+  const int64_t blocks = (g.B * S * L + 3) / 4;
+  hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)(blocks < (1 << 22) ? blocks : 1 << 22)),
+                     dim3(256), 0, st, rows, g, (int)(S * L));
   int rc = check_launch("a5_prefix_kernel");
   if (rc) return rc;
   rc = a5_launch_form<0>(rows, head, grad, g, S, L, kA5Few, st);

@@ -30,12 +30,12 @@ struct RowStage {
     }
   }
   // The same from pieces of `piece` float4s that start `step` float4s apart.
-  __device__ __forceinline__ void load_pieces(const float* src, int n4, int piece, int step) {
+  __device__ __forceinline__ void load_pieces(const float* src, int n4, int piece, int64_t step) {
 #pragma unroll
     for (int i = 0; i < kCopy4; ++i) {
       const int e = i * NTH + (int)threadIdx.x;
       const int k = e / piece;
-      buf[i] = e < n4 ? ((const float4*)src)[(size_t)k * step + (e - k * piece)]
+      buf[i] = e < n4 ? ((const float4*)src)[k * step + (e - k * piece)]
                       : make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
