@@ -261,9 +261,18 @@ int totri_volume_render_exhaustive_forward(
  * (src/render/volume.h:46-55, src/render/volume.cpp:98-111), whose kernel in
  * the reference is an empty stub (src/render/volume_cuda.cu:414-431).
  *   transient_grad [B][T][S][L]; volume_grad [B][D][H][W] written.
+ *   workspace      what the first query says, 4 bytes per element of
+ *                  transient_grad.  Voxels whose faces lie about six bins or
+ *                  more apart (or bins too many for LDS) are summed several
+ *                  times as fast from running sums, which take 8 bytes per
+ *                  element more: the second query knows the geometry and says
+ *                  which size runs fastest.
  */
 size_t totri_volume_render_exhaustive_grad_volume_workspace(int64_t B, int64_t T, int64_t S,
                                                             int64_t L);
+size_t totri_volume_render_exhaustive_grad_volume_workspace_box(
+    int64_t B, int64_t T, int64_t S, int64_t L, int64_t D, int64_t H, int64_t W,
+    const float volume_start[3], const float volume_end[3], float bin_width);
 int totri_volume_render_exhaustive_grad_volume(
     const float* transient_grad, int64_t B, int64_t T, int64_t S, int64_t L,
     const float* scan_points, const float* laser_points, float* volume_grad, int64_t D,

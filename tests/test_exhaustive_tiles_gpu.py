@@ -146,3 +146,47 @@ def test_adjoint_rows_past_two_to_the_31():
     assert (out / 36 - 1).abs().max() < 1e-5
     del G
     torch.cuda.empty_cache()
+
+
+def _sizes(B, T, S, L, res, w):
+    from totrilib_amd import _lib
+    lib = _lib.load()
+    return (lib.totri_volume_render_exhaustive_grad_volume_workspace(B, T, S, L),
+            lib.totri_volume_render_exhaustive_grad_volume_workspace_box(
+                B, T, S, L, *res, _lib.f3(VS), _lib.f3(VE), w))
+
+
+@pytest.mark.parametrize("B,T,S,L", [(1, 512, 256, 16), (2, 1000, 33, 1), (1, 2000, 1024, 1000)])
+def test_adjoint_scratch_sizes(B, T, S, L):
+    """Four bytes per bin and the points' headers; running sums only for spans
+    that need them."""
+    n = 4 * B * T * S * L
+    least, short = _sizes(B, T, S, L, (64, 8, 8), 4.0 / 64 / 4.0)
+    assert n <= least == short <= n + 16 * B * S * L + 16 * B * (S + L) + 1024
+    least, long = _sizes(B, T, S, L, (16, 8, 8), 4.0 / 16 / 40.0)
+    assert 3 * n <= long <= 3 * n + 64 * B * S * L + 16 * B * (S + L) + 2048
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,D", [(150, 20), (700, 6), (2600, 6), (9000, 6), (9000, 70)])
+def test_adjoint_least_scratch(T, D):
+    """With the first query's bytes, long spans add the bins."""
+    from totrilib_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(T)
+    res, w = (D, 5, 7), 8.0 / T
+    scan, laser = points(rng, 2, 9), points(rng, 2, 5)
+    G = rng.standard_normal((2, T, 9, 5)).astype(np.float32)
+    n = lib.totri_volume_render_exhaustive_grad_volume_workspace(2, T, 9, 5)
+    g, s, l = t(G), t(scan), t(laser)
+    out = torch.empty((2,) + res, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    for size in (n - 1, n):
+        buf = torch.full((n + 4096,), 0xff, dtype=torch.uint8, device="cuda")
+        got = lib.totri_volume_render_exhaustive_grad_volume(
+            g.data_ptr(), 2, T, 9, 5, s.data_ptr(), l.data_ptr(), out.data_ptr(), *res,
+            _lib.f3(VS), _lib.f3(VE), w, 0.0, buf.data_ptr(), size, st)
+        assert (got == 0) == (size == n)
+        assert (buf[n:] == 0xff).all()
+    ref = O.r2_adjoint(G, res, scan, laser, VS, VE, w, 0.0, mode=O.PINNED64)
+    assert rel_l2(out.cpu().numpy(), ref) < 1e-6

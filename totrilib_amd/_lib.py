@@ -93,6 +93,8 @@ SIGNATURES: dict[str, tuple] = {
         [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64,
          _F3, _F3, _c_f, _c_f, _c_p, _c_sz, _c_p]),
     "totri_volume_render_exhaustive_grad_volume_workspace": (_c_sz, [_c_i64] * 4),
+    "totri_volume_render_exhaustive_grad_volume_workspace_box": (
+        _c_sz, [_c_i64] * 7 + [_F3, _F3, _c_f]),
     "totri_volume_render_exhaustive_grad_volume": (
         _c_int,
         [_c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64,

@@ -332,7 +332,7 @@ __host__ __device__ __forceinline__ int a5_stride(int T) { return (T + 2) & ~1; 
 
 struct A5Rows {
   const float* g;     // [B][S*L][a5_row(T)] the transposed gradient
-  double* c;          // [B][S*L][a5_stride(T)] its running sums
+  double* c;          // [B][S*L][a5_stride(T)] its running sums, or null
   int* marked;        // [B][S*L] whether a row's running sums are left out
   int* count;         // [B] marked rows
 };
@@ -344,17 +344,21 @@ enum A5Take { kA5All, kA5Few, kA5Many };
 // marked row in 32.
 __device__ __forceinline__ bool a5_many(int count, int rows) { return count > rows / 32; }
 
+// The rows, the point headers (which masked reads past the last row may touch)
+// and the count come first; the running sums and the marks, two thirds of the
+// whole, are needed by long spans only, and add the bins without them.
 struct A5Layout {
-  size_t prefix, head, marked, count, end;
+  size_t head, count, least, prefix, marked, end;
 };
 
 A5Layout a5_layout(int64_t B, int64_t T, int64_t S, int64_t L) {
   A5Layout l;
-  l.prefix = align256((size_t)B * S * L * a5_row((int)T) * sizeof(float));
-  l.head = l.prefix + align256((size_t)B * S * L * a5_stride((int)T) * sizeof(double));
-  l.marked = l.head + align256((size_t)B * (S + L) * sizeof(float4));
-  l.count = l.marked + align256((size_t)B * S * L * sizeof(int));
-  l.end = l.count + align256((size_t)B * sizeof(int));
+  l.head = align256((size_t)B * S * L * a5_row((int)T) * sizeof(float));
+  l.count = l.head + align256((size_t)B * (S + L) * sizeof(float4));
+  l.least = l.count + align256((size_t)B * sizeof(int));
+  l.prefix = l.least;
+  l.marked = l.prefix + align256((size_t)B * S * L * a5_stride((int)T) * sizeof(double));
+  l.end = l.marked + align256((size_t)B * S * L * sizeof(int));
   return l;
 }
 
@@ -749,16 +753,22 @@ int a5_launch_form(const A5Rows& rows, const float4* head, float* grad, const Ex
   return check_launch("r2_adjoint_kernel");
 }
 
-// A voxel's faces are at most 2 dz / w bins apart (each leg of a path changes
-// by at most the voxel's height), so their bins at most floor(2 dz / w) + 1.
-// A wrong guess costs the second form, no error.
-int a5_launch(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g, int64_t S,
-              int64_t L, hipStream_t st) {
+// The form (K) of a call.  A voxel's faces are at most 2 dz / w bins apart
+// (each leg of a path changes by at most the voxel's height), so their bins at
+// most floor(2 dz / w) + 1.  A wrong guess costs the second form, no error.
+int a5_form(const ExGeom& g, int64_t L) {
   const double bins = 2.0 * fabs((double)g.ez - g.sz) / g.D / (double)g.w;
   StagePlan sp;
-  const bool staged = a5_tile(g, L, a5_floats<6>(g.T), &sp) > 0;
-  if (staged && bins < 1.99) return a5_launch_form<2>(rows, head, grad, g, S, L, kA5All, st);
-  if (staged && bins < 5.95) return a5_launch_form<6>(rows, head, grad, g, S, L, kA5All, st);
+  if (a5_tile(g, L, a5_floats<6>(g.T), &sp) == 0) return 0;
+  return bins < 1.99 ? 2 : bins < 5.95 ? 6 : 0;
+}
+
+int a5_launch(const A5Rows& rows, const float4* head, float* grad, const ExGeom& g, int64_t S,
+              int64_t L, hipStream_t st) {
+  const int form = a5_form(g, L);
+  if (form == 2) return a5_launch_form<2>(rows, head, grad, g, S, L, kA5All, st);
+  if (form == 6 || rows.c == nullptr)
+    return a5_launch_form<6>(rows, head, grad, g, S, L, kA5All, st);
   const int64_t blocks = (g.B * S * L + 3) / 4;
   hipLaunchKernelGGL(a5_prefix_kernel, dim3((unsigned)(blocks < (1 << 22) ? blocks : 1 << 22)),
                      dim3(256), 0, st, rows, g, (int)(S * L));
@@ -896,7 +906,17 @@ extern "C" int totri_volume_render_exhaustive_forward(
 extern "C" size_t totri_volume_render_exhaustive_grad_volume_workspace(int64_t B, int64_t T,
                                                                        int64_t S, int64_t L) {
   if (B <= 0 || T < 0 || S <= 0 || L <= 0) return 0;
-  return a5_layout(B, T, S, L).end;
+  return a5_layout(B, T, S, L).least;
+}
+
+extern "C" size_t totri_volume_render_exhaustive_grad_volume_workspace_box(
+    int64_t B, int64_t T, int64_t S, int64_t L, int64_t D, int64_t H, int64_t W,
+    const float volume_start[3], const float volume_end[3], float bin_width) {
+  if (B <= 0 || T < 0 || S <= 0 || L <= 0 || !volume_start || !volume_end) return 0;
+  const A5Layout l = a5_layout(B, T, S, L);
+  if (T == 0 || D <= 0 || H <= 0 || W <= 0) return l.least;
+  const ExGeom g = ex_geom(B, D, H, W, T, volume_start, volume_end, bin_width, 0.f);
+  return a5_form(g, L) == 0 ? l.end : l.least;
 }
 
 extern "C" int totri_volume_render_exhaustive_grad_volume(
@@ -930,7 +950,7 @@ extern "C" int totri_volume_render_exhaustive_grad_volume(
   char* ws = (char*)workspace;
   A5Rows rows;
   rows.g = (float*)ws;
-  rows.c = (double*)(ws + lay.prefix);
+  rows.c = workspace_bytes >= lay.end ? (double*)(ws + lay.prefix) : nullptr;
   rows.marked = (int*)(ws + lay.marked);
   rows.count = (int*)(ws + lay.count);
   float4* head = (float4*)(ws + lay.head);

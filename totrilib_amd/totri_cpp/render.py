@@ -265,8 +265,9 @@ def volume_render_exhaustive_grad_volume(transient_grad: torch.Tensor,
     lib = _lib.load()
     out = OutputSlot(volume_grad)
     with torch.cuda.device(dev):
-        ws, wsp = workspace(lib.totri_volume_render_exhaustive_grad_volume_workspace(B, T, S, L),
-                            dev)
+        ws, wsp = workspace(lib.totri_volume_render_exhaustive_grad_volume_workspace_box(
+            B, T, S, L, D, H, W, _lib.f3(volume_start), _lib.f3(volume_end), float(bin_width)),
+            dev)
         rc = lib.totri_volume_render_exhaustive_grad_volume(
             g.data_ptr(), B, T, S, L, sp.data_ptr(), lp.data_ptr(), out.ptr(), D, H, W,
             _lib.f3(volume_start), _lib.f3(volume_end), float(bin_width), float(bin_offset),
