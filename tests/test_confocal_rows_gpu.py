@@ -142,3 +142,27 @@ def test_small_splits(shape, n, T):
     refv = O.a1_transpose(G, mp, X, Y, Z, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64)
     assert rel_l2(out.cpu().numpy(), ref) < TOL
     assert rel_l2(gv.cpu().numpy(), refv) < TOL
+
+
+def test_more_columns_than_a_launch_has_waves():
+    """2^26 columns: the pass over the volume's columns fits a launch."""
+    from totrilib_amd.totri_cpp.render import (volume_confocal_forward,
+                                               volume_confocal_grad_measurement_points)
+    X, Y, Z, N, T, w = 8192, 8192, 2, 2, 16, 0.25
+    rng = np.random.default_rng(2)
+    cols = np.stack([rng.integers(0, X, 50), rng.integers(0, Y, 50)], 1).astype(np.int32)
+    cols[0], cols[1] = (0, 0), (X - 1, Y - 1)
+    mp = rng.uniform(-1, 1, (3, N)).astype(np.float32)
+    mp[2] = 0
+    vol = np.zeros((X, Y, Z), np.float32)
+    vol[cols[:, 0], cols[:, 1]] = rng.random((50, Z))
+    v = torch.from_numpy(vol).to(dev())
+    m = torch.from_numpy(mp).to(dev())
+    out = torch.full((N, T), float("nan"), device=dev())
+    volume_confocal_forward(v, m, out, ORIGIN, SIZE, w, 0.0)
+    ref = O.r1_forward(vol, mp, T, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64, cols=cols)
+    assert ref.any() and rel_l2(out.cpu().numpy(), ref) < TOL
+    gp = torch.full((3, N), float("nan"), device=dev())
+    volume_confocal_grad_measurement_points(gp, v, m, torch.ones(N, T, device=dev()), ORIGIN, SIZE,
+                                            w, 0.0)
+    assert gp.isfinite().all() and gp.any()

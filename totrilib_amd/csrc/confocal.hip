@@ -177,23 +177,24 @@ __device__ __forceinline__ ConfGeom all_rows(ConfGeom g) {
   return g;
 }
 
-// One wave per column.
+// One wave per column and step.
 __global__ __launch_bounds__(256) void sample_rows_kernel(const float* __restrict__ vol,
                                                           ConfGeom g, int2* __restrict__ rows) {
   const int lane = threadIdx.x & 63;
-  const int col = uniform_i32(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (col >= g.X * g.Y) return;
-  const float* v = vol + (size_t)col * g.Z;
-  int first = g.Z, last = -1;
-  for (int z0 = 0; z0 < g.Z; z0 += 64) {
-    const int z = z0 + lane;
-    const unsigned long long m = __ballot(z < g.Z && v[z] != 0.f);  // true for NaN
-    if (m == 0) continue;
-    first = min(first, z0 + (int)__builtin_ctzll(m));
-    last = z0 + 63 - (int)__builtin_clzll(m);
+  for (int col = uniform_i32(blockIdx.x * 4 + (threadIdx.x >> 6)); col < g.X * g.Y;
+       col += (int)gridDim.x * 4) {
+    const float* v = vol + (size_t)col * g.Z;
+    int first = g.Z, last = -1;
+    for (int z0 = 0; z0 < g.Z; z0 += 64) {
+      const int z = z0 + lane;
+      const unsigned long long m = __ballot(z < g.Z && v[z] != 0.f);  // true for NaN
+      if (m == 0) continue;
+      first = min(first, z0 + (int)__builtin_ctzll(m));
+      last = z0 + 63 - (int)__builtin_clzll(m);
+    }
+    if (lane == 0)
+      rows[col] = last < 0 ? make_int2(1, 0) : make_int2(max(first - 1, 0), min(last, g.Z - 2));
   }
-  if (lane == 0)
-    rows[col] = last < 0 ? make_int2(1, 0) : make_int2(max(first - 1, 0), min(last, g.Z - 2));
 }
 
 // Fast part of the decision: z_hat = fma(sqrt_fast(d2), s, cfast) gives the
@@ -3057,8 +3058,9 @@ int launch_sample_rows(const float* vol, ConfGeom* g, size_t ws, void* workspace
   const size_t end = rows_end(ws, g->X, g->Y, g->N, g->T);
   if (end == ws || workspace == nullptr || workspace_bytes < end) return TOTRI_OK;
   int2* rows = (int2*)((char*)workspace + ((ws + 255) & ~(size_t)255));
-  hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)((g->X * g->Y + 3) / 4)), dim3(256), 0,
-                     st, vol, *g, rows);
+  const int64_t blocks = ((int64_t)g->X * g->Y + 3) / 4;  // X Y < 2^30, as Z >= 2
+  hipLaunchKernelGGL(sample_rows_kernel, dim3((unsigned)(blocks < (1 << 22) ? blocks : 1 << 22)),
+                     dim3(256), 0, st, vol, *g, rows);
   g->rows = rows;
   return check_launch("sample_rows_kernel");
 }
