@@ -151,3 +151,24 @@ def test_full_splat_grad_attribute_range(big, A):
         bound += [(mag * g * r2).sum() / s ** 3]
         bound += [(np.abs(G[0, 1 + k]) * inv * g).sum() for k in range(A)]
         assert (np.abs(grad[0, i] - ref[i]) <= 64 * 2.0 ** -24 * np.array(bound)).all(), i
+
+
+@pytest.mark.gpu
+def test_full_splat_large_plane():
+    """2^28 voxels in one slice: more tiles than a launch's grid takes."""
+    from totrilib_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(5)
+    res = (1, 16384, 16384)
+    rbf = _rbf(rng, 1, 3, 0)
+    rbf[..., 2] = 0.5
+    r = torch.from_numpy(rbf).cuda()
+    vol = torch.full((1, 1) + res, -1.0, device="cuda")
+    assert lib.totri_rbf2volume_gaussian_forward(
+        r.data_ptr(), 1, 3, 0, vol.data_ptr(), *res, _lib.f3(VS), _lib.f3(VE), 0.0, None, 0,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert (vol >= 0).all()
+    vox = np.concatenate([[0, 2 ** 28 - 1], rng.integers(0, 2 ** 28, 2000)])
+    got = vol.flatten()[torch.from_numpy(vox).cuda()].cpu().numpy()
+    ref = O.splat_forward(rbf, res, VS, VE, mode=O.PURE64, vox=vox)
+    assert rel_l2(got, ref.reshape(-1)[vox]) < 1e-5

@@ -516,7 +516,7 @@ __device__ __forceinline__ bool sep_degenerate(float k) { return k == -INFINITY;
 template <int C, int MT>
 __global__ __launch_bounds__(kSepWaves * 64) void splat_sep_kernel(
     const float* __restrict__ rbf, float* __restrict__ vol, float* __restrict__ part,
-    SplatGeom g, int n_split) {
+    SplatGeom g, int n_split, unsigned first) {
   constexpr int P = MT * kSepNT;  // 16 x 16 tiles of a workgroup
   // staged RBFs during the walk, partial tiles after it
   constexpr int kStage = kSepWaves * kSepChunk * (4 + C - 1) * (int)sizeof(float);
@@ -526,8 +526,9 @@ __global__ __launch_bounds__(kSepWaves * 64) void splat_sep_kernel(
   const int r = lane & 15, q = lane >> 4;
   const int HW = g.H * g.W;
   const int n_col = (HW + kSepCols - 1) / kSepCols, n_z = (g.D + 16 * MT - 1) / (16 * MT);
-  const int tile = blockIdx.x / n_col;
-  const int col0 = (blockIdx.x - tile * n_col) * kSepCols;
+  const unsigned block = first + blockIdx.x;
+  const int tile = block / n_col;
+  const int col0 = (block - tile * n_col) * kSepCols;
   const int z0 = (tile % n_z) * (16 * MT);
   const int a0 = (tile / n_z) * kSepAttr;
   const int b = blockIdx.y, split = blockIdx.z;
@@ -1063,8 +1064,13 @@ SepPlan sep_plan(int64_t B, int64_t N, int64_t A, int64_t D, int64_t H, int64_t 
 template <int C, int MT>
 void launch_sep(const float* rbf, float* vol, float* part, const SplatGeom& g, const SepPlan& p,
                 int split, hipStream_t st) {
-  hipLaunchKernelGGL((splat_sep_kernel<C, MT>), dim3(p.grid, (unsigned)g.B, (unsigned)split),
-                     dim3(kSepWaves * 64), 0, st, rbf, vol, part, g, split);
+  // a launch holds less than 2^32 lanes along x: flat volumes take several
+  constexpr unsigned most = 1u << 22;
+  for (unsigned first = 0; first < p.grid; first += most)
+    hipLaunchKernelGGL((splat_sep_kernel<C, MT>),
+                       dim3(p.grid - first < most ? p.grid - first : most, (unsigned)g.B,
+                            (unsigned)split),
+                       dim3(kSepWaves * 64), 0, st, rbf, vol, part, g, split, first);
 }
 
 template <int C>
