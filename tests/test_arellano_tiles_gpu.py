@@ -47,3 +47,30 @@ def test_hits_equal_the_oracle(res, S, L, T, keep, vs, ve, w, off, same):
     got = got.detach().cpu().numpy().reshape(ref.shape)
     assert np.isfinite(ref).all()
     assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.parametrize("shift", [(3e3, -2e3, 1e3), (1e5, -1e5, 1e5), (1e6, 2e6, -1e6)])
+@pytest.mark.parametrize("w", [0.06, 0.25])
+def test_hits_far_from_the_origin(shift, w):
+    """The formula rounds a pair's centre to the coordinates' spacing: no hit
+    that this moves into a column is left out."""
+    from totrilib_amd.reconstruct import BackprojectionExhaustiveArellano
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(int(abs(shift[0])))
+    res, S, L, T = (9, 11, 12), 6, 3, int(9 / w)
+    sh = np.array(shift)
+    scan = (np.concatenate([rng.uniform(-1, 1, (1, 2, S)), np.zeros((1, 1, S))], 1)
+            + sh[None, :, None]).astype(np.float32)
+    laser = (np.concatenate([rng.uniform(-1, 1, (1, 2, L)), np.zeros((1, 1, L))], 1)
+             + sh[None, :, None]).astype(np.float32)
+    vs = tuple(float(v) for v in np.array([-1, -1, 0.5]) + sh)
+    ve = tuple(float(v) for v in np.array([1, 1, 2.5]) + sh)
+    tr = np.ones((1, T, S, L), np.float32)
+    dev = torch.device("cuda:0")
+    got = BackprojectionExhaustiveArellano.apply(
+        torch.from_numpy(tr).to(dev), torch.from_numpy(scan).to(dev),
+        torch.from_numpy(laser).to(dev), VolumeDef(vs, ve, res), BinDef(w, 0.0, T))
+    ref = O.arellano(tr, scan, laser, None, None, res, vs, ve, w, 0.0, mode=O.FP32)
+    got = got.detach().cpu().numpy().reshape(ref.shape)
+    assert ref.any() and np.isfinite(ref).all()
+    assert np.array_equal(got.astype(np.float64), ref)

@@ -614,13 +614,17 @@ __global__ __launch_bounds__(64) void arellano_kernel(
   }
   const float row_z = 2.f * fabsf(g.ez - g.sz) / depth;
   const float bz0 = fminf(g.sz, g.ez) - row_z, bz1 = fmaxf(g.sz, g.ez) + row_z;
-  // Smallest and largest distance of (px, py, pz) to the box, added.
-  auto box_reach = [&](float px, float py, float pz, float* lo, float* hi) {
+  const float box_far = fmaxf(fmaxf(fmaxf(fabsf(bx0), fabsf(bx1)), fmaxf(fabsf(by0), fabsf(by1))),
+                              fmaxf(fabsf(bz0), fabsf(bz1)));
+  // Smallest and largest distance of (px, py, pz) to the box, added; the largest
+  // coordinate.
+  auto box_reach = [&](float px, float py, float pz, float* lo, float* hi, float* far) {
     const float ax = fmaxf(fmaxf(bx0 - px, px - bx1), 0.f), cx = fmaxf(px - bx0, bx1 - px);
     const float ay = fmaxf(fmaxf(by0 - py, py - by1), 0.f), cy = fmaxf(py - by0, by1 - py);
     const float az = fmaxf(fmaxf(bz0 - pz, pz - bz1), 0.f), cz = fmaxf(pz - bz0, bz1 - pz);
     *lo += sqrt_fast(ax * ax + ay * ay + az * az);
     *hi += sqrt_fast(cx * cx + cy * cy + cz * cz);
+    *far = fmaxf(fmaxf(*far, fabsf(px)), fmaxf(fabsf(py), fabsf(pz)));
   };
   float nx = 0.f, ny = 0.f, nz = 0.f;
   float rsx = 0.f, rsy = 0.f, rsz = 0.f, rez = 0.f, dps = 0.f, dpe = 0.f;
@@ -684,15 +688,22 @@ __global__ __launch_bounds__(64) void arellano_kernel(
     const float k1m = r1 / r0 - 1.f;                                         // :85
     const float r1q = tc > e.len ? r1 * r1 : -INFINITY;                      // :81: no hit
     // An ellipsoid that stays clear of the box hits no column of it.  Its points
-    // have distance sums tc; rounding of the sphere it is scaled to moves that
-    // by a part in 10^3 at most where the sphere is not small (r1^2 no less
-    // than 10^-3 of the box's largest sum, squared): 4 parts are left.
-    float lo = 0.f, hi = 0.f;
+    // have distance sums tc, which the formula's roundings move.  (u = 2^-24; hi
+    // is the box's largest sum, and r1^2 >= 10^-3 hi^2.)  r1^2 is the rest of
+    // r0^2 - len^2 / 4: 3 u r0^2 / r1^2 < 2e-4 of it.  A line that passes the
+    // sphere outside counts as a hit within about 8 u hi^2 of r1^2: 5e-4 of it.
+    // Both scale the ellipsoid by under 4e-4, the sums of its points by 8e-4.  Where
+    // a line touches the sphere the root carries that error over as up to 7e-4 hi
+    // along the column, 1.4e-3 hi in the sums: 4e-3 hi holds both.  The pair's
+    // centre is rounded to u of the coordinates, in three axes, which moves a sum
+    // by under 4 u of the largest coordinate; 1e-6 of it is left.
+    float lo = 0.f, hi = 0.f, far = box_far;
     const int l = pair - s * L;
-    box_reach(sb[s], sb[S + s], sb[2 * S + s], &lo, &hi);
-    box_reach(lb[l], lb[L + l], lb[2 * L + l], &lo, &hi);
+    box_reach(sb[s], sb[S + s], sb[2 * S + s], &lo, &hi, &far);
+    box_reach(lb[l], lb[L + l], lb[2 * L + l], &lo, &hi, &far);
+    const float slack = 4e-3f * hi + 1e-6f * far;
     const bool clear = !(tc > e.len) || (r1q >= 1e-3f * hi * hi &&
-                                         (tc < lo - 4e-3f * hi || tc > hi * 1.004f));
+                                         (tc < lo - slack || tc > hi + slack));
     unsigned long long todo = __ballot(lane < n && !clear);
     auto entries = [&](const int* j, auto count) {
       constexpr int U = decltype(count)::value;
