@@ -95,3 +95,21 @@ def test_velten_exhaustive_smaller_stages(res, T, L):
     ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
     assert ref.any()
     assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("L", [1, 2, 3, 4, 5, 6, 7, 8, 13, 18])
+def test_velten_exhaustive_rows_from_global_memory(L):
+    """Rows longer than a stage: tiles of all laser points up to six, of 5 to 8
+    points above."""
+    from totrilib_amd.reconstruct import BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(L)
+    S, T, res = 11, 19000, (5, 6, 11)
+    scan, laser = points(rng, 1, S), points(rng, 1, L)
+    tr = rng.random((1, T, S, L)).astype(np.float32)
+    got = BackprojectionExhaustiveVelten.apply(
+        t(tr), t(scan), t(laser), VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T)).cpu().numpy()
+    ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
+    assert ref.any()
+    assert np.array_equal(got.astype(np.float64), ref)

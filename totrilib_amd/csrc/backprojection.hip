@@ -181,10 +181,11 @@ __device__ __forceinline__ unsigned velten_slot(int t, int T) {
 // time are staged in LDS (STAGED), or read from global memory (rows too long
 // for the stage).  The headers are uniform and come through the scalar cache.
 // Sums run over scan points in order, as the reference's loop.
-template <bool STAGED, int UN, int NTH>
+template <bool STAGED, int NTH>
 __global__ __launch_bounds__(NTH) void velten_confocal_kernel(
     const float* __restrict__ head, const float* __restrict__ rows, float* __restrict__ vol,
     BoxGeom g, int S, int R, int cap, float k2, DivConst dw) {
+  constexpr int UN = 8;  // scan points at a time
   extern __shared__ float4 lds4[];
   const int T = g.T;
   const int nv = velten_row(T);
@@ -896,19 +897,17 @@ int velten_confocal(const float* transient, int64_t B, int64_t T, int64_t S,
                      scan_points, scan_origin, g, (int)S, (int)So, rw, head, rows);
   rc = check_launch("velten_head_kernel");
   if (rc) return rc;
-  // Scan points per LDS stage: whole groups of eight, or four.  Where fewer
-  // rows fit (T above about 2550) the stage's barriers would come every few
-  // points: the rows are then read from global memory, through the caches.
+  // Scan points per LDS stage: whole groups of eight.  Where fewer rows fit (T
+  // above 2,300 bins, or 840 to 1,280 for volumes of several workgroups per CU) the
+  // stage's barriers would come every few points: the rows are then read from
+  // global memory, through the caches.
   const StagePlan sp = stage_plan(B, (int64_t)nvox);
-  int R = sp.cap / nv;
-  R = R >= 8 ? R & ~7 : R & ~3;
+  const int R = (sp.cap / nv) & ~7;
   const float k2 = 2.f * rw;
   const bool wide = sp.threads == 1024;
-  auto kernel = R >= 8  ? (wide ? velten_confocal_kernel<true, 8, 1024>
-                                : velten_confocal_kernel<true, 8, 256>)
-                : R > 0 ? (wide ? velten_confocal_kernel<true, 4, 1024>
-                                : velten_confocal_kernel<true, 4, 256>)
-                        : velten_confocal_kernel<false, 8, 256>;
+  auto kernel = R == 0 ? velten_confocal_kernel<false, 256>
+                : wide ? velten_confocal_kernel<true, 1024>
+                       : velten_confocal_kernel<true, 256>;
   const int threads = R > 0 ? sp.threads : 256;
   rc = allow_stage(kernel);
   if (rc) return rc;
@@ -1028,16 +1027,18 @@ int launch_velten_ex(const float* head, const float* rows, float* volume, const 
 // that is not full masks its last points.  Tiles of up to six points belong to
 // calls whose laser points make exactly one (their units take several scan
 // points); several tiles have seven points or more, also where that masks more
-// of the last.
+// of the last.  Where a stage holds fewer than eight rows for them, rows from
+// global memory are faster (56^3 voxels, 64 x 9 pairs, 900 bins: 0.33 ms with
+// tiles of seven staged rows).
 int velten_ex_tile(int64_t L, int64_t most) {
   static const int sizes[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
   int top = 0;
   for (int k : sizes)
     if (k <= most) top = k;
-  if (top == 0 || (L > top && top < 7)) return 0;
+  if (top == 0 || (L > top && top < 8)) return 0;
   const int64_t nt = (L + top - 1) / top;
   int64_t kt = (L + nt - 1) / nt;
-  if (nt > 1 && kt < 7) kt = 7;  // top >= 7 here
+  if (nt > 1 && kt < 7) kt = 7;  // top >= 8 here
   for (int k : sizes)
     if (k >= kt) return k;
   return 0;
@@ -1052,10 +1053,26 @@ int velten_ex(const float* head, const float* rows, float* volume, const BoxGeom
   const int pairs = ex_scan_group(kt > 0 ? kt : 1, 16) * (int64_t)kt <= fit ? 16 : 8;
   if (kt > 0 && ex_scan_group(kt, pairs) * (int64_t)kt > fit) kt = 0;
   if (kt == 0) {  // rows longer than the stage: read from global memory
-    const int64_t nt = (L + 7) / 8;
-    hipLaunchKernelGGL((velten_exhaustive_kernel<8, 0, 1, false, 256>),
-                       dim3(blocks_for(nvox), (unsigned)g.B), dim3(256), 0, st, head, rows,
-                       volume, g, (int)S, (int)L, (int)(S * nt), 0, make_div_const(g.w));
+    // up to six laser points: one tile, eight pairs a unit; else tiles of 5 to
+    // 8 points, the size that masks fewest
+    kt = (int)L;
+    if (L > 6) {
+      kt = 8;
+      for (int k = 7; k >= 5; --k)
+        if ((L + k - 1) / k * k < (L + kt - 1) / kt * kt) kt = k;
+    }
+    const int64_t sg = L > 6 ? 1 : ex_scan_group(kt, 8);
+    const int64_t units = (S + sg - 1) / sg * ((L + kt - 1) / kt);
+#define TOTRI_EXG(KT, NTL, SG) \
+  if (kt == KT && (L <= 6) == (NTL == 1)) kernel = velten_exhaustive_kernel<KT, NTL, SG, false, 256>;
+    auto kernel = velten_exhaustive_kernel<8, 0, 1, false, 256>;
+    TOTRI_EXG(1, 1, ex_scan_group(1, 8)) TOTRI_EXG(2, 1, ex_scan_group(2, 8))
+    TOTRI_EXG(3, 1, ex_scan_group(3, 8)) TOTRI_EXG(4, 1, ex_scan_group(4, 8))
+    TOTRI_EXG(5, 1, 1) TOTRI_EXG(6, 1, 1)
+    TOTRI_EXG(5, 0, 1) TOTRI_EXG(6, 0, 1) TOTRI_EXG(7, 0, 1)
+#undef TOTRI_EXG
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(nvox), (unsigned)g.B), dim3(256), 0, st, head,
+                       rows, volume, g, (int)S, (int)L, (int)units, 0, make_div_const(g.w));
     return check_launch("velten_exhaustive_kernel");
   }
   const int64_t nt = (L + kt - 1) / kt;

@@ -64,9 +64,9 @@ struct StagePlan {
 
 StagePlan stage_plan(int64_t B, int64_t nvox) {
   if (B * ((nvox + 1023) / 1024) >= 192) return {1024, kStageMax};
-  // two buffers per workgroup of the CU's 160 KiB: one, two or four of them
+  // two buffers per workgroup of the CU's 160 KiB: one to four of them
   const int64_t blocks = B * ((nvox + 255) / 256);
-  return {256, blocks <= 256 ? kStageMax : blocks <= 512 ? 10240 : 5120};
+  return {256, blocks <= 256 ? kStageMax : blocks <= 512 ? 10240 : blocks <= 768 ? 6720 : 5120};
 }
 
 }  // namespace
