@@ -172,3 +172,20 @@ def test_full_splat_large_plane():
     got = vol.flatten()[torch.from_numpy(vox).cuda()].cpu().numpy()
     ref = O.splat_forward(rbf, res, VS, VE, mode=O.PURE64, vox=vox)
     assert rel_l2(got, ref.reshape(-1)[vox]) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,A,res", [(40, 1, (2, 2, 300)), (33, 3, (1, 3, 130)),
+                                     (5, 0, (2, 1, 1000)), (3, 8, (3, 20, 128))])
+def test_full_splat_few_long_rows(N, A, res):
+    """Grids of few rows: the gradient's rows are split along x, with a
+    remainder of a chunk and of a step."""
+    rng = np.random.default_rng(N)
+    rbf = _rbf(rng, 1, N, A)
+    G = rng.standard_normal((1, 1 + A) + res).astype(np.float32)
+    ref = O.splat_forward(rbf, res, VS, VE, mode=O.PURE64)
+    gref = O.splat_grad(rbf, ref, G, VS, VE, mode=O.PURE64)
+    for ws in (True, False):
+        vol, grad, _, _ = _calls(rbf, res, G, ws)
+        assert rel_l2(vol, ref) < 1e-5
+        assert rel_l2(grad, gref) < 1e-5

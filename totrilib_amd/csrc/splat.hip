@@ -609,18 +609,23 @@ __global__ __launch_bounds__(kSepWaves * 64) void splat_sep_kernel(
   }
 
   const int any_degenerate = __syncthreads_or(degenerate);
-  // Tile p of the workgroup goes to wave p, which adds the waves' parts.
+  // Tile p of the workgroup goes to wave p, which adds the waves' parts (of
+  // those that had RBFs).
   f32x4* red = (f32x4*)lds;  // [P][kSepWaves][64]
+  const int busy = min(max(n_chunk - split * kSepWaves, 0), kSepWaves);
   f32x4 sum[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) {
     if (c > 0) __syncthreads();
+    if (wave < busy) {
 #pragma unroll
-    for (int p = 0; p < P; ++p) red[(p * kSepWaves + wave) * 64 + lane] = acc[p / kSepNT][p % kSepNT][c];
+      for (int p = 0; p < P; ++p)
+        red[(p * kSepWaves + wave) * 64 + lane] = acc[p / kSepNT][p % kSepNT][c];
+    }
     __syncthreads();
     sum[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (wave < P)
-      for (int w = 0; w < kSepWaves; ++w) sum[c] += red[(wave * kSepWaves + w) * 64 + lane];
+      for (int w = 0; w < busy; ++w) sum[c] += red[(wave * kSepWaves + w) * 64 + lane];
   }
   if (wave >= P) return;
   const int col = col0 + 16 * (wave % kSepNT) + r;
@@ -690,8 +695,8 @@ __global__ void splat_sep_finish_kernel(const float* __restrict__ part, int n_sp
 // moments, is done once per (row, RBF) on the product's output registers,
 // where a lane holds one RBF (column) and four rows.
 //
-// One workgroup: 32 RBFs, the row tiles (16 rows) of its segment, dealt over
-// its four waves.  The attribute channels come in pairs, one walk over the
+// One workgroup: 32 RBFs, the row tiles (16 rows, or a chunk of x of them) of
+// its segment, dealt over its four waves.  The attribute channels come in pairs, one walk over the
 // rows per pair (more accumulators would halve the waves in flight).
 // 20,000 RBFs -> 128^3 with one attribute take 6.1 ms (83 TFLOP/s of matrix
 // products; forming F and the Gaussians takes most of the rest), where the
@@ -706,7 +711,8 @@ constexpr int kGradCoord = 4096;  // coordinates kept in LDS, at most
 template <int NC, int AT>
 __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_sep_kernel(
     const float* __restrict__ rbf, const float* __restrict__ vol,
-    const float* __restrict__ vgrad, float* __restrict__ out, SplatGeom g, int n_seg) {
+    const float* __restrict__ vgrad, float* __restrict__ out, SplatGeom g, int n_seg, int n_xc,
+    int xw) {
   __shared__ float coord[kGradCoord + 16];
   __shared__ float red[kGradWaves][kGradRbf][4 + kMaxAttr];
   __shared__ float common[kMaxAttr];
@@ -714,7 +720,7 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
   const int r = lane & 15, q = lane >> 4;
   const int i0 = blockIdx.x * kGradRbf, seg = blockIdx.y, b = blockIdx.z;
   const int A = AT >= 0 ? AT : g.A, RC = 4 + A, W = g.W;
-  const int n_rows = g.D * g.H, n_tiles = (n_rows + 15) / 16;
+  const int n_rows = g.D * g.H, n_units = (n_rows + 15) / 16 * n_xc;
   const size_t V = (size_t)n_rows * W;
   const float* v0b = vol + (size_t)b * (1 + A) * V;
   const float* g0b = vgrad + (size_t)b * (1 + A) * V;
@@ -774,7 +780,8 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
           av[n][c] = rbf[((size_t)b * g.N + i) * RC + 3 + c0 + c] - common[c0 + c - 1];
         ms[n][c] = 0.f;
       }
-    for (int t = seg * kGradWaves + wave; t < n_tiles; t += kGradWaves * n_seg) {
+    for (int unit = seg * kGradWaves + wave; unit < n_units; unit += kGradWaves * n_seg) {
+      const int t = unit / n_xc, xb = (unit - t * n_xc) * xw, xe = min(xb + xw, W);
       f32x4 acc[kGradNT][NC][3];
 #pragma unroll
       for (int n = 0; n < kGradNT; ++n)
@@ -854,9 +861,9 @@ __global__ __launch_bounds__(kGradWaves * 64, AT < 0 ? 3 : 4) void splat_grad_se
           }
         }
       };
-      int x0 = 0;
-      for (; x0 + 16 <= W; x0 += 16) step(x0, std::true_type{});
-      if (x0 < W) step(x0, std::false_type{});
+      int x0 = xb;
+      for (; x0 + 16 <= xe; x0 += 16) step(x0, std::true_type{});
+      if (x0 < xe) step(x0, std::false_type{});
       // rows 4 q .. 4 q + 3 of the tile, one RBF per lane and product
       const int first = min(t * 16 + 4 * q, n_rows - 1);
       int zi = first / g.H, yi = first - zi * g.H;
@@ -1102,23 +1109,40 @@ int splat_forward_full(const float* rbf, float* vol, const SplatGeom& g, void* w
   return check_launch("splat_sep_finish_kernel");
 }
 
-// Row segments of the untruncated gradient: enough workgroups of 32 RBFs for
-// six per CU, while each wave keeps at least two row tiles.  Below 16 steps
-// of 16 rows x 16 x a wave (about 10 us) the second launch costs more than
-// the segments give: 50 RBFs on 16^3 took 8 us longer a call with them.
-int grad_segments(int64_t B, int64_t N, int64_t D, int64_t H, int64_t W) {
+// The untruncated gradient's work of one workgroup of 32 RBFs: row tiles, each
+// in n_xc chunks of xw voxels along x, dealt over seg segments.
+struct GradPlan {
+  int seg, n_xc, xw;
+};
+
+// Enough segments for six workgroups per CU, while each wave keeps at least two
+// units; chunks of at least 64 voxels where there are too few rows for that (a
+// grid of 2 x 2 rows of 2,048 voxels, 50 RBFs with one attribute: 162 -> 32 us).
+// Below 16 steps of 16 rows x 16 x a wave (about 10 us) the second launch costs
+// more than the segments give: 50 RBFs on 16^3 took 8 us longer a call with them.
+GradPlan grad_plan(int64_t B, int64_t N, int64_t A, int64_t D, int64_t H, int64_t W) {
   const int64_t wgs = B * ((N + kGradRbf - 1) / kGradRbf);
-  const int64_t tiles = (D * H + 15) / 16;
-  const int64_t most = tiles / (2 * kGradWaves);
-  if ((tiles + kGradWaves - 1) / kGradWaves * ((W + 15) / 16) < 16) return 1;
-  int64_t seg = wgs > 0 ? (6 * 256 + wgs - 1) / wgs : 1;
-  if (seg > most) seg = most;
-  return (int)(seg < 1 ? 1 : seg);
+  const int64_t tiles = (D * H + 15) / 16, xs = (W + 15) / 16;
+  const int64_t walks = A == 0 ? 1 : (A + 2) / 2;  // channel pairs
+  const int64_t target = wgs > 0 ? (6 * 256 + wgs - 1) / wgs : 1;
+  int64_t xc = (2 * kGradWaves * target + tiles - 1) / tiles;
+  if (xc > xs / 4) xc = xs / 4;
+  if (xc < 1) xc = 1;
+  GradPlan p;
+  p.xw = (int)((xs + xc - 1) / xc * 16);
+  p.n_xc = (int)((W + p.xw - 1) / p.xw);
+  const int64_t units = tiles * p.n_xc;
+  int64_t seg = units / (2 * kGradWaves);
+  if (seg > target) seg = target;
+  if ((units + kGradWaves - 1) / kGradWaves * (p.xw / 16) * walks < 16) seg = 1;
+  p.seg = (int)(seg < 1 ? 1 : seg);
+  return p;
 }
 
 int splat_grad_full(const float* rbf, const float* vol, const float* vgrad, float* out,
                     const SplatGeom& g, void* ws, size_t ws_bytes, hipStream_t st) {
-  int seg = grad_segments(g.B, g.N, g.D, g.H, g.W);
+  const GradPlan p = grad_plan(g.B, g.N, g.A, g.D, g.H, g.W);
+  int seg = p.seg;
   const size_t n = (size_t)g.B * g.N * (4 + g.A);
   if (ws == nullptr || ws_bytes < seg * n * sizeof(float)) seg = 1;
   float* dst = seg > 1 ? (float*)ws : out;
@@ -1126,7 +1150,8 @@ int splat_grad_full(const float* rbf, const float* vol, const float* vgrad, floa
   auto kernel = g.A == 0   ? splat_grad_sep_kernel<1, 0>
                 : g.A == 1 ? splat_grad_sep_kernel<2, 1>
                            : splat_grad_sep_kernel<2, -1>;
-  hipLaunchKernelGGL(kernel, grid, dim3(kGradWaves * 64), 0, st, rbf, vol, vgrad, dst, g, seg);
+  hipLaunchKernelGGL(kernel, grid, dim3(kGradWaves * 64), 0, st, rbf, vol, vgrad, dst, g, seg,
+                     p.n_xc, p.xw);
   int rc = check_launch("splat_grad_sep_kernel");
   if (rc || seg == 1) return rc;
   hipLaunchKernelGGL(splat_sum_segments_kernel, dim3((unsigned)((n + 15) / 16)), dim3(256), 0, st,
@@ -1197,7 +1222,7 @@ extern "C" size_t totri_rbf2volume_gaussian_grad_workspace(int64_t B, int64_t N,
                                                            int64_t D, int64_t H, int64_t W,
                                                            float truncation) {
   if (truncation > 0.f || B <= 0 || N <= 0 || A < 0 || D <= 0 || H <= 0 || W <= 0) return 0;
-  const int seg = grad_segments(B, N, D, H, W);
+  const int seg = grad_plan(B, N, A, D, H, W).seg;
   return seg > 1 ? (size_t)seg * B * N * (4 + A) * sizeof(float) : 0;
 }
 
