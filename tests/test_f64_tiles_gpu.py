@@ -46,3 +46,27 @@ def test_render_and_adjoint_tiles(shape, n, T, w, off, wall):
     volume_confocal_grad_volume(out, t64(mp), t64(G), ORIGIN, SIZE, w, off)
     assert np.array_equal(out.cpu().numpy(),
                           O.a1_transpose_f64(G, mp, X, Y, Z, ORIGIN, SIZE, w, off))
+
+
+@pytest.mark.parametrize("shape,n,T", [
+    ((3, 4, 9), 10, 65),       # tiles from 640 samples on
+    ((3, 4, 9), 9, 71),        # one sample fewer
+    ((4, 5, 8), 20, 40),
+    ((4, 4, 15), 30, 24),      # short tiles from 24 bins on
+    ((4, 4, 15), 30, 23),
+    ((4, 4, 16), 40, 16),
+    ((6, 5, 63), 8, 129),
+    ((5, 5, 8), 3, 320),
+])
+def test_adjoint_tiles_of_few_samples(shape, n, T):
+    from totrilib_amd.totri_cpp.render import volume_confocal_grad_volume
+    X, Y, Z = shape
+    rng = np.random.default_rng(T + Z)
+    mp = rng.uniform(-1, 1, (3, n))
+    mp[2] = rng.uniform(-0.1, 0.1, n)
+    G = rng.standard_normal((n, T))
+    w = 3.3 / T
+    out = torch.full(shape, float("nan"), dtype=torch.float64, device="cuda:0")
+    volume_confocal_grad_volume(out, t64(mp), t64(G), ORIGIN, SIZE, w, 0.0)
+    ref = O.a1_transpose_f64(G, mp, X, Y, Z, ORIGIN, SIZE, w, 0.0)
+    assert ref.any() and np.array_equal(out.cpu().numpy(), ref)

@@ -308,6 +308,12 @@ constexpr int kBinsF64 = 256, kProdF64 = 3, kTileF64 = 64;
 // columns, 64 points, 128 bins take 2.42 ms with 8 rows (a1_f64_kernel: 3.09)
 // and 3.59 ms with 4 (2.69).
 constexpr int kMinRowsF64 = 8;
+// Of few samples a workgroup's rounds cost more than they share (us a call with
+// a1_f64_kernel and with tiles, 64 x 64 x 16 voxels: 4 points of 48 bins 23, 26, of
+// 256 bins 44, 31; 100 x 100 x 8: 16 points of 32 bins 76, 84, of 48 bins 93, 83); in
+// tiles of few rows a unit of few bins leaves lanes idle (64 points of 16 bins 199,
+// 237, of 31 bins 265, 237).
+constexpr int kMinSamplesF64 = 640, kShortTileF64 = 16, kMinBinsShortF64 = 24;
 struct UnitF64 {
   double2 c[kBinsF64];        // alpha f2 G (row zi + 1), (1 - alpha) f2 G (row zi)
   double2 zero;               // c[kBinsF64].x = +0
@@ -350,7 +356,7 @@ __global__ __launch_bounds__(64 * (kProdF64 + 1)) void a1_rows_f64_kernel(
     if (wave < kProdF64) {
       if ((r & 63u) == 0) {
         const unsigned u = min((r + lane) * kProdF64 + wave, units - 1u);
-        il = (int)(u / (unsigned)max(chunks, 1));
+        il = (int)(u / (unsigned)chunks);
         if (r < rounds) {
           const double wx = mp[il], wy = mp[g.N + il];
           wzl = mp[2 * g.N + il];
@@ -629,10 +635,11 @@ extern "C" int totri_volume_confocal_grad_volume_f64(
   const long long n_tiles = (Z + kTileF64 - 1) / kTileF64;
   const long long blocks = X * Y * n_tiles;
   if (bin_width > 0.f && bin_offset >= 0.f && volume_size[2] > 0.f && Z >= kMinRowsF64 &&
+      N * T >= kMinSamplesF64 && (Z >= kShortTileF64 || T >= kMinBinsShortF64) &&
       Z <= (1 << 20) && blocks < (1ll << 23)) {
     hipLaunchKernelGGL(a1_rows_f64_kernel, dim3((unsigned)blocks), dim3(64 * (kProdF64 + 1)), 0,
                        (hipStream_t)stream, volume, measurement_points, transient, g,
-                       (int)n_tiles, N * T == 0 ? 0 : unit_chunks_f64(g));
+                       (int)n_tiles, unit_chunks_f64(g));
     return check_launch("a1_rows_f64_kernel");
   }
   hipLaunchKernelGGL(a1_f64_kernel, dim3(blocks_for(nv)), dim3(256), 0, (hipStream_t)stream,
