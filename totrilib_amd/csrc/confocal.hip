@@ -1364,20 +1364,31 @@ void a6_pair_kernel(
                          chunks_per_group, lds2);
 }
 
-// Sum over p < n_parts of part[p * stride], in order, sixteen loads at a time (a
-// small call has few elements and many parts): 64 parts of 32^3 voxels 28 -> 9 us,
-// the benchmark step's 7 parts of 128^3 46 -> 30 us.
-__device__ __forceinline__ float sum_parts_at(const float* __restrict__ part, size_t stride,
-                                              int n_parts) {
-  constexpr int U = 16;
-  float v = part[0];
-  for (int p = 1; p < n_parts; p += U) {
+// v plus part[p * stride], p0 <= p < n_parts, in order, U loads at a time, while
+// U are left (or, with all set, to the end).
+template <int U>
+__device__ __forceinline__ int add_parts(const float* __restrict__ part, size_t stride, int p0,
+                                         int n_parts, bool all, float* v) {
+  int p = p0;
+  for (; all ? p < n_parts : p + U <= n_parts; p += U) {
     float x[U];
 #pragma unroll
     for (int k = 0; k < U; ++k) x[k] = part[(size_t)min(p + k, n_parts - 1) * stride];
 #pragma unroll
-    for (int k = 0; k < U; ++k) v = p + k < n_parts ? v + x[k] : v;
+    for (int k = 0; k < U; ++k) *v = p + k < n_parts ? *v + x[k] : *v;
   }
+  return p;
+}
+
+// Sum over p < n_parts of part[p * stride], in order, sixteen loads at a time,
+// the rest four at a time (a small call has few elements and many parts): 64
+// parts of 32^3 voxels 28 -> 9 us, the benchmark step's 7 parts of 128^3 46 -> 30
+// us.
+__device__ __forceinline__ float sum_parts_at(const float* __restrict__ part, size_t stride,
+                                              int n_parts) {
+  float v = part[0];
+  const int p = add_parts<16>(part, stride, 1, n_parts, false, &v);
+  add_parts<4>(part, stride, p, n_parts, true, &v);
   return v;
 }
 
