@@ -158,17 +158,15 @@ __device__ __forceinline__ void depth_range(const ConfGeom& g, float wz, float z
   *dhi = ((zhi + 0.5f) * is + g.oz) - wz + margin;
 }
 
-// Sample rows [lo, hi] of column col that the render and its scan-point
-// gradient have to visit: every other row holds two zeros, whose samples add
+// g.rows[col]: the sample rows [lo, hi] of column col that the render and its
+// scan-point gradient have to visit: every other row holds two zeros, whose samples add
 // exactly 0.  An albedo is mostly empty in earnest (a surface in a box), and a
 // bin range from these rows skips the windows that miss the surface: 47 x 41
 // points off the grid, 90 x 84 x 77 voxels of a surface, 601 bins: render
 // 2.84 -> 0.80 ms, scan-point gradient 3.9 -> 0.95 ms; 3 % of the voxels
-// anywhere in 128^3, 64 x 64 points: render 7.07 -> 6.9 ms; a dense volume
-// pays 5 us.
-__device__ __forceinline__ int2 sample_rows(const ConfGeom& g, int col) {
-  return g.rows ? g.rows[col] : make_int2(0, g.Z - 2);
-}
+// anywhere in 128^3, 64 x 64 points: render 7.07 -> 6.9 ms.  A dense volume
+// pays 5 us for the pass and, where its columns are short, up to 4 % for the
+// ranges (128 x 128 x 8).
 
 // g without the row ranges, known to the compiler as such (the batched kernels
 // have none, and spend their registers elsewhere).
@@ -344,6 +342,8 @@ __device__ __forceinline__ void r1_block(
   c0 = c0 - 0.5f;
   const float delta = guard_delta(g, wz, c0, 0.f);
   const float half_m_delta = 0.5f - delta;
+  float dlo_all, dhi_all;
+  depth_range(g, wz, 0.f, (float)(g.Z - 1), &dlo_all, &dhi_all);
 
   const int chunk_first = grp * chunks_per_group;
   const int total_chunks = (n_cols + chunk_cols - 1) / chunk_cols;
@@ -399,15 +399,19 @@ __device__ __forceinline__ void r1_block(
       const float y = cell_centre(yi, g.oy, g.szy, g.Y);
       const float dx = wx - x, dy = wy - y;
       const float dx2 = dx * dx, dy2 = dy * dy;
-      const int2 rows = sample_rows(g, colc);
-      float dlo, dhi;
-      depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
+      float dlo = dlo_all, dhi = dhi_all;
+      bool filled = cvalid;
+      if (g.rows) {
+        const int2 rows = g.rows[colc];
+        depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
+        filled = cvalid && rows.x <= rows.y;
+      }
       int tlo, thi;
       bin_range(g, dx2 + dy2, dlo, dhi, &tlo, &thi);
       const int klo = (max(tlo, t_base) - t_base) >> 6;
       const int khi = (min(thi, t_base + 64 * K - 1) - t_base) >> 6;
-      const bool any = cvalid && rows.x <= rows.y && thi >= t_base &&
-                       tlo <= t_base + 64 * K - 1 && tlo <= thi;
+      const bool any =
+          filled && thi >= t_base && tlo <= t_base + 64 * K - 1 && tlo <= thi;
       // Bit k set <=> window k may hold an active sample of this column.
       const unsigned packed =
           any ? (((2u << khi) - 1u) & ~((1u << klo) - 1u)) : 0u;
@@ -554,14 +558,20 @@ __device__ __forceinline__ void r1_item(const float* __restrict__ vol,
 }
 
 // `skip` (optional): a device flag; when it is set the launch does nothing
-// (the mirror-symmetric kernel below has done the work).
-template <int K>
+// (the mirror-symmetric kernel below has done the work).  ROWS: g.rows is given.
+// Each form keeps to its own bin ranges: with one kernel for both, a capture of
+// 47 x 41 points takes 809 us instead of 789, or small dense calls 5 to 8 % longer.
+template <int K, bool ROWS>
 __global__ __launch_bounds__(kWaves * 64) void r1_forward_kernel(
     const float* __restrict__ vol, const float* __restrict__ mp,
     float* __restrict__ dst, ConfGeom g, int t_base, int n_groups, int chunk_cols,
     int chunks_per_group, const int* __restrict__ skip) {
   if (skip && *skip) return;
   extern __shared__ float2 lds2[];
+  if (ROWS)
+    __builtin_assume(g.rows != nullptr);
+  else
+    g = all_rows(g);
   r1_item<K>(vol, mp, dst, g, t_base, (int)(blockIdx.x % n_groups),
              (int)(blockIdx.x / n_groups), n_groups, chunk_cols, chunks_per_group, lds2);
 }
@@ -821,6 +831,8 @@ __device__ __forceinline__ void r1_sym_block(
   c0 = c0 - 0.5f;
   const float delta = guard_delta(g, wz, c0, 0.f);
   const float half_m_delta = 0.5f - delta;
+  float dlo_all, dhi_all;
+  depth_range(g, wz, 0.f, (float)(g.Z - 1), &dlo_all, &dhi_all);
 
   const int total_chunks = (n_reps + reps_per_chunk - 1) / reps_per_chunk;
   const int chunk_first = grp * chunks_per_group;
@@ -905,17 +917,20 @@ __device__ __forceinline__ void r1_sym_block(
       const float dxa = wx - x0, dxb = wx - x1, dya = wy - y0, dyb = wy - y1;
       const float A = dxa * dxa, B = dxb * dxb, C = dya * dya, D = dyb * dyb;
       // rows that any of the mirror columns needs
-      int2 rows = sample_rows(g, rx * g.Y + ry);
+      float dlo = dlo_all, dhi = dhi_all;
+      bool rhit = rvalid;
+      if (g.rows) {
+        int2 rows = g.rows[rx * g.Y + ry];
 #pragma unroll
-      for (int m = 1; m < M; ++m) {
-        const int xi = (m & 1) ? g.X - 1 - rx : rx, yi = (m & 2) ? g.Y - 1 - ry : ry;
-        const int2 o = sample_rows(g, xi * g.Y + yi);
-        if (o.x > o.y) continue;
-        rows = rows.x > rows.y ? o : make_int2(min(rows.x, o.x), max(rows.y, o.y));
+        for (int m = 1; m < M; ++m) {
+          const int xi = (m & 1) ? g.X - 1 - rx : rx, yi = (m & 2) ? g.Y - 1 - ry : ry;
+          const int2 o = g.rows[xi * g.Y + yi];
+          if (o.x > o.y) continue;
+          rows = rows.x > rows.y ? o : make_int2(min(rows.x, o.x), max(rows.y, o.y));
+        }
+        depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
+        rhit = rvalid && rows.x <= rows.y;
       }
-      float dlo, dhi;
-      depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
-      const bool rhit = rvalid && rows.x <= rows.y;
       unsigned packed = 0u;
       bool any = false;
 #pragma unroll
@@ -1068,6 +1083,8 @@ __device__ __forceinline__ void a6_sym_block(
   c0 = c0 - 0.5f;
   const float delta = guard_delta(g, wz, c0, 0.f);
   const float half_m_delta = 0.5f - delta;
+  float dlo_all, dhi_all;
+  depth_range(g, wz, 0.f, (float)(g.Z - 1), &dlo_all, &dhi_all);
 
   const int total_chunks = (n_reps + reps_per_chunk - 1) / reps_per_chunk;
   const int chunk_first = grp * chunks_per_group;
@@ -1152,17 +1169,20 @@ __device__ __forceinline__ void a6_sym_block(
       const float dxa = wx - x0, dxb = wx - x1, dya = wy - y0, dyb = wy - y1;
       const float A = dxa * dxa, B = dxb * dxb, C = dya * dya, D = dyb * dyb;
       // rows that any of the mirror columns needs
-      int2 rows = sample_rows(g, rx * g.Y + ry);
+      float dlo = dlo_all, dhi = dhi_all;
+      bool rhit = rvalid;
+      if (g.rows) {
+        int2 rows = g.rows[rx * g.Y + ry];
 #pragma unroll
-      for (int m = 1; m < M; ++m) {
-        const int xi = (m & 1) ? g.X - 1 - rx : rx, yi = (m & 2) ? g.Y - 1 - ry : ry;
-        const int2 o = sample_rows(g, xi * g.Y + yi);
-        if (o.x > o.y) continue;
-        rows = rows.x > rows.y ? o : make_int2(min(rows.x, o.x), max(rows.y, o.y));
+        for (int m = 1; m < M; ++m) {
+          const int xi = (m & 1) ? g.X - 1 - rx : rx, yi = (m & 2) ? g.Y - 1 - ry : ry;
+          const int2 o = g.rows[xi * g.Y + yi];
+          if (o.x > o.y) continue;
+          rows = rows.x > rows.y ? o : make_int2(min(rows.x, o.x), max(rows.y, o.y));
+        }
+        depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
+        rhit = rvalid && rows.x <= rows.y;
       }
-      float dlo, dhi;
-      depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
-      const bool rhit = rvalid && rows.x <= rows.y;
       unsigned packed = 0u;
       bool any = false;
 #pragma unroll
@@ -1527,15 +1547,16 @@ __global__ __launch_bounds__(kWaves * 64) void a6_kernel(
     const float y = cell_centre(yi, g.oy, g.szy, g.Y);
     const float dx = wx - x, dy = wy - y;
     const float dx2 = dx * dx, dy2 = dy * dy;
-    const int2 rows = sample_rows(g, colc);
+    const int2 rows = g.rows ? g.rows[colc] : make_int2(0, g.Z - 2);
+    const bool filled = cvalid && rows.x <= rows.y;
     float dlo, dhi;
     depth_range(g, wz, (float)rows.x, (float)(rows.y + 1), &dlo, &dhi);
     int tlo, thi;
     bin_range(g, dx2 + dy2, dlo, dhi, &tlo, &thi);
     const int klo = (max(tlo, t_base) - t_base) >> 6;
     const int khi = (min(thi, t_base + 64 * K - 1) - t_base) >> 6;
-    const bool any = cvalid && rows.x <= rows.y && thi >= t_base &&
-                     tlo <= t_base + 64 * K - 1 && tlo <= thi;
+    const bool any =
+        filled && thi >= t_base && tlo <= t_base + 64 * K - 1 && tlo <= thi;
     const unsigned packed = any ? (((2u << khi) - 1u) & ~((1u << klo) - 1u)) : 0u;
     unsigned long long mask = __ballot(any);
     while (mask) {
@@ -3096,7 +3117,8 @@ void launch_r1(const R1Plan& p, const float* vol, const float* mp, float* dst,
   const int scan_groups = (g.N + kWaves - 1) / kWaves;
   const int blocks = scan_groups * p.n_groups;
   const size_t lds = 2 * (size_t)p.chunk_cols * g.Z * sizeof(float2);
-  hipLaunchKernelGGL(r1_forward_kernel<K>, dim3(blocks), dim3(kWaves * 64), lds, st,
+  auto kernel = g.rows ? r1_forward_kernel<K, true> : r1_forward_kernel<K, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kWaves * 64), lds, st,
                      vol, mp, dst, g, t_base, p.n_groups, p.chunk_cols,
                      p.chunks_per_group, skip);
 }
