@@ -854,9 +854,9 @@ extern "C" size_t totri_backprojection_confocal_velten_workspace(int64_t B, int6
 namespace totri_hip {
 namespace {
 
-// A2 with its scratch (the transient's value rows, the bin thresholds and the
-// per-point constants) supplied by the caller: the workspace of the entry
-// point below, or the library's own array for the allocation-free variant.
+// A2 with its scratch (a header and a row of the transient per scan point)
+// supplied by the caller: the workspace of the entry point below, or the
+// library's own array for the allocation-free variant.
 int velten_confocal(const float* transient, int64_t B, int64_t T, int64_t S,
                     const float* scan_points, const float* scan_origin, int64_t So,
                     float* volume, int64_t D, int64_t H, int64_t W,
@@ -917,7 +917,7 @@ int velten_confocal(const float* transient, int64_t B, int64_t T, int64_t S,
   return check_launch("velten_confocal_kernel");
 }
 
-// Scratch of the allocation-free A2: the transposed transient [B][S][T].
+// Scratch of the allocation-free A2.
 // Every device that runs the library holds its own copy of this array, at
 // its own address, until the process ends.  Host code never passes the
 // array's name to a kernel (on the host it only stands for the symbol): it

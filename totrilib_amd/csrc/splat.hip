@@ -77,7 +77,6 @@ __device__ __forceinline__ float gauss_exp2(float r2, float k) {
 
 // Truncation test: keep the RBF when r2 <= (trunc * sigma)^2.
 __device__ __forceinline__ bool within(float r2, float sg, float trunc) {
-  if (!(trunc > 0.f)) return true;
   const float lim = trunc * sg;
   return !(r2 > lim * lim);
 }
@@ -385,7 +384,7 @@ __global__ __launch_bounds__(kS2Waves * 64) void splat_grad_kernel(
   float av[kMaxAttr];
 #pragma unroll
   for (int a = 0; a < kMaxAttr; ++a) av[a] = a < g.A ? p[4 + a] : 0.f;
-  const float rad = g.trunc > 0.f ? g.trunc * fabsf(sg) * 1.0001f + 1e-6f : INFINITY;
+  const float rad = g.trunc * fabsf(sg) * 1.0001f + 1e-6f;
   int xa, xb, ya, yb, za, zb;
   axis_range(xr, rad, g.W, g.sx, g.ex, &xa, &xb);
   axis_range(yr, rad, g.H, g.sy, g.ey, &ya, &yb);
