@@ -166,3 +166,43 @@ def test_more_columns_than_a_launch_has_waves():
     volume_confocal_grad_measurement_points(gp, v, m, torch.ones(N, T, device=dev()), ORIGIN, SIZE,
                                             w, 0.0)
     assert gp.isfinite().all() and gp.any()
+
+
+@pytest.mark.parametrize("scan", ["mirror", "pairs", "random"])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_non_finite_upstream_on_empty_rows(bad, scan):
+    """A NaN or an infinity times an empty voxel is NaN in the scan-point
+    gradient: of its own scan point, and of no other."""
+    from totrilib_amd.totri_cpp.render import volume_confocal_grad_measurement_points
+    X, Y, Z, T, w = 32, 32, 70, 1024, 0.003  # X Y N T = 2^28
+    rng = np.random.default_rng(8)
+    mp = wall_grid(16)
+    if scan != "mirror":
+        mp = np.stack([rng.uniform(-1, 1, 256), rng.uniform(-1, 1, 256),
+                       np.zeros(256)]).astype(np.float32)
+    if scan == "pairs":
+        mp[:, 128:] = mp[:, :128] * np.array([[-1], [1], [1]], np.float32)
+    vol = np.zeros((X, Y, Z), np.float32)
+    vol[::3, 1::2, 5] = rng.random(vol[::3, 1::2, 5].shape)
+    G = rng.standard_normal((256, T)).astype(np.float32)
+    i = 37
+    # the last bin at which a sample of scan point i is active lies on empty rows
+    ones = O.r1_forward(np.ones_like(vol), mp, T, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64, i0=i,
+                        i1=i + 1)[0]
+    lit = O.r1_forward(vol, mp, T, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64, i0=i, i1=i + 1)[0]
+    t = int(np.flatnonzero(ones)[-1])
+    assert not lit[t - 64:].any()
+    G[i, t] = bad
+    gp = torch.full((3, 256), 7.0, device=dev())
+    volume_confocal_grad_measurement_points(
+        gp, torch.from_numpy(vol).to(dev()), torch.from_numpy(np.ascontiguousarray(mp)).to(dev()),
+        torch.from_numpy(G).to(dev()), ORIGIN, SIZE, w, 0.0)
+    got = gp.cpu().numpy()
+    ref = O.a6(vol, mp, G, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64, i0=i, i1=i + 1)
+    assert np.isnan(ref[:, i]).all()
+    assert np.isnan(got[:, i]).all()
+    others = np.arange(256) != i
+    assert np.isfinite(got[:, others]).all()
+    pts = (0, 127, 200, 255)
+    refp = sum(O.a6(vol, mp, G, ORIGIN, SIZE, w, 0.0, mode=O.PINNED64, i0=k, i1=k + 1) for k in pts)
+    assert rel_l2(got[:, pts], refp[:, pts]) < TOL

@@ -113,3 +113,25 @@ def test_velten_exhaustive_rows_from_global_memory(L):
     ref = O.velten_exhaustive(tr, scan, laser, None, None, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
     assert ref.any()
     assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("far", [np.inf, 1e20, 1e15])
+@pytest.mark.parametrize("S,T", [(19, 64), (8, 3000)])
+def test_velten_confocal_far_origin(S, T, far):
+    """Origins without a bound on the path length: those scan points add
+    nothing, whatever their place in the walk's groups."""
+    from totrilib_amd.reconstruct import BackprojectionConfocalVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(S)
+    res = (3, 5, 7)
+    scan = points(rng, 1, S)
+    origin = (scan - np.array([0, 0, 0.5])).astype(np.float32)
+    origin[0, ::3, 0] = far
+    origin[0, 4, 1] = -far
+    tr = rng.random((1, T, S)).astype(np.float32)
+    got = BackprojectionConfocalVelten.apply(
+        t(tr), t(scan), VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T), t(origin)).cpu().numpy()
+    ref = O.velten_confocal(tr, scan, origin, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
+    assert ref.any()
+    assert np.array_equal(got.astype(np.float64), ref)

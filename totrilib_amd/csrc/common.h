@@ -88,8 +88,9 @@ __device__ __forceinline__ float sqrt_fast(float x) {
 // r = x - q w is exact, and RN(q + r hi) is the correctly rounded quotient
 // (Markstein's theorem, which asks for a correctly rounded hi and such a q).
 // `ok` is false where an exponent could leave the range this holds in; x must
-// be finite and below 2^60 in magnitude.  Quotients that underflow are
-// not exact, which no bin decision sees.
+// be finite and below 2^60 in magnitude (an infinite or NaN x gives NaN, which
+// floor_to_int puts outside every range).  Quotients that underflow are not
+// exact, which no bin decision sees.
 struct DivConst {
   float w, hi, lo;
   int ok;
@@ -199,7 +200,8 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
   return v;
 }
 
-// floor(x) converted to int in one instruction (v_cvt_flr_i32_f32).
+// floor(x) converted to int in one instruction (v_cvt_flr_i32_f32), which
+// saturates; NaN gives the largest or smallest int by its sign bit (measured).
 __device__ __forceinline__ int floor_to_int(float x) {
   int r;
   asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
