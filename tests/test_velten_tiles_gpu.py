@@ -135,3 +135,24 @@ def test_velten_confocal_far_origin(S, T, far):
     ref = O.velten_confocal(tr, scan, origin, res, VS, VE, 8.0 / T, 0.0, mode=O.FP32)
     assert ref.any()
     assert np.array_equal(got.astype(np.float64), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("res", [(1, 9, 8), (7, 1, 9), (6, 5, 1), (1, 1, 1), (1, 300, 400)])
+@pytest.mark.parametrize("L", [1, 3, 8, 20])
+@pytest.mark.parametrize("T", [50, 19000])
+def test_velten_single_slices(res, L, T):
+    """A grid of one voxel along an axis has NaN coordinates there, and a NaN
+    path length lies in bin 0 (the conversion of NaN to int): every voxel adds
+    bin 0 of all pairs, in their order."""
+    from totrilib_amd.reconstruct import BackprojectionConfocalVelten, BackprojectionExhaustiveVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(L)
+    S = 13
+    scan, laser = points(rng, 1, S), points(rng, 1, L)
+    tr = rng.random((1, T, S, L)).astype(np.float32)
+    vd, bd = VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T)
+    got = BackprojectionExhaustiveVelten.apply(t(tr), t(scan), t(laser), vd, bd)
+    assert (got == float(np.add.accumulate(tr[0, 0].reshape(-1))[-1])).all()
+    got = BackprojectionConfocalVelten.apply(t(tr[..., 0]), t(scan), vd, bd)
+    assert (got == float(np.add.accumulate(tr[0, 0, :, 0])[-1])).all()

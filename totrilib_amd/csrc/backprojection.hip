@@ -379,6 +379,9 @@ __global__ __launch_bounds__(NTH) void velten_exhaustive_kernel(
   const float qx = inclusive_coord(x, g.W, g.sx, g.ex);
   const float qy = inclusive_coord(y, g.H, g.sy, g.ey);
   const float qz = inclusive_coord(z, g.D, g.sz, g.ez);
+  // A grid of one voxel along an axis has no coordinate there (0 / 0): its path
+  // lengths are NaN, which the formula puts into bin 0.
+  const float reach0 = isnan(qx + qy + qz) ? INFINITY : fabsf(g.off);
   const float* hs = head + (size_t)b * (S + L) * kVeltenHead;
   const float* hl = hs + (size_t)S * kVeltenHead;
   const float* rb = rows + (size_t)b * S * L * nv;
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(NTH) void velten_exhaustive_kernel(
         dist[i][j] = dist[i][j] + lo[j];
       }
     // false for NaN or inf; uniform
-    if (dw.ok && (rs + rch + fabsf(g.off)) * dw.hi < kVeltenMaxBins) {
+    if (dw.ok && (rs + rch + reach0) * dw.hi < kVeltenMaxBins) {
       unsigned at[SG][KT];
 #pragma unroll
       for (int i = 0; i < SG; ++i)
