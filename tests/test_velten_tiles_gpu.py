@@ -156,3 +156,25 @@ def test_velten_single_slices(res, L, T):
     assert (got == float(np.add.accumulate(tr[0, 0].reshape(-1))[-1])).all()
     got = BackprojectionConfocalVelten.apply(t(tr[..., 0]), t(scan), vd, bd)
     assert (got == float(np.add.accumulate(tr[0, 0, :, 0])[-1])).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,T", [(19, 64), (16, 3000)])
+def test_velten_confocal_nan_origin(S, T):
+    """A NaN path length lies in bin 0, whatever the scan point's place in the
+    walk's groups.  (Whole numbers: sums are exact in any order.)"""
+    from totrilib_amd.reconstruct import BackprojectionConfocalVelten
+    from totrilib_amd.types import BinDef, VolumeDef
+    rng = np.random.default_rng(S)
+    res = (3, 5, 7)
+    scan = points(rng, 1, S)
+    origin = (scan - np.array([0, 0, 0.5])).astype(np.float32)
+    lost = np.arange(1, S, 4)
+    origin[0, lost, 1] = np.nan
+    tr = rng.integers(1, 50, (1, T, S)).astype(np.float32)
+    got = BackprojectionConfocalVelten.apply(
+        t(tr), t(scan), VolumeDef(VS, VE, res), BinDef(8.0 / T, 0.0, T), t(origin)).cpu().numpy()
+    kept = np.setdiff1d(np.arange(S), lost)
+    ref = O.velten_confocal(tr[..., kept], scan[:, kept], origin[:, kept], res, VS, VE, 8.0 / T,
+                            0.0, mode=O.FP32)
+    assert np.array_equal(got.astype(np.float64), ref + tr[0, 0, lost].sum())

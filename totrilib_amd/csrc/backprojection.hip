@@ -112,7 +112,9 @@ __device__ __forceinline__ int velten_bin(float e, float dso2, float w, float of
 //   {x, y, z, c, dso2, half, 0, 0}: the estimate is fma(sqrt(e), 2/w, c),
 //   c = ((dso2 - off) * (1/w)) + 0.5, and decides where its fraction lies
 //   within `half` of 1/2; c is NaN where no bound holds (every pair of that
-//   point takes the formula),
+//   point takes the formula); x is NaN where every path length is (the formula
+//   puts those into bin 0, DivConst does not: a NaN squared distance keeps to the
+//   formula's own division),
 // then one row of nv floats per scan point: bin t at t, a zero at T (nv = T + 1
 // rounded up to a multiple of 4).
 constexpr int kVeltenHead = 8;
@@ -153,7 +155,8 @@ __global__ __launch_bounds__(256) void velten_head_kernel(
   const float m = (2.f * dmax + fabsf(dso2) + fabsf(g.off)) / g.w + 1.f;
   const bool est = g.w > 0.f && m < kVeltenMaxBins;  // false for NaN or inf
   float4* h = (float4*)(head + bs * kVeltenHead);
-  h[0] = make_float4(px, py, pz, est ? (dso2 - g.off) * rw + 0.5f : __builtin_nanf(""));
+  h[0] = make_float4(isnan(dso2 - g.off) ? __builtin_nanf("") : px, py, pz,
+                     est ? (dso2 - g.off) * rw + 0.5f : __builtin_nanf(""));
   h[1] = make_float4(dso2, est ? 0.5f - kVeltenGuard * m : 0.f, 0.f, 0.f);
   rows[bs * nv + g.T] = 0.f;
 }
